@@ -1,5 +1,5 @@
 // Merged-VDB renderer: MGRenderer::render_an_image (plenvdb/lib/vdb/plenvdb.h:
-// 1029-1035 -> renderer.cu:370-424) in four kernels and no host round trip.
+// 1029-1035 -> renderer.cu:370-424) in five kernels and no host round trip.
 //
 // The reference renders in two full marches per pixel (first_look_merged
 // counts the kept samples and rewrites t_min / t_max, renderer.cu:222-268;
@@ -8,18 +8,19 @@
 // materialised sample list (cuda_rgbnet, :83-109) and an atomic composite
 // (final_render, :112-119).  Here:
 //
-//   k_render_count  a wavefront per 8x8 pixel tile, a lane per pixel: the
-//                   first march with trigetDensity's summation order; stores
-//                   the kept count and the rewritten (t_min, t_max) per pixel.
-//                   Light on registers, so it runs at full occupancy.
+//   k_render_count  the first march with trigetDensity's summation order, L
+//                   lanes per pixel taking L consecutive steps at a time (a
+//                   wave per block of 64 / L pixels); stores the kept count and
+//                   the rewritten (t_min, t_max) per pixel.
 //   k_render_fill   the second march from the rewritten t_min with
 //                   trigetDensity2's order: the tile reserves its records with
 //                   one atomic (counts scanned across the wave) and writes one
-//                   32-byte record per kept sample (12 colour features in fp16,
-//                   the weight, the pixel), at most the first march's count of
+//                   32-byte record per kept sample (its cell, fractions,
+//                   weight and pixel), at most the first march's count of
 //                   them, contiguous per pixel.  So the sample set is the
 //                   reference's, including the second march's restart
 //                   (renderer.cu:263).
+//   k_render_gather the records' colour features, a thread per record.
 //   k_render_mlp    persistent waves over 64-record chunks: the RGB MLP on
 //                   v_mfma_f32_16x16x32_f16 (weights in LDS, shared by the
 //                   workgroup's 8 waves) and each record's contribution
@@ -34,8 +35,8 @@
 // and the 12 colour channels of the voxel's index (index 0's values for
 // inactive voxels; slot `nslots` holds index 0's values for corners whose leaf
 // does not exist).  A slot is 32 bytes (fp16: exact for the fp16 data of
-// mergeddata.npz) or 64 bytes (fp32); the densities follow once more as a
-// compact array, which the marches' corner loads read.
+// mergeddata.npz) or 64 bytes (fp32); the leaves' density cells follow
+// (k_render_cells), which the marches read.
 //
 // MLP.  Layer outputs are computed transposed (features x samples) and stay in
 // registers: the D fragment of one layer (lane (g,n): features 16m+4g+i of
@@ -47,6 +48,7 @@
 // 16-byte boundaries.
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -120,17 +122,43 @@ __global__ void k_render_pack(const float* __restrict__ w0, const float* __restr
 template <typename PT>
 __global__ void k_render_payload(const int32_t* __restrict__ slot_idx, int64_t nslots,
                                  const float* __restrict__ den, const float* __restrict__ col,
-                                 int64_t nidx, PT* __restrict__ pay, PT* __restrict__ dens) {
+                                 int64_t nidx, PT* __restrict__ pay) {
     const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (s > nslots) return;
     int64_t id = s < nslots ? slot_idx[s] : 0;  // slot nslots: index 0 (missing leaves)
     if (id < 0 || id >= nidx) id = 0;           // the host checks the range
     PT* p = pay + s * 16;
     p[0] = (PT)den[id];
-    dens[s] = (PT)den[id];
 #pragma unroll
     for (int c = 0; c < 12; ++c) p[1 + c] = (PT)col[id * 12 + c];
     p[13] = p[14] = p[15] = (PT)0.f;
+}
+
+// Density cells: for every leaf, the 9 x 9 x 9 trilinear cells that a sample
+// whose rounded voxel lies in the leaf can fall in (lower corners -1 .. 7 from
+// the leaf's origin on each axis), each with its eight corner densities in the
+// corner order of the marches, contiguous.  A march step then needs one
+// 16-byte (fp16; two for fp32) load at an address that follows from the leaf
+// alone, instead of eight loads behind up to eight more leaf lookups for a
+// cell on a leaf's face.  23 MB for 1985 leaves in fp16.
+constexpr int kCellSide = 9, kLeafCells = kCellSide * kCellSide * kCellSide;
+
+template <typename PT>
+__global__ void k_render_cells(TopoView t, const PT* __restrict__ pay, int64_t nslots,
+                               PT* __restrict__ cells) {
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= t.nleaf * kLeafCells) return;
+    const int64_t leaf = c / kLeafCells;
+    const int r = (int)(c - leaf * kLeafCells);
+    const int i0 = t.origins[3 * leaf] + r / (kCellSide * kCellSide) - 1;
+    const int j0 = t.origins[3 * leaf + 1] + (r / kCellSide) % kCellSide - 1;
+    const int k0 = t.origins[3 * leaf + 2] + r % kCellSide - 1;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int64_t s = slot_of(t, i0 + ((kCx >> q) & 1), j0 + ((kCy >> q) & 1),
+                                  k0 + ((kCz >> q) & 1));
+        cells[8 * c + q] = pay[16 * (s < 0 ? nslots : s)];
+    }
 }
 
 // Workspace of one frame (pvdb_render_workspace_bytes), 256-byte aligned parts.
@@ -150,7 +178,7 @@ struct FrameBuffers {
 struct RenderArgs {
     TopoView topo;
     const void* payload;
-    const void* den;  // [nslots + 1] densities alone (the first element of each slot)
+    const void* cells;  // [nleaf][kLeafCells][8] corner densities of the leaves' cells
     int64_t nslots;
     const uint4* packed;
     float* out;
@@ -160,7 +188,8 @@ struct RenderArgs {
     float c2w[12];
     float fx, cx, fy, cy;
     float mn[3], ext[3], ws[3], inv_ws[3];
-    int32_t H, W, inverse_y, ntx, ntiles;
+    int32_t H, W, inverse_y;
+    int32_t ntx, ntiles;  // the marches' pixel tiles (a wave each): per row, in all
     float near_, stepdist, act_shift, interval, thres, bg, t_stop;
 };
 
@@ -184,13 +213,27 @@ __device__ __forceinline__ float h2f(uint16_t h) {
     return (float)__builtin_bit_cast(_Float16, h);
 }
 
-// Density of a slot from the compact density array (2 or 4 bytes a slot, so
-// the marches' corner loads share cache lines; 2 MB at 1M slots in fp16).
+// The eight corner densities of a cell, as loaded (8 fp16 or 8 fp32).
 template <bool F32PAY>
-__device__ __forceinline__ float load_den(const void* den, int64_t slot) {
-    if (F32PAY) return reinterpret_cast<const float*>(den)[slot];
-    return h2f(reinterpret_cast<const uint16_t*>(den)[slot]);
-}
+struct CellRow {
+    uint4 v[F32PAY ? 2 : 1];
+    __device__ __forceinline__ void load(const void* cells, uint32_t cell) {
+        constexpr int n = F32PAY ? 2 : 1;
+        const uint4* p = reinterpret_cast<const uint4*>(cells) + (uint64_t)n * cell;
+#pragma unroll
+        for (int k = 0; k < n; ++k) v[k] = p[k];
+    }
+    __device__ __forceinline__ float operator[](int q) const {  // q a constant after unrolling
+        if constexpr (F32PAY) {
+            const uint4& a = v[q >> 2];
+            const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+            return __uint_as_float(w[q & 3]);
+        } else {
+            const uint32_t w[4] = {v[0].x, v[0].y, v[0].z, v[0].w};
+            return h2f((uint16_t)(w[q >> 1] >> (16 * (q & 1))));
+        }
+    }
+};
 
 template <bool F32PAY>
 __device__ __forceinline__ void load_col(const void* pay, int64_t slot, float* c12) {
@@ -386,12 +429,6 @@ __device__ __forceinline__ PixelRay pixel_ray(const RenderArgs& A, int px, int p
     return R;
 }
 
-// One step of a march: advances t, applies the box and isActive(Round(xyz))
-// tests and, for a sample that passes, forms its 8 corner slots (int()
-// truncation, renderer.cu:271-300) and trilinear weights.  Returns false for a
-// rejected step.  Missing leaves are stepped over with the t += step
-// accumulation alone (see the comment inside), so t stays the reference's
-// running sum and the set of tested steps is unchanged.
 // Takes steps t <- t + s (float, round to nearest) while the next t stays
 // below tsafe, t < tend and iter < max_iter -- the loop
 //     while (t + s < tsafe && t < tend && iter < max_iter) { t += s; ++iter; }
@@ -400,32 +437,28 @@ __device__ __forceinline__ PixelRay pixel_ray(const RenderArgs& A, int px, int p
 // ulp u, and t + s rounds to (T + D) u with D = s / u rounded to nearest,
 // the same D for every step, unless s / u lies exactly half way between two
 // integers (round-half-even would then depend on T's parity) or t + s
-// reaches the binade's top.  So k steps give (T + k D) u exactly, with k
-// bounded below the binade's top and below the stopping conditions (counted
-// in double, one step of margin); the loop finishes the rest.
+// reaches the binade's top.  So k steps give (T + k D) u exactly (an integer
+// below 2^24).  k only has to be a lower bound of the loop's count: it is the
+// distance to the nearest of the limits over D u in float (at most 2^18 steps
+// at a time, where that quotient is off by less than one), less one step; the
+// loop takes the rest.
 __device__ __forceinline__ void advance_steps(float& t, float s, float tsafe, float tend,
                                               int& iter, int max_iter) {
 #pragma unroll 1
     for (int pass = 0; pass < 4; ++pass) {
         if (!(t >= 1e-20f) || !(s > 0.f) || iter >= max_iter) break;
         int e;
-        (void)frexpf(t, &e);                      // t in [2^(e-1), 2^e)
-        const float u = ldexpf(1.f, e - 24);      // ulp of the binade
-        const float q = s / u;                    // exact: a power-of-two scale
-        if (!(q >= 1.f) || !(q < 8388608.f) || q - floorf(q) == 0.5f) break;
-        const double D = (double)rintf(q);
-        const double T = (double)(t / u);         // integer in [2^23, 2^24)
-        // steps j -> j + 1 inside the binade while T + (j + 1) D <= 2^24 - 1
-        const double kb = floor((16777215.0 - T) / D);
-        // the loop's conditions for step j: T + (j + 1) D < tsafe / u, T + j D < tend / u
-        const double ks = ceil(((double)tsafe / (double)u - T) / D) - 1.0;
-        const double ke = ceil(((double)tend / (double)u - T) / D);
-        const double k = fmin(fmin(kb, ks), fmin(ke, (double)(max_iter - iter))) - 1.0;
-        if (!(k >= 4.0)) break;
-        const int ki = (int)k;
-        t = ldexpf((float)(T + (double)ki * D), e - 24);
-        iter += ki;
-        if (kb - 1.0 > k) break;  // stopped by tsafe, tend or the cap: the loop ends it
+        (void)frexpf(t, &e);                   // t in [2^(e-1), 2^e)
+        const float q = ldexpf(s, 24 - e);     // s / u, exact
+        const float D = rintf(q);
+        if (!(q >= 1.f) || !(q < 8388608.f) || fabsf(q - D) == 0.5f) break;
+        const float top = ldexpf(1.f, e), lim = fminf(tsafe, tend);
+        const float m = (fminf(lim, top) - t) / ldexpf(D, e - 24);
+        const int k = (int)fminf(fminf(m, 262144.f) - 1.f, (float)(max_iter - iter));
+        if (k < 4) break;
+        t = ldexpf((float)((int)ldexpf(t, 24 - e) + k * (int)D), e - 24);
+        iter += k;
+        if (lim < top) break;
         // at the binade's top: plain steps into the next binade, then again
         for (int z = 0; z < 4 && t + s < tsafe && t < tend && iter < max_iter; ++z) {
             t += s;
@@ -437,12 +470,6 @@ __device__ __forceinline__ void advance_steps(float& t, float s, float tsafe, fl
         ++iter;
     }
 }
-
-struct Corners {
-    int32_t slot[8];  // the host keeps nslots + 1 below 2^31
-    float u, v, w;
-    int i0, j0, k0;   // the cell's lower corner
-};
 
 // Slots of the 8 corners of the cell with lower corner (i0, j0, k0) in the
 // corner order 000,001,011,010,110,111,101,100 (slot nslots, index 0's
@@ -468,16 +495,42 @@ __device__ __forceinline__ void corner_slots(const RenderArgs& A, int i0, int j0
     }
 }
 
-__device__ __forceinline__ bool march_step(const RenderArgs& A, const PixelRay& R, float& t,
-                                           float tend, int& iter, int max_iter, BlockCache& bc,
-                                           Corners& c) {
-    t += R.step;
-    ++iter;
+// A march takes its steps L at a time: the L lanes of a ray (consecutive lanes
+// of the wave) take its next L steps.  One lane's step: t is the reference's
+// running float sum (the steps before it added one by one), `hit` whether the
+// sample lies in the box and its rounded voxel is active (isActive(Round(xyz)),
+// rintf, half to even, NanoVDB.h:774-779).
+template <bool F32PAY>
+struct Step {
+    float t;
+    bool hit;
+    int i0, j0, k0;  // the sample's cell (int() truncation, renderer.cu:271-300)
+    float u, v, w;
+    CellRow<F32PAY> den;
+    float te;        // in a missing leaf: t at the exit of the empty cube around it
+};
+
+template <bool F32PAY, int L>
+__device__ __forceinline__ Step<F32PAY> march_step(const RenderArgs& A, const PixelRay& R,
+                                                   float t0, int iter, float tend, int max_iter,
+                                                   BlockCache& bc) {
+    const int sub = (int)(threadIdx.x & (L - 1));
+    Step<F32PAY> s;
+    float t = t0, before = t0;
+#pragma unroll
+    for (int k = 0; k < L; ++k) {
+        if (k <= sub) {
+            before = t;
+            t += R.step;
+        }
+    }
+    s.t = t;
+    s.hit = false;
+    s.te = -INFINITY;
     const float p0 = R.o[0] + t * R.d[0], p1 = R.o[1] + t * R.d[1], p2 = R.o[2] + t * R.d[2];
-    if (!(p0 >= 0.f && p1 >= 0.f && p2 >= 0.f && p0 <= 1.f && p1 <= 1.f && p2 <= 1.f))
-        return false;
+    const bool in = p0 >= 0.f && p1 >= 0.f && p2 >= 0.f && p0 <= 1.f && p1 <= 1.f && p2 <= 1.f;
+    if (!(in && before < tend && iter + sub < max_iter)) return s;
     const float x = p0 * A.ws[0], y = p1 * A.ws[1], z = p2 * A.ws[2];
-    // isActive(Round(xyz)): rintf, half to even (NanoVDB.h:774-779)
     const int vi = (int)rintf(x), vj = (int)rintf(y), vk = (int)rintf(z);
     const int32_t l = bc.get(A.topo, vi, vj, vk);
     if (l < 0) {
@@ -485,34 +538,72 @@ __device__ __forceinline__ bool march_step(const RenderArgs& A, const PixelRay& 
         // empty-run map no leaf lies within r - 1 cells of it, so every step
         // until the ray leaves the rounding box of that cube of cells,
         // [8(L - r + 1) - 0.5, 8(L + r) - 0.5), is rejected by this same test.
-        // Those steps are taken with the accumulation alone (in closed form,
-        // advance_steps), stopping two steps short of the computed exit, which
-        // covers its rounding (the exit is formed with reciprocals: a relative
-        // error of a few ulps, far inside the two steps).
-        const int L[3] = {vi >> 3, vj >> 3, vk >> 3};
-        const int r = empty_run(A.topo, L[0], L[1], L[2]);
+        const int c[3] = {vi >> 3, vj >> 3, vk >> 3};
+        const int r = empty_run(A.topo, c[0], c[1], c[2]);
         float te = INFINITY;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             if (R.d[a] == 0.f) continue;
-            const float xb = R.d[a] > 0.f ? 8.f * (float)(L[a] + r) - 0.5f
-                                          : 8.f * (float)(L[a] - r + 1) - 0.5f;
+            const float xb = R.d[a] > 0.f ? 8.f * (float)(c[a] + r) - 0.5f
+                                          : 8.f * (float)(c[a] - r + 1) - 0.5f;
             te = fminf(te, (xb * A.inv_ws[a] - R.o[a]) * R.inv_d[a]);
         }
-        advance_steps(t, R.step, te - 2.f * R.step, tend, iter, max_iter);
-        return false;
+        s.te = te;
+        return s;
     }
+    s.i0 = (int)x;  // x >= 0 here: int() == floor
+    s.j0 = (int)y;
+    s.k0 = (int)z;
+    // the mask word and the cell are loaded together: both follow from the leaf
+    // (the host keeps nleaf below 2^22, so the cell's index fits 32 bits)
     const int off = voxel_offset(vi, vj, vk);
-    if (!((A.topo.masks[(int64_t)l * 8 + (off >> 6)] >> (off & 63)) & 1ull)) return false;
-    const int i0 = (int)x, j0 = (int)y, k0 = (int)z;  // x >= 0 here: int() == floor
-    c.u = x - (float)i0;
-    c.v = y - (float)j0;
-    c.w = z - (float)k0;
-    c.i0 = i0;
-    c.j0 = j0;
-    c.k0 = k0;
-    corner_slots(A, i0, j0, k0, bc, c.slot);
-    return true;
+    const uint64_t word = A.topo.masks[(int64_t)l * 8 + (off >> 6)];
+    s.den.load(A.cells, (uint32_t)l * kLeafCells +
+                            (uint32_t)(((s.i0 - (vi & ~7) + 1) * kCellSide +
+                                        (s.j0 - (vj & ~7) + 1)) * kCellSide +
+                                       (s.k0 - (vk & ~7) + 1)));
+    s.hit = (word >> (off & 63)) & 1ull;
+    s.u = x - (float)s.i0;
+    s.v = y - (float)s.j0;
+    s.w = z - (float)s.k0;
+    return s;
+}
+
+// Lane j's value in each group of L consecutive lanes (j uniform).
+template <int L, int J>
+__device__ __forceinline__ float group_read(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(
+        __builtin_bit_cast(int, x), (J << 5) | (0x1f & ~(L - 1))));
+}
+
+// f(0), ..., f(L - 1), the index a compile-time constant.
+template <int L, typename F, int K = 0>
+__device__ __forceinline__ void for_lanes(F&& f) {
+    if constexpr (K < L) {
+        f(std::integral_constant<int, K>{});
+        for_lanes<L, F, K + 1>(static_cast<F&&>(f));
+    }
+}
+
+// The next L steps of every ray of the wave: returns the ray's hits as bits and
+// moves t past the steps.  Missing leaves are stepped over with the t += step
+// accumulation alone (in closed form, advance_steps), stopping two steps short
+// of the computed exit, which covers its rounding (the exit is formed with
+// reciprocals: a relative error of a few ulps, far inside the two steps); t
+// stays the reference's running sum and the set of tested steps is unchanged.
+template <bool F32PAY, int L>
+__device__ __forceinline__ uint32_t next_steps(const RenderArgs& A, const PixelRay& R, float& t,
+                                               int& iter, float tend, int max_iter,
+                                               BlockCache& bc, Step<F32PAY>& s) {
+    const int g0 = (int)(threadIdx.x & 63 & ~(L - 1));
+    s = march_step<F32PAY, L>(A, R, t, iter, tend, max_iter, bc);
+    const uint32_t hits = (uint32_t)(__ballot(s.hit) >> g0) & ((1u << L) - 1);
+    // the state after these steps; the last one's empty cube is stepped over
+    t = group_read<L, L - 1>(s.t);
+    iter += L;
+    const float te = group_read<L, L - 1>(s.te);
+    if (te > t) advance_steps(t, R.step, te - 2.f * R.step, tend, iter, max_iter);
+    return hits;
 }
 
 __device__ __forceinline__ int march_cap(const PixelRay& R, float t0, float t1) {
@@ -522,16 +613,25 @@ __device__ __forceinline__ int march_cap(const PixelRay& R, float t0, float t1) 
     return (span >= 0.f) ? (int)fminf(span * 1.0625f + 16.f, 16777216.f) : 0;
 }
 
-// The pixel of lane `lane` of tile `tile` (8 x 8 pixels, row-major tiles).
+// The pixel of a lane of tile `tile`: a wave's 64 / L pixels, L lanes each, as a
+// block of 4 x 4, 4 x 2 or 2 x 2 (row-major tiles).
+template <int L>
+struct TileShape {
+    static_assert(L == 4 || L == 8 || L == 16, "lanes per ray");
+    static constexpr int w = L <= 8 ? 4 : 2, h = 64 / L / w;
+};
 struct TilePixel {
     int px, py;
     bool valid;
     int64_t pix;
 };
+template <int L>
 __device__ __forceinline__ TilePixel tile_pixel(const RenderArgs& A, int tile, int lane) {
+    using S = TileShape<L>;
+    const int p = lane / L;
     TilePixel P;
-    P.px = (tile % A.ntx) * 8 + (lane & 7);
-    P.py = (tile / A.ntx) * 8 + (lane >> 3);
+    P.px = (tile % A.ntx) * S::w + p % S::w;
+    P.py = (tile / A.ntx) * S::h + p / S::w;
     P.valid = P.px < A.W && P.py < A.H;
     P.pix = (int64_t)P.py * A.W + P.px;
     return P;
@@ -543,76 +643,87 @@ __device__ __forceinline__ void wave_count_add(unsigned long long* dst, unsigned
     if (lane == 0 && v) atomicAdd(dst, v);
 }
 
-// Pass 1, first_look_merged (renderer.cu:222-268): a wave per 8 x 8 tile, a
-// lane per pixel.  Counts the kept samples with trigetDensity's summation
-// order and records the rewritten t range: the first kept t minus one step,
-// and the t of the early stop (or the box exit).
-template <bool F32PAY>
+// Both marches are bound by VALU issue at 800 x 800 (318M and 219M wave
+// instructions; the search for the next samples is about half of them, powf a
+// quarter) and by the waves' chains of dependent loads in small frames.  With a
+// lane per pixel, one step at a time and eight corner loads the pair took
+// 1970 us at 800 x 800 and 1406 us at 203 x 151 (fp32), now about 950 and 250.
+//
+// Pass 1, first_look_merged (renderer.cu:222-268): counts the kept samples with
+// trigetDensity's summation order and records the rewritten t range: the first
+// kept t minus one step, and the t of the early stop (or the box exit).
+template <bool F32PAY, int L>
 __global__ void __launch_bounds__(kMarchThreads) k_render_count(RenderArgs A) {
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, sub = lane & (L - 1);
     const int tile = blockIdx.x * (kMarchThreads / 64) + (threadIdx.x >> 6);
     if (tile >= A.ntiles) return;  // uniform over the wave
     const FrameBuffers& F = A.fb;
-    const TilePixel tp = tile_pixel(A, tile, lane);
-    unsigned long long n_gather = 0;
+    const TilePixel tp = tile_pixel<L>(A, tile, lane);
+    uint32_t n_gather = 0;
     if (tp.valid) {
         const PixelRay R = pixel_ray(A, tp.px, tp.py);
         BlockCache bc;
         float t = R.tmin, T = 1.f, tmin2 = R.tmin, tmax2 = R.tmax;
         int cnt = 0, iter = 0;
         const int cap1 = march_cap(R, R.tmin, R.tmax);
-        bool first = false;
-        while (t < R.tmax && iter < cap1) {
-            Corners c;
-            if (!march_step(A, R, t, R.tmax, iter, cap1, bc, c)) continue;
-            float dv[8];
+        bool done = false;
+        Step<F32PAY> s;
+        while (!done && t < R.tmax && iter < cap1) {
+            const uint32_t hits = next_steps<F32PAY, L>(A, R, t, iter, R.tmax, cap1, bc, s);
+            if (!hits) continue;
+            float alpha = 0.f;
+            if (s.hit) {
+                // trigetDensity order (:191-220): res += den * (1-u) * (1-v) * (1-w), ...
+                float sig = 0.f;
 #pragma unroll
-            for (int q = 0; q < 8; ++q) dv[q] = load_den<F32PAY>(A.den, c.slot[q]);
-            // trigetDensity order (:191-220): res += den * (1-u) * (1-v) * (1-w), ...
-            float sig = 0.f;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const float a = ((kCx >> q) & 1) ? c.u : 1.f - c.u;
-                const float b = ((kCy >> q) & 1) ? c.v : 1.f - c.v;
-                const float e = ((kCz >> q) & 1) ? c.w : 1.f - c.w;
-                sig = sig + ((dv[q] * a) * b) * e;
+                for (int q = 0; q < 8; ++q) {
+                    const float a = ((kCx >> q) & 1) ? s.u : 1.f - s.u;
+                    const float b = ((kCy >> q) & 1) ? s.v : 1.f - s.v;
+                    const float e = ((kCz >> q) & 1) ? s.w : 1.f - s.w;
+                    sig = sig + ((s.den[q] * a) * b) * e;
+                }
+                alpha = 1.f - powf(1.f + expf(sig + A.act_shift), -A.interval);
             }
-            ++n_gather;
-            const float alpha = 1.f - powf(1.f + expf(sig + A.act_shift), -A.interval);
-            if (alpha <= A.thres) continue;
-            const float wt = T * alpha;
-            T = T * (1.f - alpha);
-            if (wt <= A.thres) continue;
-            ++cnt;
-            if (!first) {
-                tmin2 = t - R.step;
-                first = true;
-            }
-            if (T < A.t_stop) {
-                tmax2 = t;
-                break;
-            }
+            // the samples of the batch in step order, every lane of the ray alike
+            // (selects: the ray's samples rarely agree with its neighbours')
+            for_lanes<L>([&](auto k) {
+                const float al = group_read<L, k.value>(alpha);
+                const float tk = group_read<L, k.value>(s.t);
+                const bool on = !done && ((hits >> k.value) & 1u);
+                n_gather += on ? 1u : 0u;
+                const bool kept_a = on && !(al <= A.thres);
+                const float wt = T * al;
+                T = kept_a ? T * (1.f - al) : T;
+                const bool kept = kept_a && !(wt <= A.thres);
+                tmin2 = kept && cnt == 0 ? tk - R.step : tmin2;
+                cnt += kept ? 1 : 0;
+                const bool stop = kept && T < A.t_stop;
+                tmax2 = stop ? tk : tmax2;
+                done = done || stop;
+            });
         }
-        F.pix_count[tp.pix] = cnt;
-        F.tspan[tp.pix] = make_float2(tmin2, tmax2);
+        if (sub == 0) {
+            F.pix_count[tp.pix] = cnt;
+            F.tspan[tp.pix] = make_float2(tmin2, tmax2);
+        }
     }
-    if (A.counters) wave_count_add(A.counters, n_gather, lane);
+    if (A.counters) wave_count_add(A.counters, sub == 0 ? (unsigned long long)n_gather : 0, lane);
 }
 
 // Pass 2, ray_marching_merged (renderer.cu:312-367), from the rewritten t_min
 // to t_max with trigetDensity2's summation order: the tile reserves its records
 // with one atomic (pass 1's counts scanned across the wave) and writes one
-// 32-byte record per kept sample (12 colour features in fp16, the weight, the
-// pixel), at most pass 1's count of them, contiguous per pixel.
-template <bool F32PAY>
+// 32-byte record per kept sample (its cell, fractions, weight and pixel), at
+// most pass 1's count of them, contiguous per pixel.
+template <bool F32PAY, int L>
 __global__ void __launch_bounds__(kMarchThreads) k_render_fill(RenderArgs A) {
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, sub = lane & (L - 1);
     const int tile = blockIdx.x * (kMarchThreads / 64) + (threadIdx.x >> 6);
     if (tile >= A.ntiles) return;  // uniform over the wave
     const FrameBuffers& F = A.fb;
-    const TilePixel tp = tile_pixel(A, tile, lane);
+    const TilePixel tp = tile_pixel<L>(A, tile, lane);
     const int cnt = tp.valid ? F.pix_count[tp.pix] : 0;
-    int incl = cnt;
+    int incl = sub == 0 ? cnt : 0;  // a pixel counts once, at its first lane
 #pragma unroll
     for (int dd = 1; dd < 64; dd <<= 1) {
         const int o = __shfl_up(incl, dd, 64);
@@ -622,7 +733,7 @@ __global__ void __launch_bounds__(kMarchThreads) k_render_fill(RenderArgs A) {
     unsigned long long base = 0;
     if (lane == 0 && tile_total > 0) base = atomicAdd(F.total, (unsigned long long)tile_total);
     base = __shfl(base, 0, 64);
-    const int64_t start = (int64_t)base + (incl - cnt);
+    const int64_t start = (int64_t)base + (incl - cnt);  // the same in all of a pixel's lanes
 
     int r = 0;
     float T = 1.f;
@@ -634,52 +745,60 @@ __global__ void __launch_bounds__(kMarchThreads) k_render_fill(RenderArgs A) {
         float t = span.x;
         int iter = 0;
         const int cap2 = march_cap(R, span.x, tmax2);
+        Step<F32PAY> s;
         while (t < tmax2 && iter < cap2) {
-            Corners c;
-            if (!march_step(A, R, t, tmax2, iter, cap2, bc, c)) continue;
-            float dv[8];
+            const uint32_t hits = next_steps<F32PAY, L>(A, R, t, iter, tmax2, cap2, bc, s);
+            if (!hits) continue;
+            float alpha = 0.f;
+            if (s.hit) {
+                float sc[8];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) dv[q] = load_den<F32PAY>(A.den, c.slot[q]);
-            float sc[8];
+                for (int q = 0; q < 8; ++q) {
+                    const float a = ((kCx >> q) & 1) ? s.u : 1.f - s.u;
+                    const float b = ((kCy >> q) & 1) ? s.v : 1.f - s.v;
+                    const float e = ((kCz >> q) & 1) ? s.w : 1.f - s.w;
+                    sc[q] = (a * b) * e;
+                }
+                // trigetDensity2 order (:271-300): sum of den * scale, left to right
+                float sig = s.den[0] * sc[0];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const float a = ((kCx >> q) & 1) ? c.u : 1.f - c.u;
-                const float b = ((kCy >> q) & 1) ? c.v : 1.f - c.v;
-                const float e = ((kCz >> q) & 1) ? c.w : 1.f - c.w;
-                sc[q] = (a * b) * e;
+                for (int q = 1; q < 8; ++q) sig = sig + s.den[q] * sc[q];
+                alpha = 1.f - powf(1.f + expf(sig + A.act_shift), -A.interval);
             }
-            // trigetDensity2 order (:271-300): sum of den * scale, left to right
-            float sig = dv[0] * sc[0];
-#pragma unroll
-            for (int q = 1; q < 8; ++q) sig = sig + dv[q] * sc[q];
-            const float alpha = 1.f - powf(1.f + expf(sig + A.act_shift), -A.interval);
-            if (alpha <= A.thres) continue;
-            const float wt = T * alpha;
-            T = T * (1.f - alpha);
-            if (wt <= A.thres) continue;
-            if (r < cnt) {
+            int at = -1;  // this lane's record
+            float mine = 0.f;
+            for_lanes<L>([&](auto k) {
+                const float al = group_read<L, k.value>(alpha);
+                const bool kept_a = ((hits >> k.value) & 1u) && !(al <= A.thres);
+                const float wt = T * al;
+                T = kept_a ? T * (1.f - al) : T;
+                const bool kept = kept_a && !(wt <= A.thres);
+                at = kept && k.value == sub ? r : at;
+                mine = kept && k.value == sub ? wt : mine;
+                r += kept ? 1 : 0;  // may pass pass 1's count; those are not written
+            });
+            if (at >= 0 && at < cnt) {
                 // the sample's cell and fractions; k_render_gather adds its colour
-                const int64_t q = start + r;
+                const int64_t q = start + at;
                 if (q < F.capacity) {
-                    F.rec[2 * q] = make_uint4((uint32_t)c.i0, (uint32_t)c.j0, (uint32_t)c.k0,
-                                              __float_as_uint(c.u));
-                    F.rec[2 * q + 1] = make_uint4(__float_as_uint(c.v), __float_as_uint(c.w),
-                                                  __float_as_uint(wt), (uint32_t)tp.pix);
+                    F.rec[2 * q] = make_uint4((uint32_t)s.i0, (uint32_t)s.j0, (uint32_t)s.k0,
+                                              __float_as_uint(s.u));
+                    F.rec[2 * q + 1] = make_uint4(__float_as_uint(s.v), __float_as_uint(s.w),
+                                                  __float_as_uint(mine), (uint32_t)tp.pix);
                 }
             }
-            ++r;  // pass 2 may keep more than pass 1 counted; those are not written
         }
     }
     const int written = r < cnt ? r : cnt;
     // reserved records pass 2 did not fill: no cell (i0 = -1), zero weight
-    for (int k = written; k < cnt; ++k) {
+    for (int k = written + sub; k < cnt; k += L) {
         const int64_t q = start + k;
         if (q < F.capacity) {
             F.rec[2 * q] = make_uint4(0xffffffffu, 0u, 0u, 0u);
             F.rec[2 * q + 1] = make_uint4(0u, 0u, 0u, (uint32_t)tp.pix);
         }
     }
-    if (tp.valid) {
+    if (tp.valid && sub == 0) {
         F.pix_start[tp.pix] = (int32_t)(start < kMaxRecords ? start : kMaxRecords);
         F.pix_written[tp.pix] = written;
         F.t_last[tp.pix] = cnt > 0 ? T : 1.f;
@@ -693,7 +812,8 @@ __global__ void __launch_bounds__(kMarchThreads) k_render_fill(RenderArgs A) {
             row[3] = make_uint4(pe[12], pe[13], pe[14], pe[15]);
         }
     }
-    if (A.counters) wave_count_add(A.counters + 1, (unsigned long long)written, lane);
+    if (A.counters)
+        wave_count_add(A.counters + 1, sub == 0 ? (unsigned long long)written : 0, lane);
 }
 
 // Colour of each record (trigetColor, renderer.cu:303-310: corner 0's row
@@ -916,15 +1036,15 @@ struct RenderStage {
 };
 
 // Payload of (nslots + 1) slots: the slot rows (32 or 64 bytes: density and
-// 12 colour channels), then the densities alone (2 or 4 bytes a slot).
+// 12 colour channels), then the leaves' density cells (16 or 32 bytes a cell).
 struct PayloadLayout {
-    size_t den, bytes;
+    size_t cells, bytes;
 };
 PayloadLayout payload_layout(const TopoView& t, int32_t payload_f32) {
     const size_t n = (size_t)t.nleaf * 512 + 1, es = payload_f32 ? 4 : 2;
     PayloadLayout L;
-    L.den = align256(n * 16 * es);
-    L.bytes = align256(L.den + n * es);
+    L.cells = align256(n * 16 * es);
+    L.bytes = align256(L.cells + (size_t)t.nleaf * kLeafCells * 8 * es);
     return L;
 }
 
@@ -970,6 +1090,17 @@ FrameBuffers frame_buffers(void* ws, int64_t hw, int64_t capacity) {
     return F;
 }
 
+template <typename PT>
+void build_payload(const TopoView& t, const int32_t* slot_idx, const float* den, const float* col,
+                   int64_t nidx, uint8_t* p, const PayloadLayout& L, hipStream_t s) {
+    const int64_t nslots = t.nleaf * 512;
+    PT* pay = reinterpret_cast<PT*>(p);
+    hipLaunchKernelGGL(k_render_payload<PT>, dim3(pvdb_blocks(nslots + 1, 256)), dim3(256), 0, s,
+                       slot_idx, nslots, den, col, nidx, pay);
+    hipLaunchKernelGGL(k_render_cells<PT>, dim3(pvdb_blocks(t.nleaf * kLeafCells, 256)), dim3(256),
+                       0, s, t, pay, nslots, reinterpret_cast<PT*>(p + L.cells));
+}
+
 }  // namespace
 
 extern "C" {
@@ -1007,17 +1138,13 @@ int pvdb_render_build_payload(const pvdb_topology* topo, const int32_t* slot_idx
     PVDB_CHECK_ARG(slot_idx && den && col && payload, "null pointer");
     PVDB_CHECK_ARG(nidx >= 1, "the data arrays need at least index 0");
     const TopoView tv = view_of(topo);
-    const int64_t nslots = tv.nleaf * 512;
     const PayloadLayout L = payload_layout(tv, payload_f32);
     uint8_t* p = reinterpret_cast<uint8_t*>(payload);
+    hipStream_t st = (hipStream_t)stream;
     if (payload_f32)
-        hipLaunchKernelGGL(k_render_payload<float>, dim3(pvdb_blocks(nslots + 1, 256)), dim3(256),
-                           0, (hipStream_t)stream, slot_idx, nslots, den, col, nidx,
-                           reinterpret_cast<float*>(p), reinterpret_cast<float*>(p + L.den));
+        build_payload<float>(tv, slot_idx, den, col, nidx, p, L, st);
     else
-        hipLaunchKernelGGL(k_render_payload<_Float16>, dim3(pvdb_blocks(nslots + 1, 256)),
-                           dim3(256), 0, (hipStream_t)stream, slot_idx, nslots, den, col, nidx,
-                           reinterpret_cast<_Float16*>(p), reinterpret_cast<_Float16*>(p + L.den));
+        build_payload<_Float16>(tv, slot_idx, den, col, nidx, p, L, st);
     PVDB_LAUNCHED("k_render_payload");
     return PVDB_OK;
 }
@@ -1046,6 +1173,36 @@ int pvdb_render_frame_info(const pvdb_render_desc* d, uint64_t* total, int32_t**
 
 namespace {
 
+// The two marches with L lanes per ray: a wave per tile of 64 / L pixels.
+template <bool F32PAY, int L>
+int launch_marches(RenderArgs A, hipStream_t s) {
+    using S = TileShape<L>;
+    A.ntx = (A.W + S::w - 1) / S::w;
+    A.ntiles = A.ntx * ((A.H + S::h - 1) / S::h);
+    const dim3 grid((A.ntiles + kMarchThreads / 64 - 1) / (kMarchThreads / 64));
+    hipLaunchKernelGGL((k_render_count<F32PAY, L>), grid, dim3(kMarchThreads), 0, s, A);
+    PVDB_LAUNCHED("k_render_count");
+    hipLaunchKernelGGL((k_render_fill<F32PAY, L>), grid, dim3(kMarchThreads), 0, s, A);
+    PVDB_LAUNCHED("k_render_fill");
+    return PVDB_OK;
+}
+
+// Lanes per ray by the frame's pixels.  A wave's time is its longest ray's
+// chain of dependent steps, so a small frame wants each ray cut into few
+// batches (and many waves), while a frame that fills the chip is bound by VALU
+// issue and wants few lanes past the rays' ends.  Whole frames, us, at
+// 4 / 8 / 16 lanes: 64 x 64 269 / 188 / 151; 203 x 151 344 / 299 / 347;
+// 200 x 200 456 / 373 / 386; 400 x 400 702 / 702 / 926; 560 x 560 1053 / 1166 /
+// 1699; 800 x 800 1859 / 2304 / - (one and two lanes per ray: 2270 and 1922 at
+// 800 x 800, slower below).
+template <bool F32PAY>
+int launch_marches_sized(const RenderArgs& A, hipStream_t s) {
+    const int64_t px = (int64_t)A.H * A.W;
+    if (px <= 16384) return launch_marches<F32PAY, 16>(A, s);
+    if (px <= 131072) return launch_marches<F32PAY, 8>(A, s);
+    return launch_marches<F32PAY, 4>(A, s);
+}
+
 // The frame on `ws` (a 256-byte aligned workspace of at least
 // pvdb_render_workspace_bytes(H, W, capacity) bytes; the callers check it).
 int render_image(const pvdb_topology* topo, const pvdb_render_desc* d, void* ws,
@@ -1060,7 +1217,7 @@ int render_image(const pvdb_topology* topo, const pvdb_render_desc* d, void* ws,
     A.topo = t;
     A.payload = d->payload;
     const PayloadLayout PL = payload_layout(t, d->payload_f32);
-    A.den = reinterpret_cast<const uint8_t*>(d->payload) + PL.den;
+    A.cells = reinterpret_cast<const uint8_t*>(d->payload) + PL.cells;
     A.nslots = t.nleaf * 512;
     A.packed = reinterpret_cast<const uint4*>(d->weights);
     A.out = d->out;
@@ -1081,8 +1238,6 @@ int render_image(const pvdb_topology* topo, const pvdb_render_desc* d, void* ws,
     A.H = d->H;
     A.W = d->W;
     A.inverse_y = d->inverse_y;
-    A.ntx = (d->W + 7) / 8;
-    A.ntiles = A.ntx * ((d->H + 7) / 8);
     A.near_ = d->near_;
     A.stepdist = d->stepdist;
     A.act_shift = d->act_shift;
@@ -1099,25 +1254,17 @@ int render_image(const pvdb_topology* topo, const pvdb_render_desc* d, void* ws,
         PVDB_HIP(hipGetDevice(&dev));
         PVDB_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     }
-    // the two marches: a wave per 8 x 8 tile
-    const int mgrid = (A.ntiles + kMarchThreads / 64 - 1) / (kMarchThreads / 64);
     {
         RenderStage st(0, s);
-        if (d->payload_f32) {
-            hipLaunchKernelGGL(k_render_count<true>, dim3(mgrid), dim3(kMarchThreads), 0, s, A);
-            PVDB_LAUNCHED("k_render_count");
-            hipLaunchKernelGGL(k_render_fill<true>, dim3(mgrid), dim3(kMarchThreads), 0, s, A);
-            PVDB_LAUNCHED("k_render_fill");
+        const int rc = d->payload_f32 ? launch_marches_sized<true>(A, s)
+                                      : launch_marches_sized<false>(A, s);
+        if (rc != PVDB_OK) return rc;
+        if (d->payload_f32)
             hipLaunchKernelGGL(k_render_gather<true>, dim3(pvdb_blocks(A.fb.capacity, 256)),
                                dim3(256), 0, s, A);
-        } else {
-            hipLaunchKernelGGL(k_render_count<false>, dim3(mgrid), dim3(kMarchThreads), 0, s, A);
-            PVDB_LAUNCHED("k_render_count");
-            hipLaunchKernelGGL(k_render_fill<false>, dim3(mgrid), dim3(kMarchThreads), 0, s, A);
-            PVDB_LAUNCHED("k_render_fill");
+        else
             hipLaunchKernelGGL(k_render_gather<false>, dim3(pvdb_blocks(A.fb.capacity, 256)),
                                dim3(256), 0, s, A);
-        }
         PVDB_LAUNCHED("k_render_gather");
     }
     static bool smem_set = false;
