@@ -158,6 +158,10 @@ __device__ __forceinline__ void st_row(float* base, int64_t s, const float (&v)[
 // With both grids in stepmode 1 only the leaves the backward touched are
 // visited: the others have all-zero gradients, which stepmode 1 skips, so the
 // result equals the reference's all-slot pass.  NC colour channels per slot.
+// In stepmode 1 a voxel's values and moments (156 bytes) are loaded only after
+// its gradient row showed something to apply: a second round trip, but a batch
+// leaves many voxels of the leaves that it touches alone.  600 leaves, 12
+// channels: 22.0 -> 15.5 us after 1021 rays, 26.3 -> 24.9 us after 8192.
 // With a bf16 colour payload and an fp32 master copy (cmaster != nullptr) the
 // update runs on the master and the payload receives its round-to-nearest
 // bf16 value, so updates below half a bf16 step accumulate instead of being
@@ -188,10 +192,7 @@ __global__ void __launch_bounds__(256) k_sparse_adam(TopoView t, uint8_t* __rest
         float gd, pd, md, vd;
         float gg[NC], mm[NC], vv[NC], pp[NC];
     };
-    auto load = [&](int64_t s, Vox& v) {
-        v.pd = den[s];
-        v.md = mden[s];
-        v.vd = vden[s];
+    auto load_grad = [&](int64_t s, Vox& v) {
         if (G.whole) {  // the row's vectors: colour, then the density
             float r[NC + 1 + (NC == 12 ? 3 : 0)];
             const float4* p = reinterpret_cast<const float4*>(G.color + s * G.cs);
@@ -210,6 +211,19 @@ __global__ void __launch_bounds__(256) k_sparse_adam(TopoView t, uint8_t* __rest
             v.gd = G.density[s * G.ds];
             ld_row<NC>(G.color, s, v.gg, G.cs);
         }
+    };
+    // whether the step moves any of the voxel's values; a voxel without a
+    // gradient stays out of it (NaN counts as one)
+    auto wanted = [&](const Vox& v) {
+        bool w = every || v.gd != 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) w = w || v.gg[c] != 0.f;
+        return w;
+    };
+    auto load = [&](int64_t s, Vox& v) {
+        v.pd = den[s];
+        v.md = mden[s];
+        v.vd = vden[s];
         ld_row<NC>(mcol, s, v.mm);
         ld_row<NC>(vcol, s, v.vv);
         if constexpr (BF16COL) {
@@ -287,12 +301,16 @@ __global__ void __launch_bounds__(256) k_sparse_adam(TopoView t, uint8_t* __rest
         const bool a0 = (t.masks[leaf * 8 + (k >> 6)] >> (k & 63)) & 1ull;
         const bool a1 = (t.masks[leaf * 8 + 4 + (k >> 6)] >> (k & 63)) & 1ull;
         Vox v0, v1;
-        if (a0) load(s0, v0);
-        if (a1) load(s1, v1);
-        if (a0) update(s0, v0);
-        if (a1) update(s1, v1);
-        zero(s0);
-        zero(s1);
+        if (a0) load_grad(s0, v0);
+        if (a1) load_grad(s1, v1);
+        const bool w0 = a0 && wanted(v0), w1 = a1 && wanted(v1);
+        if (w0) load(s0, v0);
+        if (w1) load(s1, v1);
+        if (w0) update(s0, v0);
+        if (w1) update(s1, v1);
+        // an inactive voxel of the leaf may have been scattered to
+        if (w0 || !a0) zero(s0);
+        if (w1 || !a1) zero(s1);
         __syncthreads();
         if (threadIdx.x == 0) touched[leaf] = 0;
     }
