@@ -8,8 +8,8 @@
 //   k_ray_march    wave per ray: march again, density gather, raw2alpha, alpha cull,
 //                  transmittance product-scan with early stop, weights, weight cull;
 //                  one record per occupancy-kept sample (contiguous per ray)
-//   k_mlp_fwd      workgroup per 32-record group: colour gather + MFMA MLP -> rgb;
-//                  the features (bf16 hi, lo) and the ReLU masks kept per record
+//   k_mlp_fwd      wave per 32-record group: colour gather + MFMA MLP -> rgb;
+//                  the input row (bf16 hi) and the ReLU masks kept per record
 //   k_ray_composite wave per ray: prefix of w*rgb, ray colour, the loss terms and
 //                  their gradient per ray; a second pass forms each sample's
 //                  dL/dlogit and, through the alpha/raw2alpha adjoints, dL/dsigma
@@ -90,9 +90,9 @@ struct Records {
     uint4* xrow;       // [5 per record] the backward's MLP input row, X columns 0..39 as bf16
                        // hi parts: the 12 gathered colour features, the 27 view-direction
                        // encoding inputs and the bias input (a zero row unless weight-kept)
-    uint32_t* relu;    // [8 per record] forward ReLU masks: word 4l + j = layer l's
-                       // hidden features 32j + 16m + 4g + i (m, i < 2, 4; g < 4) at
-                       // bit 8g + 4m + i
+    uint32_t* relu;    // [8 per record] forward ReLU masks: word 4l + g = layer l's
+                       // hidden features 16m + 4g + i (m < 8, i < 4; g < 4) at
+                       // bit 16 (i % 2) + 2m + i / 2
     float4* grad;      // [4 per record] dL/dfeature (12) and dL/dsigma; in the direct-colour
                        // configurations rgb (NC) between the composite's two passes, then
                        // dL/dk0 (NC) and dL/dsigma at float kSigmaAt<NC>
@@ -114,7 +114,10 @@ struct RayBuffers {
                        // (o + d t_min, .), (d / |d|, .), the step count in the .w pair
     uint16_t* pe;      // [N][3][32] with the MLP: the ray's MLP input columns 12..39 (view
                        // direction, its sin/cos encoding, the bias column) as bf16 hi,
-                       // mid and lo rows, written by the counting march; null without
+                       // mid and lo rows, column c at position c - 8, written by the
+                       // counting march; null without
+    const uint4* zero; // [12] zeros, the row that stands for a missing leaf's colour or a dead
+                       // sample's encoding, then [4] a leaf index of -1
 };
 
 // Kept step indices the counting march stores per ray (16-bit: rays of fewer
@@ -124,13 +127,14 @@ constexpr int kStepCache = 256;
 
 // Packed bf16 MLP weights for MFMA (row-major, zero padded):
 //   w0t [128][64]  W0^T (in 0..38 used)       w1t [128][128] W1^T
-//   w2t [16][128]  W2^T (rows 0..2 used)      w2  [128][32]  W2 (cols 0..2 used)
+//   w2  [128][32]  W2 (cols 0..2 used)
 //   w1  [128][128] W1                          w0  [16][128]  W0 rows 0..15 (0..11 used)
+// fwd: the forward's weights and bias splits as its LDS image (kFwdImage),
 // and fp32 biases b0[128], b1[128], b2[3].
 struct MlpPacked {
     const uint16_t* w0t;
     const uint16_t* w1t;
-    const uint16_t* w2t;
+    const uint4* fwd;
     const uint16_t* w2;
     const uint16_t* w1;
     const uint16_t* w0;
@@ -158,13 +162,60 @@ constexpr int kPartStride = (kMlpParams + 3) & ~3;  // dW partial rows padded to
 // it later in the step): item t of kPackItems.
 struct PackArgs {
     const float* prm;
-    uint16_t *w0t, *w1t, *w2t, *w2, *w1, *w0;
+    uint16_t *w0t, *w1t, *fwd, *w2, *w1, *w0;
     float* grad;
+    uint32_t* zero;  // [64] RayBuffers::zero
 };
-constexpr int kPackItems = kMlpParams > 128 * 128 ? kMlpParams : 128 * 128;
+
+// The forward MLP's LDS image, in bf16 values (what each part holds stands at
+// SmemFwd):
+//   [6][128][8]    W0^T columns by chunk, b0's split
+//   [4][9][64][8]  per row tile b1's split, then W1^T's eight k-steps, K permuted
+//   [8][2][4][8]   W2^T rows, K permuted
+//   [2][8]         the biases' inputs
+// Packed once a step, so that every workgroup's copy is contiguous: reading the
+// fragments out of the row-major weights, 64 lines an instruction, took a small
+// step longer than its arithmetic.
+constexpr int kImgW1 = 6 * 128 * 8, kImgW2 = kImgW1 + 4 * 9 * 64 * 8, kImgOnes = kImgW2 + 8 * 2 * 4 * 8,
+              kFwdImage = kImgOnes + 2 * 8;
+constexpr int kPackItems = kMlpParams > kFwdImage ? kMlpParams : kFwdImage;
+
+__device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l);
+
+// Part j of a bias as three bf16 weights (hi, mid, lo: fp32's 24 bits), zero
+// past them; an infinite or NaN bias stays whole in hi.
+__device__ __forceinline__ uint16_t bias_part(float b, int j) {
+    uint32_t hi, mi, lo;
+    split3(b, 0.f, hi, mi, lo);
+    const bool finite = (__float_as_uint(b) & 0x7f800000u) != 0x7f800000u;
+    return j == 0 ? (uint16_t)hi : (j > 2 || !finite ? (uint16_t)0 : (uint16_t)(j == 1 ? mi : lo));
+}
+
+__device__ __forceinline__ uint16_t fwd_image_item(int t, const float* prm) {
+    const int j = t & 7;
+    // the hidden feature at position 8h + j of k-step ks
+    auto feature = [j](int ks, int h) { return 16 * ks + 8 * (j >> 2) + 4 * h + (j & 3); };
+    if (t < kImgW1) {
+        const int chunk = t >> 10, o = (t >> 3) & 127, i = 8 * chunk + j;
+        if (chunk == 5) return bias_part(prm[kB0 + o], j);
+        return i < 39 ? f2bf_bits(prm[kW0 + i * 128 + o]) : (uint16_t)0;
+    }
+    if (t < kImgW2) {
+        const int q = t - kImgW1, T = q / (9 * 512), step = (q >> 9) % 9, lane = (q >> 3) & 63;
+        const int h = lane >> 5, o = 32 * T + (lane & 31);
+        if (step == 0) return h == 0 ? bias_part(prm[kB1 + o], j) : (uint16_t)0;
+        return f2bf_bits(prm[kW1 + feature(step - 1, h) * 128 + o]);
+    }
+    if (t < kImgOnes) {
+        const int q = t - kImgW2, ks = q >> 6, h = (q >> 5) & 1, o = (q >> 3) & 3;
+        return o < 3 ? f2bf_bits(prm[kW2 + feature(ks, h) * 3 + o]) : (uint16_t)0;
+    }
+    return t - kImgOnes < 3 ? (uint16_t)0x3f80 : (uint16_t)0;  // 1, 1, 1, 0 ..
+}
 
 __device__ __forceinline__ void pack_mlp_item(int t, const PackArgs& A) {
     if (t < kMlpParams) A.grad[t] = 0.f;
+    if (t < 64) A.zero[t] = t < 48 ? 0u : 0xffffffffu;
     if (t < 128 * 128) {  // w1t / w1: 128 x 128
         const int a = t >> 7, b = t & 127;
         A.w1t[a * 128 + b] = f2bf_bits(A.prm[kW1 + b * 128 + a]);  // W1^T[out a][in b]
@@ -174,9 +225,9 @@ __device__ __forceinline__ void pack_mlp_item(int t, const PackArgs& A) {
         const int o = t >> 6, i = t & 63;
         A.w0t[o * 64 + i] = i < 39 ? f2bf_bits(A.prm[kW0 + i * 128 + o]) : (uint16_t)0;
     }
-    if (t < 16 * 128) {  // w2t [16 out][128 in], w0 [16 in][128 out]
+    if (t < kFwdImage) A.fwd[t] = fwd_image_item(t, A.prm);
+    if (t < 16 * 128) {  // w0 [16 in][128 out]
         const int o = t >> 7, i = t & 127;
-        A.w2t[o * 128 + i] = o < 3 ? f2bf_bits(A.prm[kW2 + i * 3 + o]) : (uint16_t)0;
         A.w0[o * 128 + i] = o < 12 ? f2bf_bits(A.prm[kW0 + o * 128 + i]) : (uint16_t)0;
     }
     if (t < 128 * 32) {  // w2 [128 in][32 out]

@@ -217,7 +217,7 @@ __global__ void __launch_bounds__(kMaxRayWaves * 64) k_ray_count(StepParams P, T
         }
         uint32_t h, m, l;
         split3(v, 0.f, h, m, l);
-        uint16_t* row = R.pe + 96 * (int64_t)r;
+        uint16_t* row = R.pe + 96 * (int64_t)r + 4;  // column c of a part at position c - 8
         row[lane] = (uint16_t)h;
         row[32 + lane] = (uint16_t)m;
         row[64 + lane] = (uint16_t)l;

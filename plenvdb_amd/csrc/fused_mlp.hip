@@ -2,11 +2,10 @@
 // sigmoid; plenvdb/lib/dvgo.py:91-109,354-362) on MFMA, forward and backward,
 // over groups of 32 consecutive records (two 16-sample MFMA tiles).
 //
-// Activations are computed transposed (features x samples):
+// Activations are computed transposed (features x samples, the samples being an
+// MFMA's N dimension):
 //   H0^T = relu(W0^T X^T + b0),  H1^T = relu(W1^T H0^T + b1),  L^T = W2^T H1^T + b2
-// with v_mfma_f32_16x16x32_bf16 (samples are the N dimension); each wavefront
-// owns a slice of the hidden features and exchanges activations with the
-// others through LDS.  Weights are held in bf16; gradients and the last
+// Weights are held in bf16; gradients and the last
 // hidden layer travel as (hi, lo) bf16 pairs, so each product with a weight is
 // two MFMAs, which keeps about 16 significant bits where plain bf16 keeps 8
 // (plain bf16 inputs put the colour-feature gradients several percent off an
@@ -16,10 +15,11 @@
 // sample's feature gradient by a whole term.  dW products (activation x
 // gradient) take the hi parts only.
 //
-// k_mlp_fwd gathers the colour features, keeps them per record as (hi, lo)
-// bf16 (so the backward reads 48 bytes per record instead of redoing 8
-// gathers) and writes rgb.  k_mlp_bwd recomputes H0 and H1 (for the ReLU
-// masks and the dW operands), takes each sample's dL/dlogit and dL/dsigma from
+// k_mlp_fwd gathers the colour features and writes each record's rgb, ReLU masks
+// and bf16 input row (so the backward reads 80 bytes per record instead of
+// redoing 8 gathers).  k_mlp_bwd recomputes H0 and H1 (for the dW operands) in
+// wavefronts that own a slice of the hidden features each and exchange
+// activations through LDS, takes each sample's dL/dlogit and dL/dsigma from
 // the composite pass, runs g_H1^T = W2 g_L^T, g_H0^T = W1 g_H1^T (masked by
 // the ReLUs, kept as bit masks), g_X^T = W0[0:12] g_H0^T, accumulates dW over
 // each group's 32 samples (K = 32) in registers (one partial per workgroup),
@@ -28,6 +28,7 @@
 // rule (densityvdb.cu:16-27, colorvdb.cu:28-37).  Both kernels load a group's
 // records into registers while the previous group computes.
 
+#include <cstddef>
 #include <type_traits>
 
 #include "fused_common.h"
@@ -132,31 +133,11 @@ __device__ __forceinline__ void st_fm(uint16_t* fm, int col, int fr, int lane, c
     *reinterpret_cast<uint2*>(&fm[(fr + q) * FM + (col & ~3)]) = quad_transpose(hi, q);
 }
 
-// A wave's 32-bit slice of one sample's ReLU mask is written a byte per lane:
-// lane (g, n) holds bit i of nib[mt] for feature 16 mt + 4g + i and stores
-// byte g of sample n's word, nib[0] | nib[1] << 4, so the bit of feature
-// 16 mt + 4g + i is bit 8g + 4mt + i (no exchange between the lanes).
-__device__ __forceinline__ uint8_t relu_byte(uint32_t nib0, uint32_t nib1) {
-    return (uint8_t)(nib0 | (nib1 << 4));
-}
-
 // a (bf16 weight) times a split activation
 __device__ __forceinline__ f32x4 mfma_w(const bf16x8& a, const bf16x8& bh, const bf16x8& bl,
                                         f32x4 c) {
     c = mfma16x16x32(a, bh, c);
     return mfma16x16x32(a, bl, c);
-}
-
-// Four consecutive features fr..fr+3 of sample `col` as (hi, mid, lo) triples,
-// sample-major.
-__device__ __forceinline__ void st_act3(uint16_t* sh, uint16_t* sm_, uint16_t* sl, int col,
-                                        int fr, const float* v) {
-    uint2 hi, mi, lo;
-    split3(v[0], v[1], hi.x, mi.x, lo.x);
-    split3(v[2], v[3], hi.y, mi.y, lo.y);
-    *reinterpret_cast<uint2*>(&sh[col * SM + fr]) = hi;
-    *reinterpret_cast<uint2*>(&sm_[col * SM + fr]) = mi;
-    *reinterpret_cast<uint2*>(&sl[col * SM + fr]) = lo;
 }
 
 // dW products (activation x gradient) use the hi parts only, and the backward
@@ -173,393 +154,439 @@ __device__ __forceinline__ float keep_if(uint32_t m, int k, float x) {
 }
 
 // ---- forward -----------------------------------------------------------------
-// A workgroup of 4 wavefronts takes a group of 32 records; wave w owns hidden
-// features [32w, 32w + 32) of both hidden layers (up to three workgroups per
-// CU).  X and H0 enter their products as (hi, mid, lo) triples, so the
-// pre-activations, and with them the ReLU masks the backward applies, carry
-// fp32 precision; H1 enters the logits as (hi, lo) pairs.  Per group, three
-// phases with a barrier after each:
-//   A  rgb of the previous group from its partial logits; X = [colour
-//      features | PE | 1] from the gather and view directions loaded during
-//      the previous group; the features are kept per record
-//   B  H0, then the next group's topology lookups and view-direction loads
-//   C  H1, then each wave's partial logits over its own 32 hidden features
-//      (it reads back only the H1 it wrote: no workgroup barrier between),
-//      then the next group's colour loads
-// The records are staged two groups ahead (flags and positions double-buffered
-// in LDS); W0^T and W1^T slices stay in registers, W2^T in LDS.  The ReLU
-// masks of both hidden layers are stored per record for the backward.
-struct RecInfo {
-    float x, y, z;
-    uint32_t bits;
-};
-
+// A wavefront takes a group of 32 records through the whole network by itself:
+// its activations never leave its registers, so there is no barrier and no
+// exchange between wavefronts once the weights are in LDS.  The D fragment of
+// v_mfma_f32_32x32x16_bf16 (lane (h, n), h = lane / 32: features
+// 32T + 8q + 4h + i of sample n, q, i < 4) is the next layer's B fragment when
+// that layer's weights are stored with their K index permuted to match:
+// position 8h + j of k-step 2T + t stands for feature
+// 32T + 16t + 8 (j / 4) + 4h + j % 4.  A weight fragment read from LDS (8 LDS
+// cycles) covers the three parts of the split activations: 96 cycles of its
+// SIMD's matrix core.  X and H0 enter their products as (hi, mid, lo) triples,
+// so the pre-activations, and with them the ReLU masks the backward applies,
+// carry fp32 precision; H1 enters the logits as (hi, lo) pairs.
+//
+// X has 40 columns (12 features, 27 encoding inputs, the bias input) in three
+// parts.  Stacked along K they are 15 chunks of 8 columns, two to a k-step, in
+// the order
+//   hi A, hi B | mid A, mid B | lo A, lo B | hi 2, hi 3 | hi 4, mid 2 |
+//   mid 3, mid 4 | lo 2, lo 3 | lo 4, ones
+// where chunk A is features 0..7, B features 8..11 and columns 12..15, and
+// 2..4 columns 8c..8c + 7; they sit in a tile of the wavefront's own in LDS.
+// The ones meet b0's own split, so the accumulators start at zero.
+//
+// The last group's rows past the records are stored like the others (the
+// workspace holds whole groups) and never read.
+//
+// A lane gathers four corners of its sample's colour, the other lane half the
+// other four.  The next group's leaf lookups are issued ahead of layer 0 and
+// its colour rows and encoding chunks from there to layer 1's end, so their
+// latency runs under the MFMAs; missing leaves and dead samples read rows of
+// zeros, which keeps the loop free of branches that the loads would wait in.
+//
+// What bounds it: a group is 132 MFMAs of 32 cycles of its SIMD's matrix core
+// (and 32 of 8) and about 1150 vector instructions of 4 cycles; two wavefronts
+// per SIMD (250 registers) overlap them in part.  32x32x16 MFMAs are half as many
+// to issue as 16x16x32 ones.  The splits stay an unpacking and a subtraction:
+// a dot-product instruction does both at once, but runs on the matrix core
+// and does not overlap with MFMAs.  The logits, 3 of 32 rows, use 4x4x4 MFMAs.
+//
+// Measured against four wavefronts that shared a group (32 hidden features each,
+// activations exchanged through LDS, three barriers a group): 7.80M records with
+// bf16 colour 2029 -> 982 us, 190k with fp32 colour 61.4 -> 36.8 us; 24k, one
+// group to a wavefront, 13.8 -> 14.8 us.  On 16x16x32 MFMAs 1204 us.  With the
+// gather in the march (features through memory) 900 us, and the march 485 us
+// instead of 224.
+constexpr int kFwdWaves = 4;
+constexpr int kXChunks = 15;
 struct alignas(16) SmemFwd {
-    uint16_t W2t[16 * 128];  // W2^T [16 logits (3 used)][128 hidden]
-    // X is read in phase B only and H1 in phase D only (a barrier between D
-    // and the next group's A), so they share storage
-    union {
-        struct {
-            uint16_t Xh[GS * XM], Xm[GS * XM], Xl[GS * XM];
-        } x;
-        struct {
-            uint16_t A2h[GS * SM], A2l[GS * SM];  // H1
-        } h1;
-    } u;
-    uint16_t A1h[GS * SM], A1m[GS * SM], A1l[GS * SM];  // H0
-    RecInfo ri[2][GS];
-    float4 plog[4][GS];  // each wave's partial logits (0..2) over its 32 hidden features
-    uint32_t pbits[GS];  // the flags of the group whose partial logits these are
+    uint4 w0[6 * 128];             // [chunk][hidden feature]: W0^T columns 8c .. 8c + 7; b0's split
+    uint4 w1[4 * 9 * 64];          // [row tile][step][lane]: b1's split, then W1^T's A
+                                   // fragments of the eight k-steps, K permuted
+    uint4 w2[8 * 2 * 4];           // W2^T rows [k-step][h][logit, zeros], K permuted
+    uint4 ones[2];                 // [h] the inputs that the biases' splits are multiplied with
+    uint4 x[kFwdWaves][GS][kXChunks];
 };
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + expf(-x)); }
 
+// v_mfma_f32_4x4x4_16b_bf16: sixteen 4 x 4 products, block lane / 4.  A lane
+// holds A[lane % 4][0..3] and B[0..3][lane % 4] of its block and gets
+// D[0..3][lane % 4]: for four logits' weights in A and its own sample's four
+// features in B, the lane's own logits.
+__device__ __forceinline__ f32x4 mfma4x4x4(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1,
+                                           const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, make_uint2(a0, a1)),
+                                                  __builtin_bit_cast(s16x4, make_uint2(b0, b1)), c,
+                                                  0, 0, 0);
+}
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ f32x16 mfma32x32x16(const uint4& a, const uint4& b, const f32x16& c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(a), as_bf8(b), c, 0, 0, 0);
+}
+
+// Pins the values' computation to this point: left alone, the compiler defers
+// it and keeps the activations that it comes from alive.
+__device__ __forceinline__ void pin(uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& d) {
+    asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+}
+
+__device__ __forceinline__ uint4 frag(const uint32_t (&d)[4]) {
+    return make_uint4(d[0], d[1], d[2], d[3]);
+}
+
+// Orders a wavefront's LDS writes before its own later reads.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// relu as an integer max: a float is > 0 exactly when its bits are > 0 as an
+// int, and the max keeps +NaN as torch's relu does (a float max would first
+// canonicalize the MFMA output).
+__device__ __forceinline__ float relu(float x) {
+    return __uint_as_float((uint32_t)max((int32_t)__float_as_uint(x), 0));
+}
+
+// The ReLU mask bits of a packed pair of relu'd bf16 values (their hi parts):
+// set where the value is not zero, pair p's at bits p and 16 + p.
+__device__ __forceinline__ void mask_pair(uint32_t hi, int p, uint32_t& word) {
+    uint32_t on;  // as packed integers: the generic form of this min is lowered lane by lane
+    asm("v_pk_min_u16 %0, %1, %2" : "=v"(on) : "v"(hi), "s"(0x00010001u));
+    word |= on << p;
+}
+
+// The network's weights into LDS, by the whole workgroup.
+__device__ __forceinline__ void stage_fwd_weights(SmemFwd& sm, const MlpPacked& W) {
+    static_assert(offsetof(SmemFwd, w1) == 2 * kImgW1 && offsetof(SmemFwd, w2) == 2 * kImgW2 &&
+                      offsetof(SmemFwd, ones) == 2 * kImgOnes && offsetof(SmemFwd, x) == 2 * kFwdImage,
+                  "the image is the struct's head");
+    uint4* dst = reinterpret_cast<uint4*>(&sm);
+#pragma unroll
+    for (int k = 0; k < (kFwdImage / 8 + 64 * kFwdWaves - 1) / (64 * kFwdWaves); ++k) {
+        const int e = 64 * kFwdWaves * k + (int)threadIdx.x;
+        if (e < kFwdImage / 8) dst[e] = W.fwd[e];
+    }
+}
+
 template <bool BF16COL>
-__global__ void __launch_bounds__(256, 3) k_mlp_fwd(StepParams P, TopoView topo, const void* color,
-                                                 MlpPacked W, RayBuffers R, Records rec) {
-    constexpr int MT = 2;  // 16-feature tiles per wave
+__global__ void __launch_bounds__(64 * kFwdWaves, 2)
+    k_mlp_fwd(StepParams P, TopoView topo, const void* color, MlpPacked W, RayBuffers R,
+              Records rec) {
     using Raw = std::conditional_t<BF16COL, uint2, float4>;  // one third of a colour row
     __shared__ SmemFwd sm;
-    const int tid = threadIdx.x;
-    const int wv = tid >> 6, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
-    const int f0 = 32 * wv;
-    const int pr = lane < GS / 4 ? wv * (GS / 4) + lane : -1;  // staging lanes
-    const int gs = tid >> 3, gpart = tid & 7;                  // gather: record, corner
-    const int ps = tid & (GS - 1), pp = tid >> 5;              // encoding: sample, part
-
-    // this wave's W0^T and W1^T slices in registers; W2^T in LDS
-    bf16x8 A0[MT][2], A1[MT][4];
-    float b0v[MT][4], b1v[MT][4], b2v[3];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const int row = f0 + 16 * mt + r16;
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) A0[mt][kt] = ld_frag(W.w0t + row * 64 + 32 * kt + 8 * g);
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) A1[mt][kt] = ld_frag(W.w1t + row * 128 + 32 * kt + 8 * g);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            b0v[mt][i] = W.b0[f0 + 16 * mt + 4 * g + i];
-            b1v[mt][i] = W.b1[f0 + 16 * mt + 4 * g + i];
-        }
-    }
-    b2v[0] = W.b2[0];
-    b2v[1] = W.b2[1];
-    b2v[2] = W.b2[2];
-    for (int e = tid; e < 16 * 128 / 8; e += 256)
-        reinterpret_cast<uint4*>(sm.W2t)[e] = reinterpret_cast<const uint4*>(W.w2t)[e];
-
+    // the wavefront's index as a scalar: record addresses are then scalar bases
+    // with lane offsets
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = lane_id(), n = lane & 31, h = lane >> 5;
     const int64_t total = min((int64_t)R.total[0], P.capacity);
+    if (total <= 0) return;
     const int64_t ngroups = (total + GS - 1) / GS;
-    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    // staging registers: a group's records (two groups ahead of the one computed)
-    float4 p_xyze = z4;
-    float2 p_ab = make_float2(0.f, 0.f);
-    auto stage = [&](int64_t grp) {
-        const int64_t q = grp * GS + pr;
-        p_xyze = z4;
-        p_ab = make_float2(0.f, 0.f);
-        if (pr >= 0 && grp < ngroups && q < total) {
-            p_xyze = rec.xyze[q];
-            p_ab = rec.ab[q];
-        }
-    };
-    auto commit = [&](int b) {
-        if (pr >= 0) {
-            RecInfo ri;
-            ri.x = p_xyze.x;
-            ri.y = p_xyze.y;
-            ri.z = p_xyze.z;
-            ri.bits = __float_as_uint(p_ab.y);  // zero for records past the end
-            sm.ri[b][pr] = ri;
-        }
-    };
-    // gather prefetch of the next group: this thread's corner of record gs
-    int64_t c_slot = -1;
-    float c_sc = 0.f;
-    Raw c_raw[3];
-    uint2 pe_h = make_uint2(0u, 0u), pe_m = pe_h, pe_l = pe_h;  // sample ps's X columns 12 + 4pp ..
-    auto lookup = [&](int b) {  // topology and view direction (after the records' barrier)
-        const RecInfo ri = sm.ri[b][gs];
-        c_slot = -1;
-        c_sc = 0.f;
-        if (ri.bits & kAliveW) {
-            const Cell cell = make_cell(ri.x, ri.y, ri.z);
-            const int dx = (kCx >> gpart) & 1, dy = (kCy >> gpart) & 1, dz = (kCz >> gpart) & 1;
-            const float a = dx ? cell.u : 1.f - cell.u;
-            const float bb = dy ? cell.v : 1.f - cell.v;
-            const float d = dz ? cell.w : 1.f - cell.w;
-            c_sc = (a * bb) * d;
-            c_slot = slot_of(topo, cell.i0 + dx, cell.j0 + dy, cell.k0 + dz);
-        }
-        // the encoding columns of sample ps from its ray's row (the counting
-        // march wrote them), zero for a sample that is not weight-kept
-        const uint32_t pb = sm.ri[b][ps].bits;
-        pe_h = pe_m = pe_l = make_uint2(0u, 0u);
-        if ((pb & kAliveW) && pp < 7) {
-            const uint2* row = reinterpret_cast<const uint2*>(R.pe + 96 * (int64_t)(pb & kRayMask));
-            pe_h = row[pp];
-            pe_m = row[8 + pp];
-            pe_l = row[16 + pp];
-        }
-    };
-    auto fetch = [&]() {  // the colour row of the looked-up corner
-        if constexpr (BF16COL) {
-            c_raw[0] = c_raw[1] = c_raw[2] = make_uint2(0u, 0u);
-            if (c_slot >= 0) {
-                const uint2* src = reinterpret_cast<const uint2*>(
-                    reinterpret_cast<const uint16_t*>(color) + c_slot * 12);
-                c_raw[0] = src[0];
-                c_raw[1] = src[1];
-                c_raw[2] = src[2];
-            }
-        } else {
-            c_raw[0] = c_raw[1] = c_raw[2] = z4;
-            if (c_slot >= 0) {
-                const float4* src = reinterpret_cast<const float4*>(
-                    reinterpret_cast<const float*>(color) + c_slot * 12);
-                c_raw[0] = src[0];
-                c_raw[1] = src[1];
-                c_raw[2] = src[2];
-            }
-        }
-    };
+    const int64_t stride = (int64_t)gridDim.x * kFwdWaves;
+    uint4* const xr = sm.x[wv][n];  // this lane's sample
+    const uint4* const xlast = h ? &sm.ones[0] : &xr[14];
+    // W0 fragments: this lane's rows of the k-steps' chunk pairs (A, B), (2, 3),
+    // (4, 2), (3, 4) and (4, bias)
+    const uint4* const w0ab = sm.w0 + 128 * h + n;
+    const uint4* const w023 = sm.w0 + 128 * (2 + h) + n;
+    const uint4* const w042 = sm.w0 + 128 * (4 - 2 * h) + n;
+    const uint4* const w034 = sm.w0 + 128 * (3 + h) + n;
+    const uint4* const w04b = sm.w0 + 128 * (4 + h) + n;
+    const uint4* const w1p = sm.w1 + lane;
+    const uint4* const w2p = sm.w2 + 4 * h + (n & 3);
 
-    stage(blockIdx.x);
-    commit(0);
-    stage((int64_t)blockIdx.x + gridDim.x);
-    __syncthreads();
-    lookup(0);
-    fetch();
-    int cb = 0;  // buffer of the current group's records
-    // rgb of a group from the four waves' partial logits (summed in wave
-    // order), written by the threads of its 32 samples
-    auto finish_rgb = [&](int64_t pbase) {
-        if (tid < GS) {
-            const int64_t q = pbase + tid;
-            if (q < total) {
-                const float4 l0 = sm.plog[0][tid], l1 = sm.plog[1][tid], l2 = sm.plog[2][tid],
-                             l3 = sm.plog[3][tid];
-                const bool alive = (sm.pbits[tid] & kAliveW) != 0u;
-                rec.rgb[q] = alive ? make_float4(sigmoidf_(((l0.x + l1.x) + l2.x) + l3.x + b2v[0]),
-                                                 sigmoidf_(((l0.y + l1.y) + l2.y) + l3.y + b2v[1]),
-                                                 sigmoidf_(((l0.z + l1.z) + l2.z) + l3.z + b2v[2]),
-                                                 0.f)
-                                   : z4;
+    const int32_t* const none = reinterpret_cast<const int32_t*>(R.zero + 12);  // a leaf index of -1
+    // the group two ahead: its records (position, flags); zero flags past the end
+    float rx, ry, rz;
+    uint32_t rbits;
+    auto load_records = [&](int64_t grp) {
+        const int64_t q0 = min(grp, ngroups - 1) * GS;
+        const float4 p = (rec.xyze + q0)[n];
+        rx = p.x;
+        ry = p.y;
+        rz = p.z;
+        const uint32_t b = __float_as_uint((rec.ab + q0)[n].y);
+        rbits = n < total - q0 ? b : 0u;
+    };
+    // the next group: the leaves (-1: none), voxel offsets and weights of this
+    // lane's four corners (4h .. 4h + 3 of the corner walk: x offset h, the y
+    // and z offsets mirrored in y), and the flags
+    int32_t leaf[4];
+    uint32_t off[2];  // two to a word
+    float sc[4];
+    uint32_t nbits;
+    auto lookup = [&]() {
+        nbits = rbits;
+        const bool alive = (rbits & kAliveW) != 0u;
+        const Cell cell = make_cell(rx, ry, rz);
+        const float a = h ? cell.u : 1.f - cell.u;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int dy = (c >> 1) ^ h, dz = (c & 1) ^ (c >> 1);
+            const float b = dy ? cell.v : 1.f - cell.v;
+            sc[c] = (a * b) * (dz ? cell.w : 1.f - cell.w);
+            const int i = cell.i0 + h, j = cell.j0 + dy, k = cell.k0 + dz;
+            const uint32_t vo = (uint32_t)voxel_offset(i, j, k);
+            off[c >> 1] = (c & 1) ? off[c >> 1] | (vo << 16) : vo;
+            if (topo.two_level) {  // uniform over the grid
+                leaf[c] = alive ? leaf_of(topo, i, j, k) : -1;
+            } else {  // leaf_of's lookup with a selected address instead of a branch
+                const int la = (i >> 3) - topo.lo0, lb = (j >> 3) - topo.lo1, lc = (k >> 3) - topo.lo2;
+                const bool inside = alive && (unsigned)la < (unsigned)topo.d0 &&
+                                    (unsigned)lb < (unsigned)topo.d1 && (unsigned)lc < (unsigned)topo.d2;
+                const int32_t* e = topo.table + ((la * topo.d1 + lb) * topo.d2 + lc);
+                leaf[c] = *(inside ? e : none);
             }
         }
     };
-    int64_t pbase = -1;  // the group whose partial logits wait in plog (-1: none)
-
-    for (int64_t grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {  // uniform bound
-        const int64_t base = grp * GS;
-        // ---- A. the previous group's rgb; X = [colour features (12) | PE (27) | 1 | 0...];
-        //         stage the records ----
-        if (pbase >= 0) finish_rgb(pbase);
-        {
-            // trilinear colour: corner gpart's row times its weight, summed over
-            // the record's 8 threads (zero where the record or corner is absent)
-            float v[12];
+    // colour rows of corners 2 pair, 2 pair + 1 (a missing leaf reads the row of zeros)
+    Raw raw[2][3];
+    auto fetch = [&](int pair, Raw (&raw)[2][3]) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int32_t lf = leaf[2 * pair + c];
+            const Raw* src =
+                lf >= 0 ? reinterpret_cast<const Raw*>(color) +
+                              3 * ((int64_t)lf * 512 + ((off[pair] >> (16 * c)) & 0xffffu))
+                        : reinterpret_cast<const Raw*>(R.zero);
+            raw[c][0] = src[0];
+            raw[c][1] = src[1];
+            raw[c][2] = src[2];
+        }
+    };
+    // w[c] = the pair's weighted colour
+    auto weigh = [&](int pair, const Raw (&raw)[2][3], float (&w)[12]) {
+        const float s0 = sc[2 * pair], s1 = sc[2 * pair + 1];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            float4 c0, c1;
             if constexpr (BF16COL) {
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    v[4 * k + 0] = bf_lo(c_raw[k].x) * c_sc;
-                    v[4 * k + 1] = bf_hi(c_raw[k].x) * c_sc;
-                    v[4 * k + 2] = bf_lo(c_raw[k].y) * c_sc;
-                    v[4 * k + 3] = bf_hi(c_raw[k].y) * c_sc;
-                }
+                c0 = make_float4(bf_lo(raw[0][k].x), bf_hi(raw[0][k].x), bf_lo(raw[0][k].y),
+                                 bf_hi(raw[0][k].y));
+                c1 = make_float4(bf_lo(raw[1][k].x), bf_hi(raw[1][k].x), bf_lo(raw[1][k].y),
+                                 bf_hi(raw[1][k].y));
             } else {
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    v[4 * k + 0] = c_raw[k].x * c_sc;
-                    v[4 * k + 1] = c_raw[k].y * c_sc;
-                    v[4 * k + 2] = c_raw[k].z * c_sc;
-                    v[4 * k + 3] = c_raw[k].w * c_sc;
-                }
+                c0 = raw[0][k];
+                c1 = raw[1][k];
             }
-            // butterfly over the record's eight lanes on the DPP path (folded
-            // into the adds): lanes l^1 and l^2 by quad permutes, then the
-            // other quad of the eight by the half-row mirror (lane j of the
-            // eight reads lane 7 - j, which holds the other quad's sum)
-#pragma unroll
-            for (int c = 0; c < 12; ++c)
-                v[c] += __uint_as_float(dpp<0xB1>(__float_as_uint(v[c])));  // quad_perm [1,0,3,2]
-#pragma unroll
-            for (int c = 0; c < 12; ++c)
-                v[c] += __uint_as_float(dpp<0x4E>(__float_as_uint(v[c])));  // quad_perm [2,3,0,1]
-#pragma unroll
-            for (int c = 0; c < 12; ++c)
-                v[c] += __uint_as_float(dpp<0x141>(__float_as_uint(v[c])));  // row_half_mirror
-            // the butterfly leaves the same twelve sums (bit for bit: each step
-            // adds the same two operands on every lane) in all eight lanes of
-            // the record, so lane gpart < 6 splits and stores channel pair gpart
-            if (gpart < 6) {
-                float a = v[0], b = v[1];
-#pragma unroll
-                for (int c = 1; c < 6; ++c) {
-                    a = gpart == c ? v[2 * c] : a;
-                    b = gpart == c ? v[2 * c + 1] : b;
-                }
-                uint32_t wh, wm, wl;
-                split3(a, b, wh, wm, wl);
-                reinterpret_cast<uint32_t*>(&sm.u.x.Xh[gs * XM])[gpart] = wh;
-                reinterpret_cast<uint32_t*>(&sm.u.x.Xm[gs * XM])[gpart] = wm;
-                reinterpret_cast<uint32_t*>(&sm.u.x.Xl[gs * XM])[gpart] = wl;
-                // the backward's input row, features part (X columns 0..11, hi)
-                const int64_t qq = base + gs;
-                if (qq < total) reinterpret_cast<uint32_t*>(rec.xrow + 5 * qq)[gpart] = wh;
-            }
+            w[4 * k + 0] = c0.x * s0 + c1.x * s1;
+            w[4 * k + 1] = c0.y * s0 + c1.y * s1;
+            w[4 * k + 2] = c0.z * s0 + c1.z * s1;
+            w[4 * k + 3] = c0.w * s0 + c1.w * s1;
         }
-        {
-            // positional encoding (dvgo.py:354-358) and the bias column: thread
-            // (sample ps, part pp < 7) writes X columns 12 + 4pp .. +3, as (hi,
-            // mid, lo) bf16 from its ray's encoding row
-            const uint2 hi = pe_h, mi = pe_m, lo = pe_l;
-            if (pp < 7) {
-                *reinterpret_cast<uint2*>(&sm.u.x.Xh[ps * XM + 12 + 4 * pp]) = hi;
-                *reinterpret_cast<uint2*>(&sm.u.x.Xm[ps * XM + 12 + 4 * pp]) = mi;
-                *reinterpret_cast<uint2*>(&sm.u.x.Xl[ps * XM + 12 + 4 * pp]) = lo;
-                // the backward's input row, encoding part (X columns 12 + 4pp .. +3)
-                const int64_t qq = base + ps;
-                if (qq < total)
-                    reinterpret_cast<uint2*>(rec.xrow + 5 * qq)[3 + pp] = hi;
-            } else {
-                // X columns 40..63 (zero weights) are zeroed for every group: H1
-                // of the previous group shares their storage
-                const uint4 zz = make_uint4(0u, 0u, 0u, 0u);
+    };
+    // the encoding chunks of the sample's ray (zeros unless it is weight-kept): this
+    // lane's halves of k-steps 3..7, and chunk B's columns
+    u32x4 pe[5];
+    uint2 peb[2];
+    auto fetch_pe = [&]() {
+        const u32x4* row = reinterpret_cast<const u32x4*>(
+            nbits & kAliveW ? R.pe + 96 * (int64_t)(nbits & kRayMask)
+                            : reinterpret_cast<const uint16_t*>(R.zero));
+        pe[0] = row[1 + h];
+        pe[1] = row[3 + 2 * h];
+        pe[2] = row[6 + h];
+        pe[3] = row[9 + h];
+        pe[4] = row[11];
+        peb[0] = reinterpret_cast<const uint2*>(row + 4 * h)[1];
+        peb[1] = reinterpret_cast<const uint2*>(row + 8 - 4 * h)[1];
+    };
+    // the sample's X into the wavefront's tile: v holds this lane's four corners
+    auto store_x = [&](float (&v)[12]) {
+        // the two lane halves' sums: a swap exchanges half of one value's lanes
+        // for half of another's, which leaves half h with features 6h .. 6h + 5
+        uint32_t hi[3], mi[3], lo[3];
 #pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    *reinterpret_cast<uint4*>(&sm.u.x.Xh[ps * XM + 40 + 8 * k]) = zz;
-                    *reinterpret_cast<uint4*>(&sm.u.x.Xm[ps * XM + 40 + 8 * k]) = zz;
-                    *reinterpret_cast<uint4*>(&sm.u.x.Xl[ps * XM + 40 + 8 * k]) = zz;
-                }
-            }
-        }
-        commit(cb ^ 1);                 // the next group's records
-        stage(grp + 2 * (int64_t)gridDim.x);  // and the one after's loads
-        __syncthreads();
-        // ---- B. H0^T slice = relu(W0^T X^T + b0) -> A1; next group's lookups ----
-        // k-step outer: each B fragment is read once and the (mt, nt) chains interleave
-        // the accumulators start at the bias (the MFMA adds it, no separate pass)
-        f32x4 acc[MT][NT];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                acc[mt][nt] = f32x4{b0v[mt][0], b0v[mt][1], b0v[mt][2], b0v[mt][3]};
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const int xo = (16 * nt + r16) * XM + 32 * kt + 8 * g;
-                const bf16x8 bp[3] = {ld_frag(&sm.u.x.Xh[xo]), ld_frag(&sm.u.x.Xm[xo]),
-                                      ld_frag(&sm.u.x.Xl[xo])};
-#pragma unroll
-                for (int part = 0; part < 3; ++part)
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        acc[mt][nt] = mfma16x16x32(A0[mt][kt], bp[part], acc[mt][nt]);
-            }
-        }
-        uint32_t nib[MT][NT];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                float h[4];
-                nib[mt][nt] = 0u;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    // relu as an integer select on one integer compare, which
-                    // also gives the mask bit: a float is > 0 exactly when its
-                    // bits are > 0 as an int (a float max would first
-                    // canonicalize the MFMA output, one more instruction per
-                    // value; +NaN passes through, as torch's relu passes NaN)
-                    const uint32_t hb = __float_as_uint(acc[mt][nt][i]);
-                    const bool on = (int32_t)hb > 0;
-                    h[i] = __uint_as_float(on ? hb : 0u);
-                    nib[mt][nt] |= (on ? 1u : 0u) << i;
-                }
-                st_act3(sm.A1h, sm.A1m, sm.A1l, 16 * nt + r16, f0 + 16 * mt + 4 * g, h);
-            }
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int64_t q = base + 16 * nt + r16;
-            if (q < total)
-                reinterpret_cast<uint8_t*>(rec.relu + 8 * q + wv)[g] = relu_byte(nib[0][nt], nib[1][nt]);
-        }
-        lookup(cb ^ 1);
-        __syncthreads();
-        // ---- C. H1^T slice = relu(W1^T H0^T + b1) -> A2; next group's colour loads ----
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                acc[mt][nt] = f32x4{b1v[mt][0], b1v[mt][1], b1v[mt][2], b1v[mt][3]};
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const int ho = (16 * nt + r16) * SM + 32 * kt + 8 * g;
-                const bf16x8 bp[3] = {ld_frag(&sm.A1h[ho]), ld_frag(&sm.A1m[ho]),
-                                      ld_frag(&sm.A1l[ho])};
-#pragma unroll
-                for (int part = 0; part < 3; ++part)
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        acc[mt][nt] = mfma16x16x32(A1[mt][kt], bp[part], acc[mt][nt]);
-            }
+        for (int c = 0; c < 6; ++c) {
+            const auto r = __builtin_amdgcn_permlane32_swap(
+                __float_as_uint(v[c]), __float_as_uint(v[c + 6]), false, false);
+            v[c] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
         }
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int p = 0; p < 3; ++p) split3(v[2 * p], v[2 * p + 1], hi[p], mi[p], lo[p]);
+        uint32_t* f = reinterpret_cast<uint32_t*>(xr) + 3 * h;
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                float h[4];
-                nib[mt][nt] = 0u;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    // relu as an integer select on one integer compare, which
-                    // also gives the mask bit: a float is > 0 exactly when its
-                    // bits are > 0 as an int (a float max would first
-                    // canonicalize the MFMA output, one more instruction per
-                    // value; +NaN passes through, as torch's relu passes NaN)
-                    const uint32_t hb = __float_as_uint(acc[mt][nt][i]);
-                    const bool on = (int32_t)hb > 0;
-                    h[i] = __uint_as_float(on ? hb : 0u);
-                    nib[mt][nt] |= (on ? 1u : 0u) << i;
-                }
-                st_act<false>(sm.u.h1.A2h, sm.u.h1.A2l, nullptr, 16 * nt + r16, f0 + 16 * mt + 4 * g,
-                              lane, h);
-            }
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int64_t q = base + 16 * nt + r16;
-            if (q < total)
-                reinterpret_cast<uint8_t*>(rec.relu + 8 * q + 4 + wv)[g] =
-                    relu_byte(nib[0][nt], nib[1][nt]);
+        for (int p = 0; p < 3; ++p) {
+            f[p] = hi[p];
+            f[8 + p] = mi[p];
+            f[16 + p] = lo[p];
         }
-        // partial logits over this wave's hidden features f0 .. f0 + 31 (one
-        // k-step of L^T = W2^T H1^T), read back from the H1 this wave just wrote
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        {
-            const bf16x8 w2 = ld_frag(&sm.W2t[r16 * 128 + f0 + 8 * g]);
+        uint2* b = reinterpret_cast<uint2*>(xr) + 3;  // chunk B's half of part p: b[4 p]
+        b[4 * h] = peb[0];
+        b[8 - 4 * h] = peb[1];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const int ho = (16 * nt + r16) * SM + f0 + 8 * g;
-                f32x4 a5 = {0.f, 0.f, 0.f, 0.f};
-                a5 = mfma_w(w2, ld_frag(&sm.u.h1.A2h[ho]), ld_frag(&sm.u.h1.A2l[ho]), a5);
-                if (g == 0) sm.plog[wv][16 * nt + r16] = make_float4(a5[0], a5[1], a5[2], 0.f);
-            }
-        }
-        if (tid < GS) sm.pbits[tid] = sm.ri[cb][tid].bits;
-        pbase = base;
-        fetch();
-        __syncthreads();
-        cb ^= 1;
+        for (int t = 0; t < 4; ++t) reinterpret_cast<u32x4*>(xr)[6 + 2 * t + h] = pe[t];
+        if (h == 0) reinterpret_cast<u32x4*>(xr)[14] = pe[4];
+    };
+
+    int64_t grp = (int64_t)wv * gridDim.x + blockIdx.x;
+    load_records(grp);
+    stage_fwd_weights(sm, W);  // behind the first records' loads
+    lookup();
+    load_records(grp + stride);
+    float v[12];  // the next group's colour: this lane's corners, a pair at a time
+    {
+        float w[12];
+        Raw raw1[2][3];  // one round trip for both pairs
+        fetch(0, raw);
+        fetch(1, raw1);
+        fetch_pe();
+        weigh(0, raw, v);
+        weigh(1, raw1, w);
+#pragma unroll
+        for (int c = 0; c < 12; ++c) v[c] += w[c];
+        store_x(v);
     }
-    if (pbase >= 0) finish_rgb(pbase);  // the loop ended on a barrier
+    __syncthreads();  // the weights; from here on the wavefronts run on their own
+    const float b2a = W.b2[h], b2b = W.b2[2];
+
+    for (; grp < ngroups; grp += stride) {
+        const int64_t q0 = grp * GS;
+        const bool alive = (nbits & kAliveW) != 0u;
+        uint4 xb[8];  // this group's X fragments
+#pragma unroll
+        for (int t = 0; t < 7; ++t) xb[t] = xr[2 * t + h];
+        xb[7] = *xlast;
+        {  // the backward's input row: X columns 0..39 (hi)
+            uint4* row = rec.xrow + 5 * q0 + 5 * n;
+            row[h] = xb[0];
+            row[2 + h] = xb[3];
+            // half 1 stores chunk 3 a second time
+            row[4 - h] = make_uint4(h ? xb[3].x : xb[4].x, h ? xb[3].y : xb[4].y,
+                                    h ? xb[3].z : xb[4].z, h ? xb[3].w : xb[4].w);
+        }
+        lookup();
+        load_records(grp + 2 * stride);
+        // A tile's MFMAs run in eight slots; the vector instructions of a slot
+        // turn one pair of the tile before (relu, mask, split) into the next
+        // layer's B fragments while the matrix core works, and every weight
+        // fragment is read two steps ahead of its use.  The scheduling barriers
+        // keep the compiler from gathering either kind together again.
+        uint32_t mask0[2] = {0u, 0u}, mask1[2] = {0u, 0u};  // words h and h + 2 (q even, odd)
+        uint32_t h0[8][3][4];  // layer 1's B fragments [k-step][part][dword]
+        uint32_t h1[2][4];     // layer 2's of one k-step
+        f32x16 c, d;           // a tile in the making, the one before
+        f32x4 lg = {0.f, 0.f, 0.f, 0.f};  // the sample's logits over this lane's features
+        const f32x16 zero = {};
+        auto pair0 = [&](int T, int j) {  // pair j (rows 2j, 2j + 1 of the lane) of tile T
+            uint32_t(*f)[4] = h0[2 * T + (j >> 2)];
+            split3(relu(d[2 * j]), relu(d[2 * j + 1]), f[0][j & 3], f[1][j & 3], f[2][j & 3]);
+            mask_pair(f[0][j & 3], 2 * (2 * T + (j >> 2)) + (j & 1), mask0[(j >> 1) & 1]);
+            pin(f[0][j & 3], f[1][j & 3], f[2][j & 3], mask0[(j >> 1) & 1]);
+        };
+        uint4 w2f;
+        auto pair1 = [&](int T, int j) {
+            if ((j & 3) == 1) w2f = w2p[8 * (2 * T + (j >> 2))];
+            split2(relu(d[2 * j]), relu(d[2 * j + 1]), h1[0][j & 3], h1[1][j & 3]);
+            mask_pair(h1[0][j & 3], 2 * (2 * T + (j >> 2)) + (j & 1), mask1[(j >> 1) & 1]);
+            pin(h1[0][j & 3], h1[1][j & 3], mask1[0], mask1[1]);
+            if ((j & 3) == 3) {  // layer 2's k-step 2T + j / 4
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    lg = mfma4x4x4(w2f.x, w2f.y, h1[p][0], h1[p][1], lg);
+                    lg = mfma4x4x4(w2f.z, w2f.w, h1[p][2], h1[p][3], lg);
+                }
+            }
+        };
+        // ---- layer 0: H0^T = relu(W0^T X^T + b0) ----
+        uint4 fa = w0ab[0], fb = w023[0];
+#pragma unroll
+        for (int T = 0; T < 4; ++T) {
+            if (T == 3) fetch(0, raw);  // the next group's inputs, from here to layer 1's end
+            const uint4 f2 = w042[32 * T];
+            c = mfma32x32x16(fa, xb[0], zero);
+            if (T > 0) pair0(T - 1, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            c = mfma32x32x16(fa, xb[1], c);
+            if (T > 0) pair0(T - 1, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            const uint4 f3 = w034[32 * T];
+            c = mfma32x32x16(fa, xb[2], c);
+            if (T > 0) pair0(T - 1, 2);
+            __builtin_amdgcn_sched_barrier(0);
+            c = mfma32x32x16(fb, xb[3], c);
+            if (T > 0) pair0(T - 1, 3);
+            __builtin_amdgcn_sched_barrier(0);
+            const uint4 f4 = w04b[32 * T];
+            c = mfma32x32x16(fb, xb[6], c);
+            if (T > 0) pair0(T - 1, 4);
+            __builtin_amdgcn_sched_barrier(0);
+            fa = T < 3 ? w0ab[32 * (T + 1)] : w1p[0];
+            c = mfma32x32x16(f2, xb[4], c);
+            if (T > 0) pair0(T - 1, 5);
+            __builtin_amdgcn_sched_barrier(0);
+            fb = T < 3 ? w023[32 * (T + 1)] : w1p[64];
+            c = mfma32x32x16(f3, xb[5], c);
+            if (T > 0) pair0(T - 1, 6);
+            __builtin_amdgcn_sched_barrier(0);
+            c = mfma32x32x16(f4, xb[7], c);
+            if (T > 0) pair0(T - 1, 7);
+            __builtin_amdgcn_sched_barrier(0);
+            d = c;
+        }
+        // ---- layer 1: H1^T = relu(W1^T H0^T + b1); layer 2 over its tiles ----
+#pragma unroll
+        for (int T = 0; T < 4; ++T) {
+            uint4 fn = w1p[64 * (9 * T + 2)];
+            if (T == 1) {
+                weigh(0, raw, v);
+                fetch(1, raw);
+            }
+            if (T == 3) {
+                float w[12];
+                weigh(1, raw, w);
+#pragma unroll
+                for (int i = 0; i < 12; ++i) v[i] += w[i];
+                fetch_pe();
+            }
+            c = mfma32x32x16(fa, sm.ones[h], zero);
+            fa = fb;
+            fb = fn;
+#pragma unroll
+            for (int ks = 0; ks < 8; ++ks) {
+                fn = w1p[64 * min(9 * T + ks + 3, 35)];
+                c = mfma32x32x16(fa, frag(h0[ks][0]), c);
+                c = mfma32x32x16(fa, frag(h0[ks][1]), c);
+                c = mfma32x32x16(fa, frag(h0[ks][2]), c);
+                fa = fb;
+                fb = fn;
+                if (T > 0) {
+                    pair1(T - 1, ks);
+                } else if (ks < 4) {  // the last layer-0 tile is k-steps 6 and 7's input
+                    pair0(3, 2 * ks);
+                    pair0(3, 2 * ks + 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            d = c;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) pair1(3, j);
+        store_x(v);
+        wave_lds_fence();
+        // ---- the masks and rgb ----
+        {
+            uint32_t* mw = rec.relu + 8 * q0 + 8 * n + h;
+            mw[0] = mask0[0];
+            mw[2] = mask0[1];
+            mw[4] = mask1[0];
+            mw[6] = mask1[1];
+            // the two lane halves' sums: half h is left with logit h, both with
+            // logit 2; half h finishes channel h, half 0
+            // channel 2 too (half 1 writes the unused fourth)
+            const auto r01 = __builtin_amdgcn_permlane32_swap(
+                __float_as_uint(lg[0]), __float_as_uint(lg[1]), false, false);
+            const float x = __uint_as_float(r01[0]) + __uint_as_float(r01[1]);
+            const float y = lg[2] + __shfl_xor(lg[2], 32, 64);
+            const float a = sigmoidf_(x + b2a), b = sigmoidf_(y + b2b);
+            float* rgb = reinterpret_cast<float*>(rec.rgb + q0) + 4 * n + h;
+            rgb[0] = alive ? a : 0.f;
+            rgb[2] = alive && h == 0 ? b : 0.f;
+        }
+    }
 }
 
 // Backward weights as MFMA A fragments in LDS, [tile][k-step][lane] (each
@@ -795,14 +822,15 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
         // ---- 1. this group's stage A: H0^T slice = W0^T X^T + b0 under the
         //         forward's mask -> A1h, H0f; g_H1^T slice = W2[slice] g_L^T under
         //         the mask -> G1h, G1l, G1f.  The previous group's stage C ----
-        uint32_t m0 = 0u, m1 = 0u;  // the forward's ReLU masks: bit nt * 4 + i
+        uint32_t m0 = 0u, m1 = 0u;  // the forward's ReLU masks: bit at(nt, i)
+        auto at = [](int nt, int i) { return 16 * (i & 1) + 2 * nt + (i >> 1); };
         {
-            const int sh = 8 * g + 4 * (wv & 1);  // features fr..fr+3 in word wv/2
+            // features fr..fr+3: bits 2wv, 16 + 2wv, 2wv + 1, 17 + 2wv of word g
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 const uint32_t* mw = &sm.relu[cb][8 * (16 * nt + r16)];
-                m0 |= ((mw[wv >> 1] >> sh) & 0xFu) << (nt * 4);
-                m1 |= ((mw[4 + (wv >> 1)] >> sh) & 0xFu) << (nt * 4);
+                m0 |= ((mw[g] >> (2 * wv)) & 0x30003u) << (nt * 2);
+                m1 |= ((mw[4 + g] >> (2 * wv)) & 0x30003u) << (nt * 2);
             }
         }
         f32x4 acc[NT];  // starting at the bias, as in the forward
@@ -827,7 +855,7 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
                 float gv[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    gv[i] = keep_if(m1, nt * 4 + i, c4[i]);
+                    gv[i] = keep_if(m1, at(nt, i), c4[i]);
                     db1[i] += gv[i];
                 }
                 st_act<true>(sm.G1h, sm.G1l, sm.G1f, 16 * nt + r16, fr, lane, gv);
@@ -837,7 +865,7 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
         for (int nt = 0; nt < NT; ++nt) {
             float h[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) h[i] = keep_if(m0, nt * 4 + i, acc[nt][i]);
+            for (int i = 0; i < 4; ++i) h[i] = keep_if(m0, at(nt, i), acc[nt][i]);
             st_hi_fm(sm.A1h, sm.H0f, 16 * nt + r16, fr, lane, h);
         }
         if (pbase >= 0) finish(cb ^ 1, pbase);
@@ -871,14 +899,14 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
             }
         }
         {
-            // g_H0 masked by the layer-0 word of features 32 fb .. +31
-            const uint32_t mw = sm.relu[cb][8 * (16 * sh + r16) + fb];
+            // g_H0 masked by the layer-0 bits of features 32 fb .. +31
+            const uint32_t mw = sm.relu[cb][8 * (16 * sh + r16) + g] >> (4 * fb);
 #pragma unroll
             for (int mt = 0; mt < 2; ++mt) {
                 float gv[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    gv[i] = keep_if(mw, 8 * g + 4 * mt + i, acc2[mt][i]);
+                    gv[i] = keep_if(mw, 16 * (i & 1) + 2 * mt + (i >> 1), acc2[mt][i]);
                 st_act<true>(sm.A2h, sm.A2l, sm.F3, 16 * sh + r16, 32 * fb + 16 * mt + 4 * g, lane,
                              gv);
             }
@@ -897,7 +925,7 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
         for (int nt = 0; nt < NT; ++nt) {
             float h[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) h[i] = keep_if(m1, nt * 4 + i, acc[nt][i]);
+            for (int i = 0; i < 4; ++i) h[i] = keep_if(m1, at(nt, i), acc[nt][i]);
             st_fm(sm.F2, 16 * nt + r16, fr, lane, h);
         }
         park(cb ^ 1);  // the next group's records, loaded at this group's start
@@ -981,10 +1009,8 @@ int launch_mlp(bool bwd, bool bf16col, int grid, const StepParams& P, const Topo
                            dw_partial);
         PVDB_LAUNCHED("k_mlp_bwd");
     } else {
-        if (bf16col)
-            hipLaunchKernelGGL((k_mlp_fwd<true>), dim3(grid), dim3(256), 0, s, P, t, color, W, R, rec);
-        else
-            hipLaunchKernelGGL((k_mlp_fwd<false>), dim3(grid), dim3(256), 0, s, P, t, color, W, R, rec);
+        const auto kernel = bf16col ? k_mlp_fwd<true> : k_mlp_fwd<false>;
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * kFwdWaves), 0, s, P, t, color, W, R, rec);
         PVDB_LAUNCHED("k_mlp_fwd");
     }
     return PVDB_OK;

@@ -51,15 +51,16 @@ inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintp
 
 struct Layout {
     size_t count, offset, total, t_last, ray_out, ray_grad, ray_ctot, ray_loss, ray_rgb, loss, steps,
-        pe, setup;
+        pe, setup, zero;
     size_t xyze, ab, rgb, adj, xrow, relu, grad;
-    size_t touched, dw_part, w0t, w1t, w2t, w2, w1, w0;
+    size_t touched, dw_part, w0t, w1t, fwd, w2, w1, w0;
     size_t bytes;
 };
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
-Layout layout_for(int64_t n_rays, int64_t capacity, int64_t nleaf) {
+Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
+    const int64_t capacity = (records + 31) & ~int64_t(31);  // whole groups of the forward MLP
     Layout L;
     size_t o = 0;
     auto take = [&](size_t bytes) {
@@ -80,6 +81,7 @@ Layout layout_for(int64_t n_rays, int64_t capacity, int64_t nleaf) {
     L.steps = take(2 * (size_t)kStepCache * n_rays);
     L.pe = take(2 * 96 * (size_t)n_rays);
     L.setup = take(32 * (size_t)n_rays);
+    L.zero = take(256);
     L.xyze = take(16 * capacity);
     L.ab = take(8 * capacity);
     L.rgb = take(16 * capacity);
@@ -91,7 +93,7 @@ Layout layout_for(int64_t n_rays, int64_t capacity, int64_t nleaf) {
     L.dw_part = take((size_t)4 * kPartStride * kMaxMlpGrid);
     L.w0t = take(2 * 128 * 64);
     L.w1t = take(2 * 128 * 128);
-    L.w2t = take(2 * 16 * 128);
+    L.fwd = take(2 * kFwdImage);
     L.w2 = take(2 * 128 * 32);
     L.w1 = take(2 * 128 * 128);
     L.w0 = take(2 * 16 * 128);
@@ -554,6 +556,7 @@ int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
     R.steps = reinterpret_cast<uint16_t*>(ws + L.steps);
     R.pe = direct ? nullptr : reinterpret_cast<uint16_t*>(ws + L.pe);
     R.setup = reinterpret_cast<float4*>(ws + L.setup);
+    R.zero = reinterpret_cast<const uint4*>(ws + L.zero);
     Records rec;
     rec.xyze = reinterpret_cast<float4*>(ws + L.xyze);
     rec.ab = reinterpret_cast<float2*>(ws + L.ab);
@@ -566,14 +569,14 @@ int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
     float* dw_part = reinterpret_cast<float*>(ws + L.dw_part);
     uint16_t* w0t = reinterpret_cast<uint16_t*>(ws + L.w0t);
     uint16_t* w1t = reinterpret_cast<uint16_t*>(ws + L.w1t);
-    uint16_t* w2t = reinterpret_cast<uint16_t*>(ws + L.w2t);
+    uint16_t* fwd = reinterpret_cast<uint16_t*>(ws + L.fwd);
     uint16_t* w2 = reinterpret_cast<uint16_t*>(ws + L.w2);
     uint16_t* w1 = reinterpret_cast<uint16_t*>(ws + L.w1);
     uint16_t* w0 = reinterpret_cast<uint16_t*>(ws + L.w0);
     MlpPacked W;
     W.w0t = w0t;
     W.w1t = w1t;
-    W.w2t = w2t;
+    W.fwd = reinterpret_cast<const uint4*>(fwd);
     W.w2 = w2;
     W.w1 = w1;
     W.w0 = w0;
@@ -596,7 +599,8 @@ int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
         // the counting march also packs the bf16 MLP operands and zeroes the
         // MLP gradient (accumulated by k_dw_reduce later in the step)
         StageScope sc(1, s);
-        PackArgs pk{d->mlp, w0t, w1t, w2t, w2, w1, w0, d->mlp_grad};
+        PackArgs pk{d->mlp, w0t, w1t, fwd, w2, w1, w0, d->mlp_grad,
+                    reinterpret_cast<uint32_t*>(ws + L.zero)};
         if (direct) pk.prm = nullptr;
         if ((rc = launch_ray_count(P, t, R, pk, s))) return rc;
     }
