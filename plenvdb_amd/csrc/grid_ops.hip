@@ -107,6 +107,96 @@ __global__ void __launch_bounds__(256) k_tri_bwd(TopoView t, float* __restrict__
     }
 }
 
+// The same sums as k_tri_bwd with fewer and wider atomics: a workgroup takes 64
+// consecutive points (samples of a ray lie half a voxel apart and share most of
+// their corners), links the (point, corner) pairs of each slot into a list
+// through an LDS hash, and adds every distinct slot's C sums once, a lane per
+// channel, so that one request carries a slot's row.  A pair keeps its weight
+// only; the walk multiplies it with the point's gradients, which wait in LDS.
+// k_tri_bwd is bound by its requests: one per (point, corner, channel), as a
+// lane's channels lie in instructions of their own.  200k points along random
+// rays, 12 channels: 98.4 -> 15.2 us; 1.2M points, one channel: 33.7 -> 26.2 us;
+// 100k samples of rays that all cross one region: 528 -> 27.5 us and, one
+// channel, 47.3 -> 12.6 us.  Points in no order, which share no corners, still
+// gain by the wide requests.
+constexpr int kBwdPoints = 64, kBwdPairs = 8 * kBwdPoints, kBwdSlots = 2 * kBwdPairs;
+constexpr uint32_t kNoKey = 0xffffffffu, kNoPair = 0xffffu;
+
+template <int C, int ORDER>
+__global__ void __launch_bounds__(256) k_tri_bwd_agg(TopoView t, float* __restrict__ grad,
+                                                     const float* __restrict__ xs,
+                                                     const float* __restrict__ ys,
+                                                     const float* __restrict__ zs,
+                                                     const float* __restrict__ g, int64_t n) {
+    constexpr int kLanes = C == 12 ? 16 : C == 3 ? 4 : 1;  // lanes per slot in the walk
+    __shared__ uint32_t key[kBwdSlots];   // the slot of an entry
+    __shared__ uint32_t head[kBwdSlots];  // the entry's first pair
+    __shared__ float wgt[kBwdPairs];      // a pair's weight (ORDER 0: its contribution)
+    __shared__ uint16_t next[kBwdPairs], listed[kBwdPairs];
+    __shared__ float gs[C > 1 ? kBwdPoints * C : 1];
+    __shared__ int nlisted;
+    const int tid = threadIdx.x;
+    const int64_t p0 = (int64_t)blockIdx.x * kBwdPoints;
+    const int np = (int)(n - p0 < kBwdPoints ? n - p0 : kBwdPoints);
+#pragma unroll
+    for (int e = 0; e < kBwdSlots / 256; ++e) {
+        key[tid + 256 * e] = kNoKey;
+        head[tid + 256 * e] = kNoPair;
+    }
+    if (tid == 0) nlisted = 0;
+    if constexpr (C > 1)
+        for (int e = tid; e < np * C; e += 256) gs[e] = g[p0 * C + e];
+    int64_t s[2];
+    float w[2];
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {  // pairs tid and tid + 256
+        const int pt = (tid >> 3) + 32 * it, q = tid & 7;
+        s[it] = -1;
+        w[it] = 0.f;
+        if (pt < np) {
+            const int64_t p = p0 + pt;
+            const Cell cell = make_cell(xs[p], ys[p], zs[p]);
+            const int dx = (kCx >> q) & 1, dy = (kCy >> q) & 1, dz = (kCz >> q) & 1;
+            const float a = dx ? cell.u : 1.f - cell.u;
+            const float b = dy ? cell.v : 1.f - cell.v;
+            const float d = dz ? cell.w : 1.f - cell.w;
+            w[it] = ORDER == 0 ? ((g[p] * a) * b) * d : (a * b) * d;
+            s[it] = pvdb::slot_of(t, cell.i0 + dx, cell.j0 + dy, cell.k0 + dz);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        if (s[it] < 0) continue;
+        const int pair = tid + 256 * it;
+        wgt[pair] = w[it];
+        const uint32_t k = (uint32_t)s[it];
+        uint32_t h = (k * 2654435761u) >> 22;  // kBwdSlots == 1 << 10
+        while (true) {  // at most kBwdPairs entries: a free one is met
+            const uint32_t prev = atomicCAS(&key[h], kNoKey, k);
+            if (prev == kNoKey) listed[atomicAdd(&nlisted, 1)] = (uint16_t)h;
+            if (prev == kNoKey || prev == k) break;
+            h = (h + 1) & (kBwdSlots - 1);
+        }
+        next[pair] = (uint16_t)atomicExch(&head[h], (uint32_t)pair);
+    }
+    static_assert(kBwdSlots == 1 << 10, "the hash's shift");
+    __syncthreads();
+    const int m = nlisted, c = tid & (kLanes - 1);
+    if (c >= C) return;
+    for (int e = tid / kLanes; e < m; e += 256 / kLanes) {
+        const int h = listed[e];
+        float sum = 0.f;
+        for (uint32_t p = head[h]; p != kNoPair; p = next[p]) {
+            if constexpr (C > 1)
+                sum += gs[(p >> 3) * C + c] * wgt[p];
+            else
+                sum += ORDER == 0 ? wgt[p] : g[p0 + (p >> 3)] * wgt[p];
+        }
+        if (sum != 0.f) atomicAdd(grad + (int64_t)key[h] * C + c, sum);
+    }
+}
+
 __device__ __forceinline__ bool slot_active(const TopoView& t, int64_t slot) {
     const int64_t leaf = slot >> 9;
     const int off = (int)(slot & 511);
@@ -166,11 +256,18 @@ __global__ void k_set_by_mask(TopoView t, float* __restrict__ vals,
 }
 
 // zero_grad (densityvdb.cu:353-361, colorvdb.cu:355-364): active slots only.
-__global__ void k_zero_active(TopoView t, float* __restrict__ grad, int C) {
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= t.nleaf * 512) return;
-    if (!slot_active(t, s)) return;
-    for (int c = 0; c < C; ++c) grad[s * C + c] = 0.f;
+// One thread per V consecutive values of a slot, so that a wave's stores are
+// contiguous: a thread per slot wrote its row in C stores 4 C bytes apart.  309k slots,
+// 12 channels: 16.5 -> 5.9 us.
+template <int V>
+__global__ void __launch_bounds__(256) k_zero_active(TopoView t, float* __restrict__ grad, int C) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t s = q / (C / V);
+    if (s >= t.nleaf * 512 || !slot_active(t, s)) return;
+    if constexpr (V == 4)
+        reinterpret_cast<float4*>(grad)[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+    else
+        grad[q] = 0.f;
 }
 
 // Total-variation gradient of a VDB payload: the dense kernel's rule
@@ -254,33 +351,68 @@ __global__ void __launch_bounds__(256) k_tv_add_grad(TopoView t, const float* __
         grad[e] = r[0];
 }
 
+__device__ __forceinline__ void adam1(float& p, float g, float& m, float& v, float sz, float eps,
+                                      float b0, float b1) {
+    const float nm = b0 * m + (1.f - b0) * g;
+    const float nv = b1 * v + ((1.f - b1) * g) * g;
+    m = nm;
+    v = nv;
+    p = p - (sz * nm) / (eps + sqrtf(nv));
+}
+
 // VDB Adam over all slots, one thread per (slot, group of `group` channels)
-// (densityvdb.cu:185-349, colorvdb.cu:179-351).
-__global__ void k_vdb_adam(TopoView t, float* __restrict__ param, const float* __restrict__ grad,
-                           float* __restrict__ m, float* __restrict__ v,
-                           const float* __restrict__ per_lr, int C, int group, int mode,
-                           float stepsz, float eps, float b0, float b1) {
-    const int ngroups = C / group;
+// (densityvdb.cu:185-349, colorvdb.cu:179-351).  G: the group, when it is known
+// (0: any); a thread's loads are then all issued before its first store.  1M
+// slots, 12 channels and one, 42% of the voxels updated, nothing cached: 84.9 ->
+// 64.1 us for both grids.
+template <int G>
+__global__ void __launch_bounds__(256) k_vdb_adam(TopoView t, float* __restrict__ param,
+                                                  const float* __restrict__ grad,
+                                                  float* __restrict__ m, float* __restrict__ v,
+                                                  const float* __restrict__ per_lr, int C,
+                                                  int group, int mode, float stepsz, float eps,
+                                                  float b0, float b1) {
+    const int grp_n = G > 0 ? G : group;
+    const int ngroups = C / grp_n;
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= t.nleaf * 512 * ngroups) return;
     const int64_t s = q / ngroups;
-    const int grp = (int)(q - s * ngroups);
-    if (!slot_active(t, s)) return;
-    const int64_t base = s * C + (int64_t)grp * group;
-    if (mode == 1) {
-        bool all0 = true;
-        for (int c = 0; c < group; ++c) all0 &= grad[base + c] == 0.f;
-        if (all0) return;
-    }
-    float sz = stepsz;
-    if (mode == 2) sz = per_lr[s] * stepsz;
-    for (int c = 0; c < group; ++c) {
-        const float g = grad[base + c];
-        const float nm = b0 * m[base + c] + (1.f - b0) * g;
-        const float nv = b1 * v[base + c] + ((1.f - b1) * g) * g;
-        m[base + c] = nm;
-        v[base + c] = nv;
-        param[base + c] = param[base + c] - (sz * nm) / (eps + sqrtf(nv));
+    const int64_t base = q * grp_n;
+    if constexpr (G > 0) {
+        float gg[G], pp[G], mm[G], vv[G];
+#pragma unroll
+        for (int c = 0; c < G; ++c) gg[c] = grad[base + c];
+        if (!slot_active(t, s)) return;
+        if (mode == 1) {
+            bool all0 = true;
+#pragma unroll
+            for (int c = 0; c < G; ++c) all0 &= gg[c] == 0.f;
+            if (all0) return;
+        }
+        const float sz = mode == 2 ? per_lr[s] * stepsz : stepsz;
+#pragma unroll
+        for (int c = 0; c < G; ++c) {
+            mm[c] = m[base + c];
+            vv[c] = v[base + c];
+            pp[c] = param[base + c];
+        }
+#pragma unroll
+        for (int c = 0; c < G; ++c) {
+            adam1(pp[c], gg[c], mm[c], vv[c], sz, eps, b0, b1);
+            m[base + c] = mm[c];
+            v[base + c] = vv[c];
+            param[base + c] = pp[c];
+        }
+    } else {
+        if (!slot_active(t, s)) return;
+        if (mode == 1) {
+            bool all0 = true;
+            for (int c = 0; c < group; ++c) all0 &= grad[base + c] == 0.f;
+            if (all0) return;
+        }
+        const float sz = mode == 2 ? per_lr[s] * stepsz : stepsz;
+        for (int c = 0; c < group; ++c)
+            adam1(param[base + c], grad[base + c], m[base + c], v[base + c], sz, eps, b0, b1);
     }
 }
 
@@ -311,6 +443,13 @@ void launch_fwd(const TopoView& t, const float* vals, int cdyn, const float* xs,
 template <int C, int ORDER>
 void launch_bwd(const TopoView& t, float* grad, int cdyn, const float* xs, const float* ys,
                 const float* zs, const float* g, int64_t n, hipStream_t s) {
+    if constexpr (C > 0) {
+        if (t.nleaf < (int64_t(1) << 23) - 1) {  // every slot below the hash's empty key
+            hipLaunchKernelGGL((k_tri_bwd_agg<C, ORDER>), dim3(pvdb_blocks(n, kBwdPoints)),
+                               dim3(256), 0, s, t, grad, xs, ys, zs, g, n);
+            return;
+        }
+    }
     hipLaunchKernelGGL((k_tri_bwd<C, ORDER>), dim3(pvdb_blocks(n, 256)), dim3(256), 0, s, t, grad,
                        cdyn, xs, ys, zs, g, n);
 }
@@ -450,8 +589,10 @@ int pvdb_zero_active(const pvdb_topology* topo, float* grad, int32_t channels, v
     PVDB_CHECK_ARG(channels >= 1 && grad, "bad arguments");
     const TopoView t = pvdb::view_of(topo);
     if (t.nleaf == 0) return PVDB_OK;
-    hipLaunchKernelGGL(k_zero_active, dim3(pvdb_blocks(t.nleaf * 512, 256)), dim3(256), 0,
-                       (hipStream_t)stream, t, grad, channels);
+    const bool vec4 = channels % 4 == 0 && reinterpret_cast<uintptr_t>(grad) % 16 == 0;
+    const int64_t n = t.nleaf * 512 * (vec4 ? channels / 4 : channels);
+    hipLaunchKernelGGL(vec4 ? k_zero_active<4> : k_zero_active<1>, dim3(pvdb_blocks(n, 256)),
+                       dim3(256), 0, (hipStream_t)stream, t, grad, channels);
     PVDB_LAUNCHED("k_zero_active");
     return PVDB_OK;
 }
@@ -468,7 +609,8 @@ int pvdb_vdb_adam(const pvdb_topology* topo, float* param, const float* grad, fl
     const TopoView t = pvdb::view_of(topo);
     if (t.nleaf == 0) return PVDB_OK;
     const int64_t n = t.nleaf * 512 * (channels / group);
-    hipLaunchKernelGGL(k_vdb_adam, dim3(pvdb_blocks(n, 256)), dim3(256), 0, (hipStream_t)stream,
+    const auto kernel = group == 3 ? k_vdb_adam<3> : group == 1 ? k_vdb_adam<1> : k_vdb_adam<0>;
+    hipLaunchKernelGGL(kernel, dim3(pvdb_blocks(n, 256)), dim3(256), 0, (hipStream_t)stream,
                        t, param, grad, exp_avg, exp_avg_sq, per_lr, channels, group, mode, stepsz,
                        eps, beta0, beta1);
     PVDB_LAUNCHED("k_vdb_adam");
