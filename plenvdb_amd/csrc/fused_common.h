@@ -14,9 +14,9 @@
 //                  their gradient per ray; a second pass forms each sample's
 //                  dL/dlogit and, through the alpha/raw2alpha adjoints, dL/dsigma
 //   k_loss_reduce  the per-ray loss terms summed in a fixed order
-//   k_mlp_bwd      workgroup per CU over 32-record groups: recompute from the
-//                  kept features under the kept masks, MFMA MLP backward, dW
-//                  partials; per-record feature and sigma gradients
+//   k_mlp_bwd      workgroup per CU over rounds of four 32-record groups: MFMA MLP
+//                  backward under the kept masks, H0 and H1 recomputed from the kept
+//                  input rows, dW partials; per-record feature and sigma gradients
 //   k_scatter_agg  workgroups over 32- or 64-record chunks: corner contributions
 //                  summed per slot in an LDS hash, device atomics per distinct slot
 //   k_dw_reduce    the dW partials summed in a fixed order (+ the MLP Adam)
@@ -126,19 +126,13 @@ struct RayBuffers {
 constexpr int kStepCache = 256;
 
 // Packed bf16 MLP weights for MFMA (row-major, zero padded):
-//   w0t [128][64]  W0^T (in 0..38 used)       w1t [128][128] W1^T
-//   w2  [128][32]  W2 (cols 0..2 used)
-//   w1  [128][128] W1                          w0  [16][128]  W0 rows 0..15 (0..11 used)
+//   w2  [128][32]  W2 (cols 0..2 used)         w0  [16][128]  W0 rows 0..15 (0..11 used)
 // fwd: the forward's weights and bias splits as its LDS image (kFwdImage),
-// and fp32 biases b0[128], b1[128], b2[3].
+// and fp32 biases b1[128], b2[3].
 struct MlpPacked {
-    const uint16_t* w0t;
-    const uint16_t* w1t;
     const uint4* fwd;
     const uint16_t* w2;
-    const uint16_t* w1;
     const uint16_t* w0;
-    const float* b0;
     const float* b1;
     const float* b2;
 };
@@ -162,7 +156,7 @@ constexpr int kPartStride = (kMlpParams + 3) & ~3;  // dW partial rows padded to
 // it later in the step): item t of kPackItems.
 struct PackArgs {
     const float* prm;
-    uint16_t *w0t, *w1t, *fwd, *w2, *w1, *w0;
+    uint16_t *fwd, *w2, *w0;
     float* grad;
     uint32_t* zero;  // [64] RayBuffers::zero
 };
@@ -216,15 +210,6 @@ __device__ __forceinline__ uint16_t fwd_image_item(int t, const float* prm) {
 __device__ __forceinline__ void pack_mlp_item(int t, const PackArgs& A) {
     if (t < kMlpParams) A.grad[t] = 0.f;
     if (t < 64) A.zero[t] = t < 48 ? 0u : 0xffffffffu;
-    if (t < 128 * 128) {  // w1t / w1: 128 x 128
-        const int a = t >> 7, b = t & 127;
-        A.w1t[a * 128 + b] = f2bf_bits(A.prm[kW1 + b * 128 + a]);  // W1^T[out a][in b]
-        A.w1[a * 128 + b] = f2bf_bits(A.prm[kW1 + a * 128 + b]);   // W1[in a][out b]
-    }
-    if (t < 128 * 64) {  // w0t [128 out][64 in]
-        const int o = t >> 6, i = t & 63;
-        A.w0t[o * 64 + i] = i < 39 ? f2bf_bits(A.prm[kW0 + i * 128 + o]) : (uint16_t)0;
-    }
     if (t < kFwdImage) A.fwd[t] = fwd_image_item(t, A.prm);
     if (t < 16 * 128) {  // w0 [16 in][128 out]
         const int o = t >> 7, i = t & 127;

@@ -1,6 +1,6 @@
 // Fused step, sample side: the view-dependent RGB MLP (39-128-128-3, ReLU,
 // sigmoid; plenvdb/lib/dvgo.py:91-109,354-362) on MFMA, forward and backward,
-// over groups of 32 consecutive records (two 16-sample MFMA tiles).
+// over groups of 32 consecutive records.
 //
 // Activations are computed transposed (features x samples, the samples being an
 // MFMA's N dimension):
@@ -17,16 +17,14 @@
 //
 // k_mlp_fwd gathers the colour features and writes each record's rgb, ReLU masks
 // and bf16 input row (so the backward reads 80 bytes per record instead of
-// redoing 8 gathers).  k_mlp_bwd recomputes H0 and H1 (for the dW operands) in
-// wavefronts that own a slice of the hidden features each and exchange
-// activations through LDS, takes each sample's dL/dlogit and dL/dsigma from
+// redoing 8 gathers).  k_mlp_bwd takes each sample's dL/dlogit and dL/dsigma from
 // the composite pass, runs g_H1^T = W2 g_L^T, g_H0^T = W1 g_H1^T (masked by
-// the ReLUs, kept as bit masks), g_X^T = W0[0:12] g_H0^T, accumulates dW over
-// each group's 32 samples (K = 32) in registers (one partial per workgroup),
-// and writes each record's feature and sigma gradients; the scatter
+// the forward's ReLU masks), g_X^T = W0[0:12] g_H0^T, recomputes H0 and H1 for the
+// dW operands, accumulates dW in registers (one partial per workgroup), and
+// writes each record's feature and sigma gradients; the scatter
 // (fused_scatter.hip) then adds them to the grids with the "leaf must exist"
 // rule (densityvdb.cu:16-27, colorvdb.cu:28-37).  Both kernels load a group's
-// records into registers while the previous group computes.
+// records into registers while an earlier group computes.
 
 #include <cstddef>
 #include <type_traits>
@@ -43,115 +41,9 @@ using namespace pvdb;
 
 namespace {
 
-constexpr int GS = 32;       // records per group
-constexpr int NT = GS / 16;  // 16-sample MFMA tiles per group
-constexpr int XM = 72;       // sample-major stride of X (64 + 8)
-constexpr int SM = 136;      // sample-major stride of 128-wide activations (128 + 8)
-constexpr int GM = 24;       // sample-major stride of dL/dlogit (16 + 8)
-constexpr int FM = 40;       // feature-major stride (32 samples + 8; rows 16-byte aligned)
-constexpr int XF_ROWS = 48;  // feature-major X rows: inputs 0..39 are used
-
-__device__ __forceinline__ bf16x8 ld_frag(const uint16_t* p) {  // 16-byte aligned
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    return __builtin_bit_cast(bf16x8, v);
-}
-
-__device__ __forceinline__ s16x4 ld_frag4(const uint16_t* p) {
-    const uint2 v = *reinterpret_cast<const uint2*>(p);
-    return __builtin_bit_cast(s16x4, v);
-}
+constexpr int GS = 32;  // records per group
 
 __device__ __forceinline__ bf16x8 as_bf8(const uint4& v) { return __builtin_bit_cast(bf16x8, v); }
-
-__device__ __forceinline__ void split_bf(float x, uint16_t& h, uint16_t& l) {
-    uint32_t hh, ll;
-    split2(x, 0.f, hh, ll);
-    h = (uint16_t)hh;
-    l = (uint16_t)ll;
-}
-
-// DPP permutation within rows (quad permutes, the half-row mirror), all lanes
-// active: every lane reads a valid source, so the move needs no old value
-// (update_dpp's would be materialised with a v_mov).
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
-}
-
-// A lane holds four consecutive features (rows) of one sample; the four lanes of
-// a quad hold four consecutive samples.  Returns row (lane & 3) of the quad's
-// four samples, as four bf16 in two dwords: two quad swaps instead of four
-// 2-byte stores per lane.
-__device__ __forceinline__ uint2 quad_transpose(uint2 h, int q) {
-    const uint32_t v0 = h.x & 0xffffu, v1 = h.x >> 16, v2 = h.y & 0xffffu, v3 = h.y >> 16;
-    // exchange 1 (lanes q, q^1): even lanes gather rows 0/2, odd lanes rows 1/3, of the pair
-    const uint32_t send = (q & 1) ? (v0 | (v2 << 16)) : (v1 | (v3 << 16));
-    const uint32_t recv = dpp<0xB1>(send);  // quad_perm [1,0,3,2]
-    const uint32_t A = (q & 1) ? ((recv & 0xffffu) | (v1 << 16)) : (v0 | (recv << 16));
-    const uint32_t B = (q & 1) ? ((recv >> 16) | (v3 << 16)) : (v2 | (recv & 0xffff0000u));
-    // exchange 2 (lanes q, q^2): rows (q & 1) and (q & 1) + 2 of the two pairs
-    const uint32_t send2 = (q & 2) ? A : B;
-    const uint32_t recv2 = dpp<0x4E>(send2);  // quad_perm [2,3,0,1]
-    return (q & 2) ? make_uint2(recv2, B) : make_uint2(A, recv2);
-}
-
-// Four consecutive features fr..fr+3 of sample `col`: sample-major (hi, lo)
-// pairs into sh/sl, and (FMC) the hi parts feature-major into fm.
-template <bool FMC>
-__device__ __forceinline__ void st_act(uint16_t* sh, uint16_t* sl, uint16_t* fm, int col, int fr,
-                                       int lane, const float* v) {
-    uint2 hi, lo;
-    split2(v[0], v[1], hi.x, lo.x);
-    split2(v[2], v[3], hi.y, lo.y);
-    *reinterpret_cast<uint2*>(&sh[col * SM + fr]) = hi;
-    *reinterpret_cast<uint2*>(&sl[col * SM + fr]) = lo;
-    if constexpr (FMC) {
-        const int q = lane & 3;
-        *reinterpret_cast<uint2*>(&fm[(fr + q) * FM + (col & ~3)]) = quad_transpose(hi, q);
-    }
-}
-
-// The hi parts of four consecutive features fr..fr+3 of sample `col`:
-// sample-major into sh and feature-major into fm.
-__device__ __forceinline__ void st_hi_fm(uint16_t* sh, uint16_t* fm, int col, int fr, int lane,
-                                         const float* v) {
-    uint2 hi, lo;
-    split2(v[0], v[1], hi.x, lo.x);
-    split2(v[2], v[3], hi.y, lo.y);
-    *reinterpret_cast<uint2*>(&sh[col * SM + fr]) = hi;
-    const int q = lane & 3;
-    *reinterpret_cast<uint2*>(&fm[(fr + q) * FM + (col & ~3)]) = quad_transpose(hi, q);
-}
-
-// The hi parts of four consecutive features fr..fr+3 of sample `col`,
-// feature-major into fm (the feature-major half of st_act<true>).
-__device__ __forceinline__ void st_fm(uint16_t* fm, int col, int fr, int lane, const float* v) {
-    uint2 hi, lo;
-    split2(v[0], v[1], hi.x, lo.x);
-    split2(v[2], v[3], hi.y, lo.y);
-    const int q = lane & 3;
-    *reinterpret_cast<uint2*>(&fm[(fr + q) * FM + (col & ~3)]) = quad_transpose(hi, q);
-}
-
-// a (bf16 weight) times a split activation
-__device__ __forceinline__ f32x4 mfma_w(const bf16x8& a, const bf16x8& bh, const bf16x8& bl,
-                                        f32x4 c) {
-    c = mfma16x16x32(a, bh, c);
-    return mfma16x16x32(a, bl, c);
-}
-
-// dW products (activation x gradient) use the hi parts only, and the backward
-// recomputes the activations they take from hi parts: the sums over a step's
-// samples average that rounding (a device check keeps every MLP gradient
-// within 6e-4 of FP64), so the gradients' lo parts stay sample-major.
-
-// x where bit k of m is set, else +0: the bit sign-extended by one v_bfe_i32
-// and ANDed with x's bits (two instructions; a compare and a select take
-// three, with the bit extraction)
-__device__ __forceinline__ float keep_if(uint32_t m, int k, float x) {
-    const uint32_t all = (uint32_t)__builtin_amdgcn_sbfe((int)m, k, 1);
-    return __uint_as_float(__float_as_uint(x) & all);
-}
 
 // ---- forward -----------------------------------------------------------------
 // A wavefront takes a group of 32 records through the whole network by itself:
@@ -589,398 +481,522 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
     }
 }
 
-// Backward weights as MFMA A fragments in LDS, [tile][k-step][lane] (each
-// wave's W1 rows for the g_H0 product, 32 x 128, sit in its registers):
-//   W2  [8 row tiles of 16 hidden][64] x 8 bytes   (K = 16 logits, 3 used)
-//   W0  [4 k-steps of 32 hidden][64] x 16 bytes    (rows: the 12 features)
-constexpr int kBw2Frags = 8 * 64, kBw0Frags = 4 * 64;
-
 // ---- backward ----------------------------------------------------------------
-// One workgroup of 8 wavefronts per CU (two per SIMD); wave w owns hidden
-// features [16w, 16w + 16) of both hidden layers, except in the g_H0 product
-// (phase 8), where it owns features [32(w/2), +32) of samples [16(w%2), +16).
-// Per group of 32 records three stages of work, each pairing products that
-// do not depend on one another:
-//   A  H0^T = W0^T X^T + b0 under the forward's ReLU mask m0    -> A1h, H0f
-//      g_H1^T = W2 g_L^T masked by m1                           -> G1h, G1l, G1f
-//   B  H1^T = W1^T H0^T + b1 under the forward's mask m1         -> F2
-//      g_H0^T = W1 g_H1^T masked by m0                          -> A2h, A2l, F3
-//      dW1 += H0^T g_H1; the next group's records are parked
-//   C  dW2 += H1^T g_L; dW0 += X^T g_H0; waves 0-1: g_X^T = W0[0:12] g_H0^T
-//      over the whole hidden layer, written from registers as the records'
-//      feature gradients
-// run as two barrier-separated steps: group k's A with group k-1's C, then
-// group k's B.  The input rows X come whole from the forward pass (features,
-// encoding, bias input), so group k+1's A needs nothing computed after group
-// k's B.
-// H0 and H1 are recomputed for the dW operands only (from hi parts, one MFMA
-// per product): the masks come from the forward pass (per-record words), so the
-// backward applies exactly the ReLU pattern the forward applied.
-// X (features, encoding, bias), the per-sample adjoints and the flags are
-// double-buffered, so the next group's inputs are staged while this one runs.
-constexpr int kBwdWaves = 8;
+// A workgroup takes rounds of four 32-record groups with four pairs of
+// wavefronts, two wavefronts to a SIMD.  Of a pair, the gradient wavefront runs
+// its group's chain
+//   g_H1^T = W2 g_L^T (masked), g_H0^T = W1 g_H1^T (masked), g_X^T = W0[0:12] g_H0^T
+// with the gradients as (hi, lo) pairs, in registers from end to end as in the
+// forward: a D fragment of 32x32x16 is the next product's B fragment under the
+// permuted K order.  The other, the weight wavefront, recomputes
+//   H0^T = relu(W0^T X^T + b0), H1 = relu(H0 W1 + b1)
+// from hi parts (for the dW operands only: the gradients are masked by the
+// forward's own ReLU masks; H1 comes out a feature to a lane, since its operands
+// are the same fragments in the other order), adds its group's H1^T g_L to dW2, and
+// then a slice of the whole round's dW1 += H0^T g_H1 (64 x 64) and dW0 += X^T g_H0
+// (all inputs x 32).  Those contract over samples, so their operands cross
+// wavefronts: H0, g_H1, g_H0 (hi) and X lie in LDS a row to a sample, and are read
+// through the transposing LDS load, which hands a lane four samples of its
+// feature.  W1 sits in LDS once: the gradient wavefronts read W1 rows out of the
+// W1^T fragments with the same load.
+//
+// A round has two intervals, a barrier after each, so that one copy of the
+// buffers will do:
+//   1  weight: dW1 and dW0 of the round before      gradient: g_H1, a quarter of g_H0
+//   2  weight: H0, H1, dW2                          gradient: stores, the rest
+// Within a wavefront a tile is masked, split or relu'd pair by pair between the
+// next tile's MFMAs.
+//
+// The rows' 8-byte pieces (four features) are permuted by the sample's index so
+// that neither the stores (32 rows, one piece each) nor the transposing loads
+// (four rows x 32 features to a wavefront half) meet in a bank.
+//
+// What bounds it: a round is 180 MFMAs of 32 cycles per SIMD and about as many
+// cycles of vector work (1200 instructions of 4), which the two wavefronts overlap
+// in part, and 40% of the time in the CU's LDS.
+//
+// Measured against eight wavefronts that shared one group (16 hidden features
+// each, every product's operands through LDS on 16x16x32 MFMAs): 7.80M records
+// 2632 -> 1175 us, 190k 98.2 -> 49.2 us, 24k 25.0 -> 14.3 us.  On the way: tiles
+// split after their MFMAs instead of between the next one's 1228 us; db1 summed
+// over lanes at each round (32 registers fewer, three instructions a pair more) and
+// the stores' and loads' addresses formed each time 1350 us; spilling registers
+// 2386 us.
+constexpr int kBwdPairs = 4;                   // wavefront pairs, a group each
+constexpr int kBwdWaves = 2 * kBwdPairs;
+constexpr int kRoundRec = kBwdPairs * GS;      // records of a round
+constexpr int kFragPitch = 576, kHalfPitch = 288;  // W1^T fragments in LDS (16-bit values): lane
+                                                   // halves 64 bytes, fragments 128 bytes of the
+                                                   // 256-byte bank row apart
 struct alignas(16) SmemBwd {
-    uint4 Bw0[kBw0Frags];
-    uint2 Bw2[kBw2Frags];
-    uint32_t relu[2][GS * 8];  // the forward's ReLU mask words of each record
-    uint16_t Xh[2][GS * XM];
-    uint16_t Xf[2][XF_ROWS * FM];
-    uint16_t A1h[GS * SM];               // H0 (hi), sample-major
-    uint16_t G1h[GS * SM], G1l[GS * SM]; // g_H1, sample-major
-    uint16_t A2h[GS * SM], A2l[GS * SM]; // g_H0, sample-major
-    uint16_t GLh[2][GS * GM], GLl[2][GS * GM];
-    uint16_t H0f[128 * FM];              // H0, feature-major
-    uint16_t F2[128 * FM];               // H1, feature-major
-    uint16_t G1f[128 * FM];              // g_H1, feature-major
-    uint16_t F3[128 * FM];               // g_H0, feature-major
-    uint16_t GLf[2][16 * FM];
-    float gsig[2][GS];
-    uint32_t bits[2][GS];
+    uint16_t g1[kRoundRec * 128];   // g_H1, g_H0 and H0 (hi) by sample
+    uint16_t g0[kRoundRec * 128];
+    uint16_t h0[kRoundRec * 128];
+    uint16_t x[kRoundRec * 40 + 24];  // X by sample; loads of columns 40..63 run into the next row
+    uint4 w0[6 * 128];              // the forward image's W0^T chunks and b0's split
+    uint16_t w1[32 * kFragPitch];   // the forward image's W1^T fragments [row tile][k-step]
+    uint4 w2[128];                  // W2's rows as g_H1's A fragments, b1 in the last word
+    uint4 w0g[8 * 2 * 12];          // W0[0:12] as g_X's A fragments [k-step][h][feature]
+    uint16_t gl[kBwdPairs][3 * GS]; // dL/dlogit (hi) by logit
 };
+static_assert(sizeof(SmemBwd) <= 160 * 1024, "a CU's LDS");
+
+// Four samples of this lane's feature, from the pieces that the lane's group of
+// 16 points at: lane i names row i / 4's piece i % 4 and receives column i.
+__device__ __forceinline__ uint2 ld_tr(const void* p) {
+    const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) s16x4*)(p));
+    return __builtin_bit_cast(uint2, v);
+}
+__device__ __forceinline__ uint4 ld_tr2(const void* p, const void* q) {
+    const uint2 a = ld_tr(p), b = ld_tr(q);
+    return make_uint4(a.x, a.y, b.x, b.y);
+}
+
+// sum over each half of the wavefront, in its last lane
+__device__ __forceinline__ float half_sum(float x) {
+    x += dpp_mov<kDppRowShr1>(x, 0.f);
+    x += dpp_mov<kDppRowShr2>(x, 0.f);
+    x += dpp_mov<kDppRowShr4>(x, 0.f);
+    x += dpp_mov<kDppRowShr8>(x, 0.f);
+    x += dpp_mov<kDppRowBcast15, 0xa>(x, 0.f);
+    return x;
+}
+
+// relu of two floats as a bf16 pair: rounding keeps order and zero, so the max,
+// of packed integers as in relu, may follow the conversion
+__device__ __forceinline__ uint32_t relu_bf2(float a, float b) {
+    uint32_t r;
+    asm("v_pk_max_i16 %0, %1, 0" : "=v"(r) : "v"(pk_bf(a, b)));
+    return r;
+}
+
+// x where bit k of m is set, else +0: the bit sign-extended by one v_bfe_i32
+// and ANDed with x's bits (two instructions; a compare and a select take
+// three, with the bit extraction)
+__device__ __forceinline__ float keep_if(uint32_t m, int k, float x) {
+    const uint32_t all = (uint32_t)__builtin_amdgcn_sbfe((int)m, k, 1);
+    return __uint_as_float(__float_as_uint(x) & all);
+}
+
+__device__ __forceinline__ void stage_bwd_weights(SmemBwd& sm, const MlpPacked& W) {
+    constexpr int NTH = 64 * kBwdWaves;
+    const int tid = threadIdx.x;
+    for (int e = tid; e < 6 * 128; e += NTH) sm.w0[e] = W.fwd[e];
+    const uint4* img = W.fwd + kImgW1 / 8;  // [row tile][9 steps, the first the bias][lane]
+#pragma unroll
+    for (int k = 0; k < 32 * 64 / NTH; ++k) {
+        const int e = tid + NTH * k, f = e >> 6, l = e & 63;
+        *reinterpret_cast<uint4*>(sm.w1 + f * kFragPitch + (l >> 5) * kHalfPitch + 8 * (l & 31)) =
+            img[((f >> 3) * 9 + 1 + (f & 7)) * 64 + l];
+    }
+    if (tid < 128) {  // K: the logits' hi parts, their lo parts
+        const uint2 w = *reinterpret_cast<const uint2*>(W.w2 + 32 * tid);  // w0 w1 | w2 0
+        sm.w2[tid] = make_uint4(w.x, (w.y & 0xffffu) | (w.x << 16), (w.x >> 16) | (w.y << 16),
+                                __float_as_uint(W.b1[tid]));
+    } else if (tid < 128 + 8 * 2 * 12) {
+        const int e = tid - 128, m = e % 12, h = (e / 12) & 1, ks = e / 24;
+        const uint2* src = reinterpret_cast<const uint2*>(W.w0 + 128 * m + 16 * ks + 4 * h);
+        sm.w0g[e] = make_uint4(src[0].x, src[0].y, src[2].x, src[2].y);
+    }
+}
 
 __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPacked W,
                                                             RayBuffers R, Records rec,
                                                             float* __restrict__ dw_partial) {
-    constexpr int NTH = 64 * kBwdWaves;
     __shared__ SmemBwd sm;
-    const int tid = threadIdx.x;
-    const int wv = tid >> 6, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
-    const int f0 = 16 * wv;
-    const int fr = f0 + 4 * g;  // the 4 features of this lane's D fragment rows
-    const int pr = lane < GS / kBwdWaves ? wv * (GS / kBwdWaves) + lane : -1;  // staging lanes
-
-    // forward weight slices in registers (this wave's rows of W0^T and W1^T)
-    bf16x8 A0[2], A1[4];
-    float b0v[4], b1v[4];
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) A0[kt] = ld_frag(W.w0t + (f0 + r16) * 64 + 32 * kt + 8 * g);
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt) A1[kt] = ld_frag(W.w1t + (f0 + r16) * 128 + 32 * kt + 8 * g);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        b0v[i] = W.b0[fr + i];
-        b1v[i] = W.b1[fr + i];
-    }
-    // the g_H0 product's tile of this wave: hidden features 32 fb .. +31 (two
-    // row tiles) of samples 16 sh .. +15; W1 rows [32 in][128 out] as MFMA A
-    // fragments, in registers
-    const int fb = wv >> 1, sh = wv & 1;
-    bf16x8 Bw1r[2][4];
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-            Bw1r[mt][kt] = ld_frag(W.w1 + (32 * fb + 16 * mt + r16) * 128 + 32 * kt + 8 * g);
-    // the other backward weights -> LDS
-    for (int f = tid; f < kBw2Frags + kBw0Frags; f += NTH) {
-        const int ln = f & 63, gg = ln >> 4, rr = ln & 15;
-        if (f < kBw2Frags) {  // W2 [128 in][32 out (3 used)], K = 16
-            const int t = f >> 6;
-            sm.Bw2[f] = *reinterpret_cast<const uint2*>(W.w2 + (16 * t + rr) * 32 + 4 * gg);
-        } else {  // W0 rows 0..15 [16][128]
-            const int q = f - kBw2Frags, kt = q >> 6;
-            sm.Bw0[q] = *reinterpret_cast<const uint4*>(W.w0 + rr * 128 + 32 * kt + 8 * gg);
-        }
-    }
-    f32x4 dW0[3], dW1[8], dW2;
-    float db1[4] = {0.f, 0.f, 0.f, 0.f}, db2[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-    for (int a = 0; a < 3; ++a) dW0[a] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int a = 0; a < 8; ++a) dW1[a] = f32x4{0.f, 0.f, 0.f, 0.f};
-    dW2 = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // constant parts of the double buffers: X columns 40..63, feature-major X
-    // rows 40..47, logits 3..15
-    for (int e = tid; e < 2 * GS * 24; e += NTH) {
-        const int b = e / (GS * 24), row = (e / 24) % GS, col = 40 + e % 24;
-        sm.Xh[b][row * XM + col] = 0;
-    }
-    for (int e = tid; e < 2 * (XF_ROWS - 40) * FM; e += NTH) {
-        const int b = e / ((XF_ROWS - 40) * FM);
-        sm.Xf[b][40 * FM + e % ((XF_ROWS - 40) * FM)] = 0;
-    }
-    for (int e = tid; e < 2 * GS * GM; e += NTH) {
-        if (e % GM >= 3) {
-            (&sm.GLh[0][0])[e] = 0;
-            (&sm.GLl[0][0])[e] = 0;
-        }
-    }
-    for (int e = tid; e < 2 * 16 * FM; e += NTH)
-        if ((e % (16 * FM)) >= 3 * FM) (&sm.GLf[0][0])[e] = 0;
-
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int w = wv & (kBwdPairs - 1);  // the group of the round
+    const int lane = lane_id(), n = lane & 31, h = lane >> 5;
     const int64_t total = min((int64_t)R.total[0], P.capacity);
-    const int64_t ngroups = (total + GS - 1) / GS;
-    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    const uint4 zu4 = make_uint4(0u, 0u, 0u, 0u);
-
-    // register prefetch of a group's records: the staging lanes (4 per wave, a
-    // record each) take its flags, adjoints and ReLU masks; the row lanes (20
-    // per wave) one 16-byte fifth of its input row each.  Every address
-    // follows from the record index alone, so the loads of the next group are
-    // issued at the start of the current one and land during its products.
-    float4 p_adj = z4;
-    uint32_t p_bits = 0u;
-    uint4 p_r0 = zu4, p_r1 = zu4, p_x = zu4;
-    const int xe = (lane >= 32 && lane < 52) ? wv * 20 + (lane - 32) : -1;
-    const int xr = xe / 5, xj = xe % 5;  // row lane: record, 8-column part
-    auto stage = [&](int64_t grp) {
-        const int64_t q = grp * GS + pr;
-        p_adj = z4;
-        p_bits = 0u;
-        p_r0 = p_r1 = zu4;
-        if (pr >= 0 && grp < ngroups && q < total) {
-            p_bits = __float_as_uint(rec.ab[q].y);
-            p_adj = rec.adj[q];
-            p_r0 = reinterpret_cast<const uint4*>(rec.relu)[2 * q];  // ReLU masks
-            p_r1 = reinterpret_cast<const uint4*>(rec.relu)[2 * q + 1];
-        }
-        const int64_t qx = grp * GS + xr;
-        p_x = zu4;
-        if (xe >= 0 && grp < ngroups && qx < total) p_x = rec.xrow[5 * qx + xj];
+    const int64_t nrounds = (total + kRoundRec - 1) / kRoundRec;
+    const int64_t r0 = blockIdx.x, stride = gridDim.x;
+    float* const out = dw_partial + (int64_t)blockIdx.x * kPartStride;
+    float* const red = reinterpret_cast<float*>(sm.g1);  // the last reductions' room
+    constexpr int kRedDb1 = 4 * 384, kRedDb2 = kRedDb1 + 4 * 128;  // after dW2's [4][384]
+    stage_bwd_weights(sm, W);
+    // where this lane's sample stores its pieces, and what it points the
+    // transposing loads at: row rr (+ 4h + 8jj + 16t) and piece pc of 16 c16 features
+    const int rr = (lane & 15) >> 2, pc = lane & 3, c16 = (lane >> 4) & 1;
+    // the bytes of this lane's first piece in its sample's row: piece 8T + 2q + h lies at
+    // the same offset ^ (64 T + 16 q).  Anew in each round: as loop invariants the
+    // sixteen addresses would take as many registers
+    auto row_at = [&]() {
+        uint32_t at = 256 * (GS * w + n) + 8 * ((((n & 3) << 3) | (n >> 2)) ^ h);
+        asm volatile("" : "+v"(at));
+        return at;
     };
-    // staged records -> buffer b: flags, adjoints (dL/dlogit as (hi, lo) pairs,
-    // dL/dsigma), ReLU masks, and the input rows (X columns 0..39, sample-major
-    // and feature-major)
-    auto park = [&](int b) {
-        if (pr >= 0) {
-            sm.bits[b][pr] = p_bits;  // zero for records past the end
-            sm.gsig[b][pr] = p_adj.w;
-            reinterpret_cast<uint4*>(&sm.relu[b][8 * pr])[0] = p_r0;
-            reinterpret_cast<uint4*>(&sm.relu[b][8 * pr])[1] = p_r1;
-            const float gl[3] = {p_adj.x, p_adj.y, p_adj.z};
-            db2[0] += gl[0];
-            db2[1] += gl[1];
-            db2[2] += gl[2];
+    auto piece = [](uint16_t* rows, uint32_t at, int T, int q) {
+        return reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(rows) + (at ^ (64u * T + 16u * q)));
+    };
+
+    if (wv >= kBwdPairs) {
+        // ---- the gradient chain ----
+        float4 adj, nadj;
+        uint32_t mk[4], nmk[4], bits, nbits;  // ReLU mask words: layer 0's h, h + 2, layer 1's
+        auto load = [&](int64_t rnd) {  // the next round's
+            const int64_t q = rnd * kRoundRec + GS * w + n;
+            nadj = make_float4(0.f, 0.f, 0.f, 0.f);
+            nmk[0] = nmk[1] = nmk[2] = nmk[3] = nbits = 0u;
+            if (q < total) {
+                nadj = rec.adj[q];
+                nbits = __float_as_uint(rec.ab[q].y);
+                const uint32_t* m = rec.relu + 8 * q + h;
+                nmk[0] = m[0];
+                nmk[1] = m[2];
+                nmk[2] = m[4];
+                nmk[3] = m[6];
+            }
+        };
+        float db1[64], db2[3] = {0.f, 0.f, 0.f};  // this lane's sample of each round
+#pragma unroll
+        for (int i = 0; i < 64; ++i) db1[i] = 0.f;
+        // W1 rows (lane: in-feature n of a tile) out of the W1^T fragments
+        const uint16_t* const wa = sm.w1 + c16 * kFragPitch + (pc & 1) * kHalfPitch +
+                                   8 * (4 * h + rr) + 4 * (pc >> 1);
+        const uint4* const w0p = sm.w0g + 12 * h + (n < 12 ? n : 0);
+        const f32x16 zero = {};
+        uint32_t gh[8][4], glo[8][4];  // g_H1's B fragments [k-step][dword], hi and lo
+        f32x16 gx;
+        f32x16 d;                      // a finished tile, split while the next one's MFMAs run
+        float va, vb;
+        // pair j (rows 2j, 2j + 1 of the lane) of tile T in two steps: masked, then split
+        auto mask_of = [&](int T, int j, uint32_t ma, uint32_t mb) {
+            const uint32_t m = (j >> 1) & 1 ? mb : ma;
+            const int p = 2 * (2 * T + (j >> 2)) + (j & 1);
+            va = keep_if(m, p, d[2 * j]);
+            vb = keep_if(m, 16 + p, d[2 * j + 1]);
+        };
+        auto w1 = [&](int T, int ks) {
+            const uint16_t* a = wa + ((ks >> 1) * 8 + 2 * T) * kFragPitch + 128 * (ks & 1);
+            return ld_tr2(a, a + 64);
+        };
+        // pair j of g_H1's tile T: gh, glo and db1
+        auto pair1 = [&](int T, int j) {
+            mask_of(T, j, mk[2], mk[3]);
+            db1[16 * T + 2 * j] += va;
+            db1[16 * T + 2 * j + 1] += vb;
+            uint32_t &hi = gh[2 * T + (j >> 2)][j & 3], &lo = glo[2 * T + (j >> 2)][j & 3];
+            split2(va, vb, hi, lo);
+            // here, not at the round's end with va and vb alive till then
+            asm volatile("" : "+v"(db1[16 * T + 2 * j]), "+v"(db1[16 * T + 2 * j + 1]), "+v"(hi), "+v"(lo));
+        };
+        uint32_t hi[8], lo[8];  // g_H0's pairs of a tile
+        // layer 0's features of tile T into the records' gradients
+        auto add_gx = [&](int T) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const uint4 f = w0p[24 * (2 * T + t)];
+                gx = mfma32x32x16(f, make_uint4(lo[4 * t], lo[4 * t + 1], lo[4 * t + 2], lo[4 * t + 3]), gx);
+                gx = mfma32x32x16(f, make_uint4(hi[4 * t], hi[4 * t + 1], hi[4 * t + 2], hi[4 * t + 3]), gx);
+            }
+        };
+        auto pair0_split = [&](int j) {
+            split2(va, vb, hi[j], lo[j]);
+            asm volatile("" : "+v"(hi[j]), "+v"(lo[j]));
+        };
+        load(r0);
+        __syncthreads();  // the weights
+        for (int64_t rnd = r0; rnd < nrounds; rnd += stride) {
+            // ---- interval 1 ----
+            adj = nadj;
+            bits = nbits;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mk[i] = nmk[i];
+            {
+                uint32_t h01, l01, h2, l2;
+                split2(adj.x, adj.y, h01, l01);
+                split2(adj.z, 0.f, h2, l2);
+                db2[0] += adj.x;
+                db2[1] += adj.y;
+                db2[2] += adj.z;
+                if (h == 0) {
+                    uint16_t* g = &sm.gl[w][n];
+                    g[0] = (uint16_t)(h01 & 0xffffu);
+                    g[GS] = (uint16_t)(h01 >> 16);
+                    g[2 * GS] = (uint16_t)h2;
+                }
+                const uint4 b = h ? make_uint4(0u, 0u, 0u, 0u)
+                                  : make_uint4(h01, h2 | (l01 << 16), (l01 >> 16) | (l2 << 16), 0u);
+                auto w2 = [&](int T) {
+                    const uint4 f = sm.w2[32 * T + n];
+                    return make_uint4(h ? 0u : f.x, h ? 0u : f.y, h ? 0u : f.z, 0u);
+                };
+                // g_H1 a tile at a time, each followed by its k-steps of g_H0's first tile
+                // under the next one's split
+                f32x16 e = mfma32x32x16(w2(0), b, zero), c;
+#pragma unroll
+                for (int T = 0; T < 5; ++T) {
+                    uint4 f0, f1;
+                    d = e;
+                    if (T < 3) e = mfma32x32x16(w2(T + 1), b, zero);
+                    if (T > 0) {
+                        f0 = w1(0, 2 * T - 2);
+                        f1 = w1(0, 2 * T - 1);
+                    }
+                    if (T < 4) {
+                        pair1(T, 0);
+                        pair1(T, 1);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if (T > 0) {
+                            const int ks = 2 * T - 2 + (k >> 1);
+                            c = mfma32x32x16(k < 2 ? f0 : f1, frag(k & 1 ? gh[ks] : glo[ks]),
+                                             T == 1 && k == 0 ? zero : c);
+                        }
+                        if (T < 4) {
+                            pair1(T, 2 + k);
+                            if (k == 3) pair1(T, 6);
+                            if (k == 3) pair1(T, 7);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                d = c;
+            }
+            __syncthreads();
+            // ---- interval 2 ----
+            load(rnd + stride);
+            const uint32_t at = row_at();
+            gx = zero;
+            uint4 f[3] = {w1(1, 0), w1(1, 1)};  // read two steps ahead
+#pragma unroll
+            for (int T = 1; T < 4; ++T) {
+                f32x16 c = zero;
+#pragma unroll
+                for (int ks = 0; ks < 8; ++ks) {
+                    const int k = 8 * (T - 1) + ks;
+                    if (k < 22) f[(k + 2) % 3] = w1(1 + (k + 2) / 8, (k + 2) & 7);
+                    c = mfma32x32x16(f[k % 3], frag(glo[ks]), c);
+                    mask_of(T - 1, ks, mk[0], mk[1]);
+                    if (T == 1 && (ks & 1))  // g_H1's rows, between the first MFMAs
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const uint32_t* g = gh[ks - 1 + (q >> 1)] + 2 * (q & 1);
+                            *piece(sm.g1, at, ks >> 1, q) = make_uint2(g[0], g[1]);
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                    c = mfma32x32x16(f[k % 3], frag(gh[ks]), c);
+                    pair0_split(ks);
+                    if (ks & 1) *piece(sm.g0, at, T - 1, ks >> 1) = make_uint2(hi[ks - 1], hi[ks]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                add_gx(T - 1);
+                d = c;
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                mask_of(3, j, mk[0], mk[1]);
+                pair0_split(j);
+                if (j & 1) *piece(sm.g0, at, 3, j >> 1) = make_uint2(hi[j - 1], hi[j]);
+            }
+            add_gx(3);
+            // the record's gradient row: lane half h holds features 4h .. 4h + 3
+            // and, half 0, 8 .. 11; half 1 adds dL/dsigma
+            const int64_t q = rnd * kRoundRec + GS * w + n;
+            if (q < total) {
+                const bool on = (bits & kAliveW) != 0u;
+                float4* row = rec.grad + 4 * q + h;
+                row[0] = on ? make_float4(gx[0], gx[1], gx[2], gx[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+                row[2] = h ? make_float4(adj.w, 0.f, 0.f, 0.f)
+                           : on ? make_float4(gx[4], gx[5], gx[6], gx[7]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            __syncthreads();
+        }
+        __syncthreads();  // the weight wavefronts have read the last round's buffers
+        // db1 and db2: each wavefront's samples, then the four wavefronts'
+#pragma unroll
+        for (int i = 0; i < 64; ++i) {
+            const float v = half_sum(db1[i]);
+            if (n == 31) red[kRedDb1 + 128 * w + 32 * (i >> 4) + 8 * ((i >> 2) & 3) + 4 * h + (i & 3)] = v;
+        }
+#pragma unroll
+        for (int o = 0; o < 3; ++o) {
+            const float v = half_sum(db2[o]);
+            if (lane == 31) red[kRedDb2 + 4 * w + o] = v;
+        }
+    } else {
+        // ---- the weights ----
+        f32x16 dW1[2][2], dW0[2];
+        f32x4 dW2[4];
+        const f32x16 zero = {};
+#pragma unroll
+        for (int a = 0; a < 2; ++a) dW1[a][0] = dW1[a][1] = dW0[a] = zero;
+#pragma unroll
+        for (int T = 0; T < 4; ++T) dW2[T] = f32x4{0.f, 0.f, 0.f, 0.f};
+        uint4 xb[3];  // the group's X fragments: columns 8h, 16 + 8h, and 32 (h = 1: the bias inputs)
+        auto load = [&](int64_t rnd) {
+            const int64_t q = rnd * kRoundRec + GS * w + n;
+            xb[0] = xb[1] = xb[2] = make_uint4(0u, 0u, 0u, 0u);
+            if (q < total) {
+                const uint4* row = rec.xrow + 5 * q;
+                xb[0] = row[h];
+                xb[1] = row[2 + h];
+                if (h == 0) xb[2] = row[4];
+            }
+        };
+        const uint4* const w0p = sm.w0 + 128 * h + n;
+        const uint16_t* const w1p = sm.w1 + h * kHalfPitch + 8 * n;
+        // dW1 and dW0 of the round in the buffers
+        auto dw = [&]() {
+            uint4 fr[2][7];  // a k-step's operands, read one step ahead
+            // bytes from a group's first row: [feature tile][t][jj], and X's
+            uint32_t fa[5][2][2], xa;
+            {
+                int ro = rr, po = 4 * c16 + pc;
+                asm volatile("" : "+v"(ro), "+v"(po));  // anew in each round, like row_at
+                const int tile[5] = {2 * (w & 1), 2 * (w & 1) + 1, 2 * (w >> 1), 2 * (w >> 1) + 1, w};
+#pragma unroll
+                for (int f = 0; f < 5; ++f)
+#pragma unroll
+                    for (int tj = 0; tj < 4; ++tj)  // row 16 t + 8 jj + 4 h + rr, piece 8 T + po, swizzled
+                        fa[f][tj >> 1][tj & 1] = 256u * (8 * tj + 4 * h + ro) + 64u * (tile[f] ^ ro) +
+                                                 8u * (po ^ (2 * tj + h));
+                xa = 80u * (4 * h + ro) + 8u * po;
+            }
+            auto rd = [&](int g, int t, uint4 (&f)[7]) {
+                auto feat = [&](const uint16_t* rows, int i) {
+                    const uint8_t* b = reinterpret_cast<const uint8_t*>(rows + GS * 128 * g);
+                    return ld_tr2(b + fa[i][t][0], b + fa[i][t][1]);
+                };
+                f[0] = feat(sm.h0, 0);
+                f[2] = feat(sm.g1, 2);
+                f[1] = feat(sm.h0, 1);
+                f[3] = feat(sm.g1, 3);
+                const uint8_t* x = reinterpret_cast<const uint8_t*>(sm.x + 40 * (GS * g + 16 * t)) + xa;
+                f[4] = ld_tr2(x, x + 8 * 80);
+                f[6] = feat(sm.g0, 4);
+                f[5] = ld_tr2(x + 64, x + 64 + 8 * 80);
+            };
+            rd(0, 0, fr[0]);
+#pragma unroll
+            for (int g = 0; g < kBwdPairs; ++g)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const uint4(&f)[7] = fr[t];
+                    if (t == 0)
+                        rd(g, 1, fr[1]);
+                    else if (g + 1 < kBwdPairs)
+                        rd(g + 1, 0, fr[0]);
+                    dW1[0][0] = mfma32x32x16(f[0], f[2], dW1[0][0]);
+                    dW1[1][0] = mfma32x32x16(f[1], f[2], dW1[1][0]);
+                    dW1[0][1] = mfma32x32x16(f[0], f[3], dW1[0][1]);
+                    dW1[1][1] = mfma32x32x16(f[1], f[3], dW1[1][1]);
+                    dW0[0] = mfma32x32x16(f[4], f[6], dW0[0]);
+                    dW0[1] = mfma32x32x16(f[5], f[6], dW0[1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+        };
+        load(r0);
+        __syncthreads();  // the weights
+        for (int64_t rnd = r0; rnd < nrounds; rnd += stride) {
+            // ---- interval 1 ----
+            if (rnd != r0) dw();
+            __syncthreads();
+            // ---- interval 2 ----
+            {
+                uint4* xr = reinterpret_cast<uint4*>(sm.x + (GS * w + n) * 40);
+                xr[h] = xb[0];
+                xr[2 + h] = xb[1];
+                if (h == 0)
+                    xr[4] = xb[2];
+                else
+                    xb[2] = make_uint4(0x3f803f80u, 0x3f80u, 0u, 0u);
+            }
+            uint32_t h0[8][4];
+            const uint32_t at = row_at();
+            f32x16 c, d;  // a tile in the making, the one before
+            auto pair0 = [&](int T, int j) {
+                uint32_t* f = h0[2 * T + (j >> 2)];
+                f[j & 3] = relu_bf2(d[2 * j], d[2 * j + 1]);
+                if (j & 1) *piece(sm.h0, at, T, j >> 1) = make_uint2(f[(j & 3) - 1], f[j & 3]);
+            };
+#pragma unroll
+            for (int T = 0; T < 4; ++T) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    c = mfma32x32x16(w0p[256 * k + 32 * T], xb[k], k == 0 ? zero : c);
+                    if (T > 0) {
+                        pair0(T - 1, 3 * k);
+                        pair0(T - 1, 3 * k + 1);
+                        if (k < 2) pair0(T - 1, 3 * k + 2);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                d = c;
+            }
+            load(rnd + stride);
+            uint2 gl[4];  // dL/dlogit (lane & 3; the fourth's sums go unused) of samples 8q + 4h ..
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                gl[q] = *reinterpret_cast<const uint2*>(&sm.gl[w][GS * min(lane & 3, 2) + 8 * q + 4 * h]);
+            auto w1 = [&](int k) { return *reinterpret_cast<const uint4*>(w1p + k * kFragPitch); };
+            uint4 f1[3] = {w1(0), w1(1)};  // read two steps ahead
+            uint32_t r[2];
+            auto pair1 = [&](int T, int j) {
+                r[j & 1] = relu_bf2(d[2 * j], d[2 * j + 1]);
+                if (j & 1) dW2[T] = mfma4x4x4(gl[j >> 1].x, gl[j >> 1].y, r[0], r[1], dW2[T]);
+            };
+#pragma unroll
+            for (int T = 0; T < 4; ++T) {
+                const float b1 = __uint_as_float(sm.w2[32 * T + n].w);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) c[i] = b1;
+#pragma unroll
+                for (int ks = 0; ks < 8; ++ks) {
+                    const int k = 8 * T + ks;
+                    if (k < 30) f1[(k + 2) % 3] = w1(k + 2);
+                    c = mfma32x32x16(frag(h0[ks]), f1[k % 3], c);
+                    if (T > 0)
+                        pair1(T - 1, ks);
+                    else if (ks < 4) {  // the last layer-0 tile is k-steps 6 and 7's input
+                        pair0(3, 2 * ks);
+                        pair0(3, 2 * ks + 1);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                d = c;
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) pair1(3, j);
+            __syncthreads();
+        }
+        if (r0 < nrounds) dw();
+        __syncthreads();  // the buffers are free for the reductions
+#pragma unroll
+        for (int T = 0; T < 4; ++T)
 #pragma unroll
             for (int o = 0; o < 3; ++o) {
-                uint16_t h, l;
-                split_bf(gl[o], h, l);
-                sm.GLh[b][pr * GM + o] = h;
-                sm.GLl[b][pr * GM + o] = l;
-                sm.GLf[b][o * FM + pr] = h;
+                const float v = dW2[T][o] + __shfl_xor(dW2[T][o], 32, 64);
+                if (h == 0) red[384 * w + 3 * (32 * T + n) + o] = v;
             }
-        }
-        if (xe >= 0) {
-            *reinterpret_cast<uint4*>(&sm.Xh[b][xr * XM + 8 * xj]) = p_x;  // 16-byte aligned
-            const uint32_t w4[4] = {p_x.x, p_x.y, p_x.z, p_x.w};
+        // ---- this workgroup's dW partial ----
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                sm.Xf[b][(8 * xj + 2 * c) * FM + xr] = (uint16_t)(w4[c] & 0xffffu);
-                sm.Xf[b][(8 * xj + 2 * c + 1) * FM + xr] = (uint16_t)(w4[c] >> 16);
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int in = 32 * a + 8 * (i >> 2) + 4 * h + (i & 3);
+                out[kW1 + (64 * (w & 1) + in) * 128 + 64 * (w >> 1) + n] = dW1[a][0][i];
+                out[kW1 + (64 * (w & 1) + in) * 128 + 64 * (w >> 1) + 32 + n] = dW1[a][1][i];
+                if (in < 39)
+                    out[kW0 + in * 128 + 32 * w + n] = dW0[a][i];
+                else if (in == 39)
+                    out[kB0 + 32 * w + n] = dW0[a][i];
             }
-        }
-    };
-    // stage C of a group whose g_H0 and H1 sit in A2h/A2l, F3 and F2 (its
-    // inputs in buffer b, its records from pbase): dW2, dW0 and the records'
-    // feature gradients
-    auto finish = [&](int b, int64_t pbase) {
-        // dW2[in = f0 + row][out] += sum over the group's samples H1[s][in] gL[s][out]
-        dW2 = mfma16x16x32(ld_frag(&sm.F2[(f0 + r16) * FM + 8 * g]),
-                           ld_frag(&sm.GLf[b][r16 * FM + 8 * g]), dW2);
-        {
-            const bf16x8 bh = ld_frag(&sm.F3[(f0 + r16) * FM + 8 * g]);
-#pragma unroll
-            for (int mi = 0; mi < 3; ++mi)
-                dW0[mi] = mfma16x16x32(ld_frag(&sm.Xf[b][(16 * mi + r16) * FM + 8 * g]), bh, dW0[mi]);
-        }
-        if (wv < NT) {
-            const int nt = wv;
-            f32x4 gx = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
-                const int go = (16 * nt + r16) * SM + 32 * kt + 8 * g;
-                gx = mfma_w(as_bf8(sm.Bw0[kt * 64 + lane]), ld_frag(&sm.A2h[go]),
-                            ld_frag(&sm.A2l[go]), gx);
-            }
-            // lane (g, r16): features 4g..4g+3 of sample 16 nt + r16 = part g of its
-            // record's gradient; part 3 carries dL/dsigma
-            const int sidx = 16 * nt + r16;
-            const int64_t q = pbase + sidx;
-            if (q < total) {
-                const uint32_t bits = sm.bits[b][sidx];
-                float4 v = z4;
-                if (g < 3) {
-                    if (bits & kAliveW) v = make_float4(gx[0], gx[1], gx[2], gx[3]);
-                } else {
-                    v.x = sm.gsig[b][sidx];
-                }
-                rec.grad[4 * q + g] = v;
-            }
-        }
-    };
-
-    stage(blockIdx.x);
-    park(0);
-    __syncthreads();
-    int cb = 0;          // buffer of the current group
-    int64_t pbase = -1;  // the previous group, whose stage C is pending (-1: none)
-
-    for (int64_t grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {  // uniform bound
-        const int64_t base = grp * GS, next = grp + gridDim.x;
-        stage(next);  // in flight during this group's products, parked at its end
-        // ---- 1. this group's stage A: H0^T slice = W0^T X^T + b0 under the
-        //         forward's mask -> A1h, H0f; g_H1^T slice = W2[slice] g_L^T under
-        //         the mask -> G1h, G1l, G1f.  The previous group's stage C ----
-        uint32_t m0 = 0u, m1 = 0u;  // the forward's ReLU masks: bit at(nt, i)
-        auto at = [](int nt, int i) { return 16 * (i & 1) + 2 * nt + (i >> 1); };
-        {
-            // features fr..fr+3: bits 2wv, 16 + 2wv, 2wv + 1, 17 + 2wv of word g
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const uint32_t* mw = &sm.relu[cb][8 * (16 * nt + r16)];
-                m0 |= ((mw[g] >> (2 * wv)) & 0x30003u) << (nt * 2);
-                m1 |= ((mw[4 + g] >> (2 * wv)) & 0x30003u) << (nt * 2);
-            }
-        }
-        f32x4 acc[NT];  // starting at the bias, as in the forward
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{b0v[0], b0v[1], b0v[2], b0v[3]};
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const int xo = (16 * nt + r16) * XM + 32 * kt + 8 * g;
-                acc[nt] = mfma16x16x32(A0[kt], ld_frag(&sm.Xh[cb][xo]), acc[nt]);
-            }
-        }
-        {
-            const s16x4 a = __builtin_bit_cast(s16x4, sm.Bw2[wv * 64 + lane]);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                f32x4 c4 = {0.f, 0.f, 0.f, 0.f};
-                const int go = (16 * nt + r16) * GM + 4 * g;
-                c4 = mfma16x16x16(a, ld_frag4(&sm.GLh[cb][go]), c4);
-                c4 = mfma16x16x16(a, ld_frag4(&sm.GLl[cb][go]), c4);
-                float gv[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    gv[i] = keep_if(m1, at(nt, i), c4[i]);
-                    db1[i] += gv[i];
-                }
-                st_act<true>(sm.G1h, sm.G1l, sm.G1f, 16 * nt + r16, fr, lane, gv);
-            }
-        }
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            float h[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) h[i] = keep_if(m0, at(nt, i), acc[nt][i]);
-            st_hi_fm(sm.A1h, sm.H0f, 16 * nt + r16, fr, lane, h);
-        }
-        if (pbase >= 0) finish(cb ^ 1, pbase);
-        __syncthreads();
-        // ---- 2. B. H1^T slice = W1^T H0^T + b1 under the mask -> F2 (dW2 only);
-        //         g_H0^T tile = W1[rows] g_H1^T under the mask -> A2h, A2l, F3;
-        //         dW1 += H0^T g_H1; the next group's records are parked ----
-        // (g_H0 in 32 features x 16 samples per wave: half the g_H1 reads of 16 x 32)
-        f32x4 acc2[2];
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt) acc2[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            const int go = (16 * sh + r16) * SM + 32 * kt + 8 * g;
-            const bf16x8 bh = ld_frag(&sm.G1h[go]), bl = ld_frag(&sm.G1l[go]);
-#pragma unroll
-            for (int mt = 0; mt < 2; ++mt) acc2[mt] = mfma_w(Bw1r[mt][kt], bh, bl, acc2[mt]);
-        }
-        {
-            // dW1[in][out] += sum over samples H0[s][in] g_H1[s][out]; this wave's
-            // block: inputs 64 (wv & 1) .. +63, outputs 32 (wv >> 1) .. +31 (fewer
-            // LDS reads than a full column of 128 inputs x 16 outputs)
-            const int i0 = 64 * (wv & 1), o0 = 32 * (wv >> 1);
-            const bf16x8 b0 = ld_frag(&sm.G1f[(o0 + r16) * FM + 8 * g]);
-            const bf16x8 b1 = ld_frag(&sm.G1f[(o0 + 16 + r16) * FM + 8 * g]);
-#pragma unroll
-            for (int mi = 0; mi < 4; ++mi) {
-                const bf16x8 a = ld_frag(&sm.H0f[(i0 + 16 * mi + r16) * FM + 8 * g]);
-                dW1[2 * mi] = mfma16x16x32(a, b0, dW1[2 * mi]);
-                dW1[2 * mi + 1] = mfma16x16x32(a, b1, dW1[2 * mi + 1]);
-            }
-        }
-        {
-            // g_H0 masked by the layer-0 bits of features 32 fb .. +31
-            const uint32_t mw = sm.relu[cb][8 * (16 * sh + r16) + g] >> (4 * fb);
-#pragma unroll
-            for (int mt = 0; mt < 2; ++mt) {
-                float gv[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    gv[i] = keep_if(mw, 16 * (i & 1) + 2 * mt + (i >> 1), acc2[mt][i]);
-                st_act<true>(sm.A2h, sm.A2l, sm.F3, 16 * sh + r16, 32 * fb + 16 * mt + 4 * g, lane,
-                             gv);
-            }
-        }
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{b1v[0], b1v[1], b1v[2], b1v[3]};
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const int ho = (16 * nt + r16) * SM + 32 * kt + 8 * g;
-                acc[nt] = mfma16x16x32(A1[kt], ld_frag(&sm.A1h[ho]), acc[nt]);
-            }
-        }
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            float h[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) h[i] = keep_if(m1, at(nt, i), acc[nt][i]);
-            st_fm(sm.F2, 16 * nt + r16, fr, lane, h);
-        }
-        park(cb ^ 1);  // the next group's records, loaded at this group's start
-        __syncthreads();
-        pbase = base;
-        cb ^= 1;
-    }
-    if (pbase >= 0) finish(cb ^ 1, pbase);  // the loop ended on a barrier
-
-    // ---- flush this workgroup's dW partial ----
-    float* out = dw_partial + (int64_t)blockIdx.x * kPartStride;
-#pragma unroll
-    for (int mi = 0; mi < 3; ++mi)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int in = 16 * mi + 4 * g + i, o = f0 + r16;
-            if (in < 39)
-                out[kW0 + in * 128 + o] = dW0[mi][i];
-            else if (in == 39)
-                out[kB0 + o] = dW0[mi][i];
-        }
-#pragma unroll
-    for (int t = 0; t < 8; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int in = 64 * (wv & 1) + 16 * (t >> 1) + 4 * g + i;
-            const int o = 32 * (wv >> 1) + 16 * (t & 1) + r16;
-            out[kW1 + in * 128 + o] = dW1[t][i];
-        }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        if (r16 < 3) out[kW2 + (fr + i) * 3 + r16] = dW2[i];
-        float v = db1[i];
-        v += __shfl_xor(v, 1, 64);
-        v += __shfl_xor(v, 2, 64);
-        v += __shfl_xor(v, 4, 64);
-        v += __shfl_xor(v, 8, 64);
-        if (r16 == 0) out[kB1 + fr + i] = v;
-    }
-    // db2 was accumulated by the staging lanes (park); the loop ended on a barrier,
-    // so gsig[0] is free for the per-wave sums
-#pragma unroll
-    for (int o = 0; o < 3; ++o) {
-        float v = pr >= 0 ? db2[o] : 0.f;
-        v += __shfl_xor(v, 1, 64);
-        v += __shfl_xor(v, 2, 64);
-        v += __shfl_xor(v, 4, 64);
-        if (lane == 0) sm.gsig[0][4 * wv + o] = v;
     }
     __syncthreads();
+    const int tid = threadIdx.x;
+    if (tid < 384) {
+        out[kW2 + tid] = ((red[tid] + red[384 + tid]) + red[768 + tid]) + red[1152 + tid];
+    } else {
+        const float* d = red + kRedDb1 + (tid - 384);
+        out[kB1 + tid - 384] = ((d[0] + d[128]) + d[256]) + d[384];
+    }
     if (tid < 3) {
-        float v = 0.f;
-#pragma unroll
-        for (int w = 0; w < kBwdWaves; ++w) v += sm.gsig[0][4 * w + tid];
-        out[kB2 + tid] = v;
+        const float* d = red + kRedDb2 + tid;
+        out[kB2 + tid] = ((d[0] + d[4]) + d[8]) + d[12];
     }
 }
 

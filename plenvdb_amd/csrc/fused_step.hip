@@ -53,7 +53,7 @@ struct Layout {
     size_t count, offset, total, t_last, ray_out, ray_grad, ray_ctot, ray_loss, ray_rgb, loss, steps,
         pe, setup, zero;
     size_t xyze, ab, rgb, adj, xrow, relu, grad;
-    size_t touched, dw_part, w0t, w1t, fwd, w2, w1, w0;
+    size_t touched, dw_part, fwd, w2, w0;
     size_t bytes;
 };
 
@@ -91,11 +91,8 @@ Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
     L.grad = take(64 * capacity);
     L.touched = take(nleaf > 0 ? nleaf : 1);
     L.dw_part = take((size_t)4 * kPartStride * kMaxMlpGrid);
-    L.w0t = take(2 * 128 * 64);
-    L.w1t = take(2 * 128 * 128);
     L.fwd = take(2 * kFwdImage);
     L.w2 = take(2 * 128 * 32);
-    L.w1 = take(2 * 128 * 128);
     L.w0 = take(2 * 16 * 128);
     L.bytes = o;
     return L;
@@ -567,20 +564,13 @@ int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
     rec.grad = reinterpret_cast<float4*>(ws + L.grad);
     uint8_t* touched = ws + L.touched;
     float* dw_part = reinterpret_cast<float*>(ws + L.dw_part);
-    uint16_t* w0t = reinterpret_cast<uint16_t*>(ws + L.w0t);
-    uint16_t* w1t = reinterpret_cast<uint16_t*>(ws + L.w1t);
     uint16_t* fwd = reinterpret_cast<uint16_t*>(ws + L.fwd);
     uint16_t* w2 = reinterpret_cast<uint16_t*>(ws + L.w2);
-    uint16_t* w1 = reinterpret_cast<uint16_t*>(ws + L.w1);
     uint16_t* w0 = reinterpret_cast<uint16_t*>(ws + L.w0);
     MlpPacked W;
-    W.w0t = w0t;
-    W.w1t = w1t;
     W.fwd = reinterpret_cast<const uint4*>(fwd);
     W.w2 = w2;
-    W.w1 = w1;
     W.w0 = w0;
-    W.b0 = direct ? nullptr : d->mlp + kB0;
     W.b1 = direct ? nullptr : d->mlp + kB1;
     W.b2 = direct ? nullptr : d->mlp + kB2;
 
@@ -599,7 +589,7 @@ int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
         // the counting march also packs the bf16 MLP operands and zeroes the
         // MLP gradient (accumulated by k_dw_reduce later in the step)
         StageScope sc(1, s);
-        PackArgs pk{d->mlp, w0t, w1t, fwd, w2, w1, w0, d->mlp_grad,
+        PackArgs pk{d->mlp, fwd, w2, w0, d->mlp_grad,
                     reinterpret_cast<uint32_t*>(ws + L.zero)};
         if (direct) pk.prm = nullptr;
         if ((rc = launch_ray_count(P, t, R, pk, s))) return rc;
