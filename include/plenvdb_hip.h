@@ -111,6 +111,12 @@ int pvdb_set_values_by_mask(const pvdb_topology* topo, float* vals, const uint8_
 int pvdb_tv_add_grad(const pvdb_topology* topo, const float* vals /*dev*/, float* grad /*dev*/,
                      int32_t channels, int32_t rx, int32_t ry, int32_t rz, float wx, float wy,
                      float wz, int32_t dense_mode, void* stream);
+/* World points [n][3] to index space, (p - min) / (max - min) * (world_size - 1)
+ * (grid.py:77-78), as rows out[0..n) = x, out[n..2n) = y, out[2n..3n) = z.  xyz_min,
+ * xyz_max and ws_minus_1 are dev [3]. */
+int pvdb_world_to_index(const float* pts /*dev*/, int64_t n, const float* xyz_min,
+                        const float* xyz_max, const float* ws_minus_1, float* out /*dev*/,
+                        void* stream);
 /* zero_grad (densityvdb.cu:353-368, colorvdb.cu:355-371; plenvdb.cpp:94,120). */
 int pvdb_zero_active(const pvdb_topology* topo, float* grad, int32_t channels, void* stream);
 /* DensityOpt/ColorOpt::step_optimizer kernels (plenvdb.h:751-789;
@@ -308,6 +314,10 @@ typedef struct pvdb_step_desc {
     int32_t stepmode_color;
 } pvdb_step_desc;
 
+/* Writes the three step sizes of pvdb_step_desc.adam_scalars (dev [3]) on `stream`,
+ * from the host's values and without a wait: before each replay of a captured step. */
+int pvdb_fused_set_scalars(float* adam_scalars, float stepsz_density, float stepsz_color,
+                           float step_size_mlp, void* stream);
 /* The default launch shapes (pvdb_step_desc.launch) on the current device. */
 int pvdb_fused_launch_defaults(int32_t* launch4);
 /* Workspace bytes for n_rays rays, `capacity` records and nleaf leaves (-1 on bad sizes). */

@@ -103,6 +103,14 @@ __global__ void k_fill_u8(uint8_t* p, int64_t n, uint8_t v) {
     if (i < n) p[i] = v;
 }
 
+__global__ void k_set_scalars(float* p, float a, float b, float c) {
+    if (threadIdx.x == 0) {
+        p[0] = a;
+        p[1] = b;
+        p[2] = c;
+    }
+}
+
 __device__ __forceinline__ void adam1(float& p, float g, float& m, float& v, float sz, float eps,
                                       float b0, float b1) {
     const float nm = b0 * m + (1.f - b0) * g;
@@ -394,6 +402,15 @@ int pvdb_fused_launch_defaults(int32_t* launch4) {
     launch4[1] = kScatterGrid;
     launch4[2] = kScatterChunk;
     launch4[3] = kRayWaves;
+    return PVDB_OK;
+}
+
+int pvdb_fused_set_scalars(float* adam_scalars, float stepsz_density, float stepsz_color,
+                           float step_size_mlp, void* stream) {
+    PVDB_CHECK_ARG(adam_scalars != nullptr, "adam_scalars is NULL");
+    hipLaunchKernelGGL(k_set_scalars, dim3(1), dim3(64), 0, (hipStream_t)stream, adam_scalars,
+                       stepsz_density, stepsz_color, step_size_mlp);
+    PVDB_LAUNCHED("k_set_scalars");
     return PVDB_OK;
 }
 

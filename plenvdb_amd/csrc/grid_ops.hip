@@ -197,6 +197,20 @@ __global__ void __launch_bounds__(256) k_tri_bwd_agg(TopoView t, float* __restri
     }
 }
 
+// World to index coordinates (grid.py:77-78), a point to a thread, transposed to the
+// rows that the gather and the scatter read.  As tensor operations this was five
+// launches, 32 us of device time for 1.2M points and about as long on the host.
+__global__ void __launch_bounds__(256) k_world_to_index(const float* __restrict__ pts, int64_t n,
+                                                        const float* __restrict__ mn,
+                                                        const float* __restrict__ mx,
+                                                        const float* __restrict__ ws,
+                                                        float* __restrict__ out) {
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= n) return;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) out[a * n + p] = (pts[3 * p + a] - mn[a]) / (mx[a] - mn[a]) * ws[a];
+}
+
 __device__ __forceinline__ bool slot_active(const TopoView& t, int64_t slot) {
     const int64_t leaf = slot >> 9;
     const int off = (int)(slot & 511);
@@ -581,6 +595,17 @@ int pvdb_tv_add_grad(const pvdb_topology* topo, const float* vals, float* grad,
                            (hipStream_t)stream, t, vals, grad, channels, rx, ry, rz, wy / 6.f,
                            wz / 6.f, dense_mode != 0 ? 1 : 0);
     PVDB_LAUNCHED("k_tv_add_grad");
+    return PVDB_OK;
+}
+
+int pvdb_world_to_index(const float* pts, int64_t n, const float* xyz_min, const float* xyz_max,
+                        const float* ws_minus_1, float* out, void* stream) {
+    PVDB_CHECK_ARG(n >= 0, "n must be >= 0");
+    if (n == 0) return PVDB_OK;
+    PVDB_CHECK_ARG(pts && xyz_min && xyz_max && ws_minus_1 && out, "null pointer");
+    hipLaunchKernelGGL(k_world_to_index, dim3(pvdb_blocks(n, 256)), dim3(256), 0,
+                       (hipStream_t)stream, pts, n, xyz_min, xyz_max, ws_minus_1, out);
+    PVDB_LAUNCHED("k_world_to_index");
     return PVDB_OK;
 }
 

@@ -11,6 +11,7 @@ import numpy as np
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import lib
 from .plenvdb import ColorVDB, DensityVDB
@@ -62,9 +63,25 @@ class VDBGrid(nn.Module):
         """(pts-min)/(max-min)*(world_size-1), grid.py:77-78."""
         return (pts - self.xyz_min) / (self.xyz_max - self.xyz_min) * self.ws_minus_1
 
+    def _index_points(self, xyz):
+        """wld2idx of the points as [3, N] rows: one launch for plain contiguous
+        fp32 points on the current device that take no gradient, tensor operations
+        for the rest (the values are the same)."""
+        b = (self.xyz_min, self.xyz_max, self.ws_minus_1)
+        if (type(xyz) is torch.Tensor and xyz.is_cuda and xyz.dtype == torch.float32
+                and xyz.shape[-1:] == (3,) and xyz.is_contiguous() and not xyz.requires_grad
+                and xyz.get_device() == torch.cuda.current_device() and forward_ad._current_level < 0
+                and all(t.device == xyz.device and t.dtype == torch.float32 and t.numel() == 3
+                        and t.is_contiguous() for t in b)):
+            n = xyz.numel() // 3
+            out = torch.empty(3, n, dtype=torch.float32, device=xyz.device)
+            lib.call("pvdb_world_to_index", lib.ptr(xyz), n, *map(lib.ptr, b), lib.ptr(out), lib.stream())
+            return out
+        return self.wld2idx(xyz).reshape(-1, 3).t().contiguous().float()
+
     def forward(self, xyz):
         shape = xyz.shape[:-1]
-        pts = self.wld2idx(xyz).reshape(-1, 3).t().contiguous().float().requires_grad_()
+        pts = self._index_points(xyz).requires_grad_()
         out = QueryVerticalInVDB.apply(pts, self.grid).reshape([*shape, self.channels])
         if self.channels == 1:
             out = out.squeeze(-1)

@@ -69,3 +69,29 @@ def test_scatter_keeps_nan_and_infinity():
     row = v.grad[int((3 << 6) | (3 << 3) | 3)].cpu()
     assert torch.isnan(row[0]) and torch.isinf(row[1]) and row[11] == -0.125
     assert (row[2:11] == 0).all()
+
+
+@pytest.mark.parametrize("n", [0, 1, 255, 257])
+def test_index_points_equal_tensor_operations(n):
+    from plenvdb_amd.grid import VDBGrid
+
+    g = VDBGrid(1, [37, 20, 9], [-1.5, -0.25, 0.1], [1.5, 0.75, 2.0], topology=_topo(37, 1)).to("cuda")
+    xyz = torch.randn(n, 3, device="cuda") * 2
+    xyz[: n // 4] = float("inf")
+    want = g.wld2idx(xyz).t().contiguous()
+    torch.testing.assert_close(g._index_points(xyz), want, rtol=0, atol=0, equal_nan=True)
+    strided = torch.empty(3, n, device="cuda").copy_(xyz.t()).t()
+    torch.testing.assert_close(g._index_points(strided), want, rtol=0, atol=0, equal_nan=True)
+    assert not xyz.requires_grad
+    lead = g._index_points(xyz.requires_grad_())  # keeps its place in the caller's graph
+    assert lead.requires_grad
+
+
+def test_step_refuses_a_foreign_capture(monkeypatch):
+    from plenvdb_amd import scenes
+    from plenvdb_amd.fused import FusedTrainer
+
+    tr = FusedTrainer(scenes.make_scene("c2", n_rays=8))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="capture_graph"):
+        tr.step()
