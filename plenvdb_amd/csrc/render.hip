@@ -1,5 +1,5 @@
 // Merged-VDB renderer: MGRenderer::render_an_image (plenvdb/lib/vdb/plenvdb.h:
-// 1029-1035 -> renderer.cu:370-424) in five kernels and no host round trip.
+// 1029-1035 -> renderer.cu:370-424) in four kernels and no host round trip.
 //
 // The reference renders in two full marches per pixel (first_look_merged
 // counts the kept samples and rewrites t_min / t_max, renderer.cu:222-268;
@@ -20,11 +20,10 @@
 //                   them, contiguous per pixel.  So the sample set is the
 //                   reference's, including the second march's restart
 //                   (renderer.cu:263).
-//   k_render_gather the records' colour features, a thread per record.
-//   k_render_mlp    persistent waves over 64-record chunks: the RGB MLP on
-//                   v_mfma_f32_16x16x32_f16 (weights in LDS, shared by the
-//                   workgroup's 8 waves) and each record's contribution
-//                   w / (1 + exp(-raw)) (final_render).
+//   k_render_mlp    persistent waves over 32-record groups: the records' colour
+//                   features gathered under the group before's MFMAs, the RGB MLP on
+//                   v_mfma_f32_32x32x16_f16 (weights in LDS) and each record's
+//                   contribution w / (1 + exp(-raw)) (final_render).
 //   k_render_composite  per pixel: T_last * bg plus its records' contributions,
 //                   eight lanes per pixel reading its run of records together
 //                   (a fixed order, so frames are reproducible).
@@ -39,13 +38,11 @@
 // (k_render_cells), which the marches read.
 //
 // MLP.  Layer outputs are computed transposed (features x samples) and stay in
-// registers: the D fragment of one layer (lane (g,n): features 16m+4g+i of
-// sample n) is the B fragment of the next once the next layer's weights are
-// stored with their K index permuted accordingly (see kperm).  Weights are
-// fp16 in LDS, read as 16-byte fragments.  The first layer's input row is
-// [feature 0..11 | 0 x4 | PE 0..26 | 1 | 0 ...] (64 halves), so its bias is a
-// weight column and a record's 16-byte halves and the pixel's PE row land on
-// 16-byte boundaries.
+// registers: the D fragment of one layer is the B fragment of the next once the
+// next layer's weights are stored with their K index permuted accordingly (see
+// rperm).  Weights are fp16 in LDS, read as 16-byte fragments.  The first layer's
+// input row is [feature 0..11 | PE 0..26 | 1] (40 halves), so its bias is a weight
+// column; a pixel's PE row holds column c at position c - 8.
 #include <cmath>
 #include <mutex>
 #include <type_traits>
@@ -66,22 +63,26 @@ using namespace pvdb;
 namespace {
 
 constexpr int kHid = 128;
-constexpr int kWaves = 8;   // MLP waves per workgroup: they share the LDS weights
-constexpr int XS = 72;      // halves per staged input row (64 + 8)
-constexpr int kPeIn = 16;   // first-layer input of PE component 0
-constexpr int kW0Frag = 8 * 2 * 64 * 8;  // [m-tile 8][k-step 2][lane][8]
-constexpr int kW1Frag = 8 * 4 * 64 * 8;  // [m-tile 8][k-step 4][lane][8]
-constexpr int kW2Frag = 4 * 64 * 8;      // [k-step 4][lane][8]
+constexpr int kMlpWaves = 4;  // MLP waves per workgroup: they share the LDS weights
+// The MLP's LDS image, as pvdb_render_pack_weights lays it out.
+struct alignas(16) RenderSmem {
+    uint4 w0[6 * 128];  // [chunk][hidden feature]: W0^T columns 8c .. 8c + 7 (39: b0; 40..47: 0)
+    uint4 w1[32 * 64];  // [row tile][k-step][lane]: W1^T's A fragments, K permuted
+    uint4 w2[8 * 2 * 4];  // [k-step][h][logit]: W2^T rows, K permuted
+    float b[128 + 4];   // b1, b2
+};
+constexpr int kW0Frag = 6 * 128 * 8, kW1Frag = 32 * 64 * 8, kW2Frag = 8 * 2 * 4 * 8;
 constexpr int kPackedHalves = kW0Frag + kW1Frag + kW2Frag;
-constexpr int kBiasFloats = 128 + 4;  // b1, b2 (padded)
+constexpr int kBiasFloats = 128 + 4;
 constexpr int kPackedBytes = kPackedHalves * 2 + kBiasFloats * 4;
+static_assert(sizeof(RenderSmem) == kPackedBytes, "the image is the struct");
 constexpr int kMarchThreads = 256;    // 4 waves per march workgroup
 constexpr int64_t kMaxRecords = 0x7fffffffll;  // record indices are int32 in the pixel table
 
-// Position j (0..7) of k-step s in lane group g holds feature kperm(s, g, j):
-// the features lane group g of the previous layer's D fragments carries.
-__host__ __device__ __forceinline__ int kperm(int s, int g, int j) {
-    return 32 * s + 4 * g + (j & 3) + ((j >> 2) << 4);
+// Position j (0..7) of k-step s in lane half h holds feature rperm(s, h, j): what
+// that half of the previous layer's D fragments carries.
+__host__ __device__ __forceinline__ int rperm(int s, int h, int j) {
+    return 16 * s + 8 * (j >> 2) + 4 * h + (j & 3);
 }
 
 __global__ void k_render_pack(const float* __restrict__ w0, const float* __restrict__ b0,
@@ -91,27 +92,16 @@ __global__ void k_render_pack(const float* __restrict__ w0, const float* __restr
                               float* __restrict__ outb) {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx < kW0Frag) {
-        const int j = idx & 7, lane = (idx >> 3) & 63, ms = idx >> 9;
-        const int s = ms & 1, m = ms >> 1, g = lane >> 4, r = lane & 15;
-        const int o = 16 * m + r, in = 32 * s + 8 * g + j;
-        float v = 0.f;
-        if (in < dcol)
-            v = w0[in * kHid + o];
-        else if (in >= kPeIn && in < kPeIn + dpe)
-            v = w0[(dcol + in - kPeIn) * kHid + o];
-        else if (in == kPeIn + dpe)
-            v = b0[o];
-        outh[idx] = (_Float16)v;
+        const int in = 8 * (idx >> 10) + (idx & 7), o = (idx >> 3) & 127;
+        outh[idx] = (_Float16)(in < dcol + dpe ? w0[in * kHid + o] : in == dcol + dpe ? b0[o] : 0.f);
     } else if (idx < kW0Frag + kW1Frag) {
         const int q = idx - kW0Frag;
-        const int j = q & 7, lane = (q >> 3) & 63, ms = q >> 9;
-        const int s = ms & 3, m = ms >> 2, g = lane >> 4, r = lane & 15;
-        outh[idx] = (_Float16)w1[kperm(s, g, j) * kHid + 16 * m + r];
+        const int lane = (q >> 3) & 63, ts = q >> 9;
+        outh[idx] = (_Float16)w1[rperm(ts & 7, lane >> 5, q & 7) * kHid + 32 * (ts >> 3) + (lane & 31)];
     } else if (idx < kPackedHalves) {
         const int q = idx - kW0Frag - kW1Frag;
-        const int j = q & 7, lane = (q >> 3) & 63, s = q >> 9;
-        const int g = lane >> 4, r = lane & 15;
-        outh[idx] = (_Float16)(r < dout ? w2[kperm(s, g, j) * dout + r] : 0.f);
+        const int o = (q >> 3) & 3;
+        outh[idx] = (_Float16)(o < dout ? w2[rperm(q >> 6, (q >> 5) & 1, q & 7) * dout + o] : 0.f);
     } else if (idx < kPackedHalves + kBiasFloats) {
         const int q = idx - kPackedHalves;
         outb[q] = q < 128 ? b1[q] : (q - 128 < dout ? b2[q - 128] : 0.f);
@@ -169,7 +159,7 @@ struct FrameBuffers {
     float2* tspan;                   // [HW] pass 2's t range (rewritten t_min, t_max)
     int32_t* pix_written;            // [HW] records pass 2 filled (<= count)
     float* t_last;                   // [HW] transmittance after pass 2
-    uint4* pe;                       // [HW][4] PE row: 27 halves, 1, 0 x4
+    uint4* pe;                       // [HW][4] PE row: 0 x4, 27 halves, 1
     uint4* rec;                      // [capacity][2] records
     float4* contrib;                 // [capacity] w * sigmoid(raw), per channel
     int64_t capacity;
@@ -235,112 +225,18 @@ struct CellRow {
     }
 };
 
-template <bool F32PAY>
-__device__ __forceinline__ void load_col(const void* pay, int64_t slot, float* c12) {
-    if (F32PAY) {
-        const float4* p = reinterpret_cast<const float4*>(pay) + slot * 4;
-        const float4 a = p[0], b = p[1], c = p[2], d = p[3];
-        c12[0] = a.y; c12[1] = a.z; c12[2] = a.w;
-        c12[3] = b.x; c12[4] = b.y; c12[5] = b.z; c12[6] = b.w;
-        c12[7] = c.x; c12[8] = c.y; c12[9] = c.z; c12[10] = c.w;
-        c12[11] = d.x;
-    } else {
-        const uint4* p = reinterpret_cast<const uint4*>(pay) + slot * 2;
-        const uint4 a = p[0], b = p[1];
-        const uint32_t w[7] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z};
-#pragma unroll
-        for (int c = 0; c < 12; ++c) {
-            const int h = c + 1;  // half index: 0 is the density
-            c12[c] = h2f((uint16_t)(w[h >> 1] >> (16 * (h & 1))));
-        }
-    }
-}
-
 __device__ __forceinline__ f16x8 as_h8(const uint4& v) { return __builtin_bit_cast(f16x8, v); }
-
-// RGB logits of the 64 samples staged in this wave's rows of sX (row =
-// lane); lanes 0..15 write them to sL (the rows of empty tiles hold zeros, so
-// their logits are the bias and are not read).  All four 16-sample tiles go
-// through each layer together, so every weight fragment read from LDS feeds
-// four MFMAs and the tiles' activations stay in registers.
-__device__ __forceinline__ void wave_mlp(const uint4* __restrict__ sW, const float* __restrict__ sB,
-                                         const _Float16* __restrict__ sX, float* __restrict__ sL,
-                                         int lane) {
-    const int g = lane >> 4, r16 = lane & 15;
-    const uint4* W0 = sW;
-    const uint4* W1 = sW + kW0Frag / 8;
-    const uint4* W2 = W1 + kW1Frag / 8;
-    uint32_t h0[4][4][4];  // [tile][k-step][dword]: layer-1 B fragments (fp16 pairs)
-    {
-        f16x8 xb[4][2];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                xb[u][s] = as_h8(*reinterpret_cast<const uint4*>(sX + (16 * u + r16) * XS +
-                                                                 32 * s + 8 * g));
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            const f16x8 a0 = as_h8(W0[(m * 2 + 0) * 64 + lane]);
-            const f16x8 a1 = as_h8(W0[(m * 2 + 1) * 64 + lane]);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                acc = mfma16x16x32h(a0, xb[u][0], acc);
-                acc = mfma16x16x32h(a1, xb[u][1], acc);
-                const int s = m >> 1, d = (m & 1) * 2;
-                h0[u][s][d] = relu_pack2(acc[0], acc[1]);
-                h0[u][s][d + 1] = relu_pack2(acc[2], acc[3]);
-            }
-        }
-    }
-    // layer 1, and layer 2 as its outputs appear: layer 2's k-step s takes
-    // layer 1's output tiles 2s and 2s + 1, so only one k-step of H1 is live
-    const float b2x = sB[128], b2y = sB[129], b2z = sB[130];
-    f32x4 acc2[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) acc2[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s2 = 0; s2 < 4; ++s2) {
-        uint32_t hk[4][4];  // [tile][dword]: layer 2's B fragments of k-step s2
-#pragma unroll
-        for (int mm = 0; mm < 2; ++mm) {
-            const int m = 2 * s2 + mm;
-            // the accumulators start at the bias (the MFMA adds it)
-            const float4 bias = *reinterpret_cast<const float4*>(sB + 16 * m + 4 * g);
-            f32x4 acc[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc[u] = f32x4{bias.x, bias.y, bias.z, bias.w};
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const f16x8 a = as_h8(W1[(m * 4 + s) * 64 + lane]);
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const uint4 bv = make_uint4(h0[u][s][0], h0[u][s][1], h0[u][s][2], h0[u][s][3]);
-                    acc[u] = mfma16x16x32h(a, as_h8(bv), acc[u]);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                hk[u][2 * mm] = relu_pack2(acc[u][0], acc[u][1]);
-                hk[u][2 * mm + 1] = relu_pack2(acc[u][2], acc[u][3]);
-            }
-        }
-        const f16x8 a2 = as_h8(W2[s2 * 64 + lane]);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            acc2[u] = mfma16x16x32h(a2, as_h8(make_uint4(hk[u][0], hk[u][1], hk[u][2], hk[u][3])),
-                                    acc2[u]);
-    }
-    if (g == 0) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            float* dst = sL + (16 * u + r16) * 4;
-            dst[0] = acc2[u][0] + b2x;
-            dst[1] = acc2[u][1] + b2y;
-            dst[2] = acc2[u][2] + b2z;
-        }
-    }
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ f32x16 mfma32x32x16h(const uint4& a, const uint4& b, const f32x16& c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(as_h8(a), as_h8(b), c, 0, 0, 0);
+}
+// v_mfma_f32_4x4x4_16b_f16: sixteen 4 x 4 products, block lane / 4; a lane holds
+// A[lane % 4][0..3] and B[0..3][lane % 4] of its block and gets D[0..3][lane % 4].
+__device__ __forceinline__ f32x4 mfma4x4x4h(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1,
+                                            const f32x4& c) {
+    typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, make_uint2(a0, a1)),
+                                              __builtin_bit_cast(f16x4, make_uint2(b0, b1)), c, 0, 0, 0);
 }
 
 // Leaf index of (i,j,k) through a one-entry cache of its 8^3 block.
@@ -377,8 +273,8 @@ __device__ __forceinline__ void pixel_dir(const RenderArgs& A, int px, int py, f
         rd[a] = dx * A.c2w[4 * a] + dy * A.c2w[4 * a + 1] + dz * A.c2w[4 * a + 2];
 }
 
-// The pixel's PE row (27 components of the view direction, dvgo.py:91-109
-// order, then the bias input 1 and four zeros) as 16 packed fp16 pairs.
+// The pixel's PE row (four zeros, then 27 components of the view direction,
+// dvgo.py:91-109 order, and the bias input 1) as 16 packed fp16 pairs.
 __device__ __forceinline__ void pixel_pe(const RenderArgs& A, int px, int py, uint32_t* pe) {
     float rd[3];
     pixel_dir(A, px, py, rd);
@@ -402,8 +298,8 @@ __device__ __forceinline__ void pixel_pe(const RenderArgs& A, int px, int py, ui
     }
     p27[27] = 1.f;  // the bias input
 #pragma unroll
-    for (int q = 0; q < 14; ++q) pe[q] = pack2(p27[2 * q], p27[2 * q + 1]);
-    pe[14] = pe[15] = 0u;
+    for (int q = 0; q < 14; ++q) pe[2 + q] = pack2(p27[2 * q], p27[2 * q + 1]);
+    pe[0] = pe[1] = 0u;
 }
 
 __device__ __forceinline__ PixelRay pixel_ray(const RenderArgs& A, int px, int py) {
@@ -468,30 +364,6 @@ __device__ __forceinline__ void advance_steps(float& t, float s, float tsafe, fl
     while (t + s < tsafe && t < tend && iter < max_iter) {
         t += s;
         ++iter;
-    }
-}
-
-// Slots of the 8 corners of the cell with lower corner (i0, j0, k0) in the
-// corner order 000,001,011,010,110,111,101,100 (slot nslots, index 0's
-// values, for a corner whose leaf does not exist).
-__device__ __forceinline__ void corner_slots(const RenderArgs& A, int i0, int j0, int k0,
-                                             BlockCache& bc, int32_t* slot) {
-    if (((i0 & 7) != 7) & ((j0 & 7) != 7) & ((k0 & 7) != 7)) {
-        // the cell lies inside one 8^3 block: one lookup, slots by in-leaf offset
-        const int32_t l0 = bc.get(A.topo, i0, j0, k0);
-        const int32_t s0 = l0 * 512 + voxel_offset(i0, j0, k0);
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int cx = (kCx >> q) & 1, cy = (kCy >> q) & 1, cz = (kCz >> q) & 1;
-            slot[q] = l0 < 0 ? (int32_t)A.nslots : s0 + ((cx << 6) | (cy << 3) | cz);
-        }
-        return;
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        const int cx = (kCx >> q) & 1, cy = (kCy >> q) & 1, cz = (kCz >> q) & 1;
-        const int32_t lq = bc.get(A.topo, i0 + cx, j0 + cy, k0 + cz);
-        slot[q] = lq < 0 ? (int32_t)A.nslots : lq * 512 + voxel_offset(i0 + cx, j0 + cy, k0 + cz);
     }
 }
 
@@ -778,7 +650,7 @@ __global__ void __launch_bounds__(kMarchThreads) k_render_fill(RenderArgs A) {
                 r += kept ? 1 : 0;  // may pass pass 1's count; those are not written
             });
             if (at >= 0 && at < cnt) {
-                // the sample's cell and fractions; k_render_gather adds its colour
+                // the sample's cell and fractions
                 const int64_t q = start + at;
                 if (q < F.capacity) {
                     F.rec[2 * q] = make_uint4((uint32_t)s.i0, (uint32_t)s.j0, (uint32_t)s.k0,
@@ -816,147 +688,232 @@ __global__ void __launch_bounds__(kMarchThreads) k_render_fill(RenderArgs A) {
         wave_count_add(A.counters + 1, sub == 0 ? (unsigned long long)written : 0, lane);
 }
 
-// Colour of each record (trigetColor, renderer.cu:303-310: corner 0's row
-// times its weight, then the others added in corner order, fp32), written over
-// the record's cell as 12 fp16 features: a thread per record, so the colour
-// loads run at full lane occupancy instead of inside the marches' divergent
-// loops.  Records: in (i0, j0, k0, u | v, w, weight, pixel), out (features
-// 0..7 | 8..11, weight, pixel); i0 = -1 marks a reserved record without a
-// sample (zero features).
+// The records' colour and the MLP over them: a wavefront takes 32 records
+// through the network by itself, activations in registers (the D fragment of
+// v_mfma_f32_32x32x16_f16, lane (h, n): features 32T + 8q + 4h + i of sample n, is the
+// next layer's B fragment under the K order of rperm).  The colour (trigetColor,
+// renderer.cu:303-310) is gathered ahead, four corners to a lane and the other four
+// in the lane's other half, under the MFMAs of the group before, so the features
+// never see memory.  Each record's contribution is w / (1 + exp(-raw)) per channel
+// (final_render, renderer.cu:112-119).  Records: (i0, j0, k0, u | v, w, weight,
+// pixel); i0 = -1 marks a reserved record without a sample (no contribution).
+//
+// What bounds it: the CU's address unit and L1, one row part a lane and cycle (590
+// cycles a group, 68% of the time at 800 x 800); the group's 44 MFMAs of 32 cycles
+// of its SIMD's matrix core and 440 vector instructions of 4 run beside it (44% and
+// 50%).  Three wavefronts per SIMD (fp16 payload) cover most of the loads' latency.
+//
+// Measured against a gather kernel of a thread per record, which wrote the features
+// back into the records, and an MLP kernel with four 16-sample tiles a wavefront:
+// 800 x 800, fp16 365 + 572 -> 719 us (the frame 1880 -> 1604 us); 203 x 151, fp32
+// 34 + 45 -> 62 us (352 -> 325 us).
 template <bool F32PAY>
-__global__ void __launch_bounds__(256) k_render_gather(RenderArgs A) {
+__global__ void __launch_bounds__(64 * kMlpWaves, F32PAY ? 2 : 3) k_render_mlp(RenderArgs A) {
+    constexpr int kRow = F32PAY ? 4 : 2;  // 16-byte parts of a colour row
+    __shared__ RenderSmem sm;
     const FrameBuffers& F = A.fb;
-    const unsigned long long tot = *F.total;
-    const int64_t n = (int64_t)(tot < (unsigned long long)F.capacity ? tot : F.capacity);
-    // one thread per record (the grid covers the capacity): each thread's
-    // chain of dependent loads (record, leaf table, colour rows) is short, and
-    // the waves in flight overlap them
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < n) {
-        const uint4 a = F.rec[2 * q], b = F.rec[2 * q + 1];
-        uint4 o0 = make_uint4(0u, 0u, 0u, 0u), o1 = make_uint4(0u, 0u, b.z, b.w);
-        const int i0 = (int)a.x, j0 = (int)a.y, k0 = (int)a.z;
-        if (i0 >= 0) {
-            const float u = __uint_as_float(a.w), v = __uint_as_float(b.x), w = __uint_as_float(b.y);
-            BlockCache bc;
-            int32_t slot[8];
-            corner_slots(A, i0, j0, k0, bc, slot);
-            float sc[8];
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const float wa = ((kCx >> c) & 1) ? u : 1.f - u;
-                const float wb = ((kCy >> c) & 1) ? v : 1.f - v;
-                const float we = ((kCz >> c) & 1) ? w : 1.f - w;
-                sc[c] = (wa * wb) * we;
-            }
-            float f[12], cq[12];
-            load_col<F32PAY>(A.payload, slot[0], cq);
-#pragma unroll
-            for (int ch = 0; ch < 12; ++ch) f[ch] = cq[ch] * sc[0];
-#pragma unroll
-            for (int c = 1; c < 8; ++c) {
-                load_col<F32PAY>(A.payload, slot[c], cq);
-#pragma unroll
-                for (int ch = 0; ch < 12; ++ch) f[ch] = f[ch] + cq[ch] * sc[c];
-            }
-            o0 = make_uint4(pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]),
-                            pack2(f[6], f[7]));
-            o1.x = pack2(f[8], f[9]);
-            o1.y = pack2(f[10], f[11]);
-        }
-        F.rec[2 * q] = o0;
-        F.rec[2 * q + 1] = o1;
-    }
-}
-
-// The MLP over the records, 64 per wave-chunk; each record's contribution
-// w / (1 + exp(-raw)) per channel (final_render, renderer.cu:112-119).
-__global__ void __launch_bounds__(64 * kWaves) k_render_mlp(RenderArgs A) {
-    extern __shared__ uint4 smem[];
-    uint4* sW = smem;  // weights + biases
-    float* sB = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(smem) + kPackedHalves * 2);
-    _Float16* sXall = reinterpret_cast<_Float16*>(reinterpret_cast<uint8_t*>(smem) + kPackedBytes);
-    float* sLall = reinterpret_cast<float*>(sXall + kWaves * 64 * XS);
-
-    for (int i = threadIdx.x; i < kPackedBytes / 16; i += blockDim.x) sW[i] = A.packed[i];
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    _Float16* sX = sXall + wv * 64 * XS;
-    float* sL = sLall + wv * 64 * 4;
-    uint4* row = reinterpret_cast<uint4*>(sX + lane * XS);
-    row[6] = row[7] = make_uint4(0u, 0u, 0u, 0u);  // inputs 48..63 stay zero
-    __syncthreads();
-
-    const FrameBuffers& F = A.fb;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = (int)(threadIdx.x & 63), n = lane & 31, h = lane >> 5;
     const unsigned long long tot = *F.total;
     if (A.counters && blockIdx.x == 0 && threadIdx.x == 0) A.counters[2] = tot;
-    const int64_t n = (int64_t)(tot < (unsigned long long)F.capacity ? tot : F.capacity);
-    const int64_t nchunks = (n + 63) / 64;
-    const int64_t stride = (int64_t)gridDim.x * kWaves;
-    // Two-stage prefetch: a chunk's records arrive one chunk ahead and its
-    // pixels' PE rows (which need the records) are loaded while the chunk
-    // before it runs the MLP, so neither load's latency sits in front of the
-    // MFMAs.
-    const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-    auto load_rec = [&](int64_t ch, uint4& a, uint4& b) {
-        const int64_t q = ch * 64 + lane;
-        a = b = z;
-        if (ch < nchunks && q < n) {
-            a = F.rec[2 * q];
-            b = F.rec[2 * q + 1];
+    const int64_t total = (int64_t)(tot < (unsigned long long)F.capacity ? tot : F.capacity);
+    if (total <= 0) return;
+    const int64_t ngroups = (total + 31) / 32, stride = (int64_t)gridDim.x * kMlpWaves;
+    const TopoView& topo = A.topo;
+
+    // the group two ahead: its records (the last record again past the end)
+    uint4 ra, rb;
+    auto load_records = [&](int64_t grp) {
+        const int64_t q = min(min(grp, ngroups - 1) * 32 + n, total - 1);
+        ra = F.rec[2 * q];
+        rb = F.rec[2 * q + 1];
+    };
+    // the next group: slots and weights of this lane's four corners (4h .. 4h + 3 of the
+    // corner walk: x offset h, the y and z offsets mirrored in y), weight, pixel
+    int32_t slot[4];
+    float sc[4], nweight;
+    uint32_t npix;
+    auto lookup = [&]() {
+        const int i0 = (int)ra.x, j0 = (int)ra.y, k0 = (int)ra.z;
+        const float u = __uint_as_float(ra.w), v = __uint_as_float(rb.x), w = __uint_as_float(rb.y);
+        nweight = i0 >= 0 ? __uint_as_float(rb.z) : -1.f;  // no sample's weight is negative
+        npix = rb.w;
+        const float a = h ? u : 1.f - u;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int dy = (c >> 1) ^ h, dz = (c & 1) ^ (c >> 1);
+            sc[c] = (a * (dy ? v : 1.f - v)) * (dz ? w : 1.f - w);
+            const int i = i0 + h, j = j0 + dy, k = k0 + dz;
+            int32_t leaf;
+            if (topo.two_level) {  // uniform over the frame
+                leaf = leaf_of(topo, i, j, k);
+            } else {  // leaf_of's lookup without a branch
+                const int la = (i >> 3) - topo.lo0, lb = (j >> 3) - topo.lo1, lc = (k >> 3) - topo.lo2;
+                const bool inside = (unsigned)la < (unsigned)topo.d0 && (unsigned)lb < (unsigned)topo.d1 &&
+                                    (unsigned)lc < (unsigned)topo.d2;
+                leaf = topo.table[inside ? (la * topo.d1 + lb) * topo.d2 + lc : 0];
+                leaf = inside ? leaf : -1;
+            }
+            slot[c] = leaf < 0 ? (int32_t)A.nslots : leaf * 512 + voxel_offset(i, j, k);
         }
     };
-    auto load_pe = [&](int64_t ch, const uint4& b, uint4* pe) {
-        const int64_t q = ch * 64 + lane;
-        pe[0] = pe[1] = pe[2] = pe[3] = z;
-        if (ch < nchunks && q < n) {
-            const uint4* pr = F.pe + 4 * (int64_t)b.w;
-            pe[0] = pr[0];
-            pe[1] = pr[1];
-            pe[2] = pr[2];
-            pe[3] = pr[3];
+    uint4 raw[2][kRow];  // the colour rows of corners 2 pair, 2 pair + 1
+    auto fetch = [&](int pair) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const uint4* src = reinterpret_cast<const uint4*>(A.payload) + (int64_t)slot[2 * pair + c] * kRow;
+#pragma unroll
+            for (int k = 0; k < kRow; ++k) raw[c][k] = src[k];
         }
     };
-    int64_t ch = (int64_t)blockIdx.x * kWaves + wv;
-    uint4 ca, cb, cpe[4], na, nb;
-    load_rec(ch, ca, cb);
-    load_pe(ch, cb, cpe);
-    load_rec(ch + stride, na, nb);
-    for (; ch < nchunks; ch += stride) {
-        const int64_t q = ch * 64 + lane;
-        const bool live = q < n;
-        row[0] = ca;
-        row[1] = make_uint4(cb.x, cb.y, 0u, 0u);
-        row[2] = cpe[0];
-        row[3] = cpe[1];
-        row[4] = cpe[2];
-        row[5] = cpe[3];
-        // the next chunk's PE rows and the records of the one after
-        uint4 npe[4], fa, fb;
-        load_pe(ch + stride, nb, npe);
-        load_rec(ch + 2 * stride, fa, fb);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        wave_mlp(sW, sB, sX, sL, lane);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (live) {
-            const float w = __uint_as_float(cb.z);
-            const float* lg = sL + lane * 4;
-            // w * sigmoid(raw) with the hardware exp and reciprocal (a few ulps,
-            // far inside the fp16 MLP's own rounding)
-            F.contrib[q] = make_float4(w * __builtin_amdgcn_rcpf(1.f + __expf(-lg[0])),
-                                       w * __builtin_amdgcn_rcpf(1.f + __expf(-lg[1])),
-                                       w * __builtin_amdgcn_rcpf(1.f + __expf(-lg[2])), 0.f);
+    float v[12];  // this lane's corners' weighted colour
+    auto weigh = [&](int pair) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const float s = sc[2 * pair + c];
+            const uint32_t* r = reinterpret_cast<const uint32_t*>(raw[c]);
+#pragma unroll
+            for (int ch = 0; ch < 12; ++ch) {
+                const int e = ch + 1;  // element 0 is the density
+                const float x = F32PAY ? __uint_as_float(r[e]) : h2f((uint16_t)(r[e >> 1] >> (16 * (e & 1))));
+                v[ch] = pair == 0 && c == 0 ? x * s : fmaf(x, s, v[ch]);
+            }
         }
-        __builtin_amdgcn_wave_barrier();  // sL and the rows are rewritten by the next chunk
-        ca = na;
-        cb = nb;
-        cpe[0] = npe[0];
-        cpe[1] = npe[1];
-        cpe[2] = npe[2];
-        cpe[3] = npe[3];
-        na = fa;
-        nb = fb;
+    };
+    uint4 pe2, pe4;  // the pixel's encoding: chunk 2 + h, chunk 4, and chunk 1's half
+    uint2 peb;
+    auto fetch_pe = [&]() {
+        const uint4* row = F.pe + 4 * (int64_t)npix;
+        pe2 = row[1 + h];
+        pe4 = row[3];
+        peb = reinterpret_cast<const uint2*>(row)[1];
+    };
+    uint4 xb[3];  // a group's X fragments: columns 8h, 16 + 8h, 32 + 8h
+    auto form_x = [&]() {
+        // the two lane halves' sums: half 0 is left with features 0..7, half 1 with 8..11
+        float f[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const auto r = __builtin_amdgcn_permlane32_swap(
+                __float_as_uint(v[c]), __float_as_uint(v[c < 4 ? c + 8 : c]), false, false);
+            f[c] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        }
+        xb[0] = make_uint4(pack2(f[0], f[1]), pack2(f[2], f[3]), h ? peb.x : pack2(f[4], f[5]),
+                           h ? peb.y : pack2(f[6], f[7]));
+        xb[1] = pe2;
+        xb[2] = make_uint4(h ? 0u : pe4.x, h ? 0u : pe4.y, h ? 0u : pe4.z, h ? 0u : pe4.w);
+    };
+
+    int64_t grp = (int64_t)wv * gridDim.x + blockIdx.x;
+    load_records(grp);
+    {
+        uint4* dst = reinterpret_cast<uint4*>(&sm);
+        for (int e = threadIdx.x; e < kPackedBytes / 16; e += 64 * kMlpWaves) dst[e] = A.packed[e];
+    }
+    lookup();
+    load_records(grp + stride);
+    fetch(0);
+    weigh(0);
+    fetch(1);
+    fetch_pe();
+    weigh(1);
+    form_x();
+    __syncthreads();  // the weights; from here on the wavefronts run on their own
+    const uint4* const w0p = sm.w0 + 128 * h + n;
+    const uint4* const w1p = sm.w1 + lane;
+    const uint4* const w2p = sm.w2 + 4 * h + (n & 3);
+    const float* const b1p = sm.b + 4 * h;
+    const float b2a = sm.b[128 + h], b2b = sm.b[130];
+
+    for (; grp < ngroups; grp += stride) {
+        const float weight = nweight;
+        lookup();
+        load_records(grp + 2 * stride);
+        uint32_t h0[8][4], h1[4];  // layer 1's B fragments [k-step][dword], layer 2's of one k-step
+        f32x16 c, d;               // a tile in the making, the one before
+        f32x4 lg = {0.f, 0.f, 0.f, 0.f};
+        const f32x16 zero = {};
+        auto pair0 = [&](int T, int j) {
+            h0[2 * T + (j >> 2)][j & 3] = relu_pack2(d[2 * j], d[2 * j + 1]);
+        };
+        uint4 w2f;
+        auto pair1 = [&](int T, int j) {
+            if ((j & 3) == 0) w2f = w2p[8 * (2 * T + (j >> 2))];
+            h1[j & 3] = relu_pack2(d[2 * j], d[2 * j + 1]);
+            if ((j & 3) == 3) {  // layer 2's k-step 2T + j / 4
+                lg = mfma4x4x4h(w2f.x, w2f.y, h1[0], h1[1], lg);
+                lg = mfma4x4x4h(w2f.z, w2f.w, h1[2], h1[3], lg);
+            }
+        };
+        // ---- layer 0; the next group's first corners are fetched from here on ----
+        uint4 f0[3] = {w0p[0], w0p[256]};  // weight fragments, read two steps ahead
+#pragma unroll
+        for (int T = 0; T < 4; ++T) {
+            if (T == 2) fetch(0);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const int s = 3 * T + k;
+                if (s < 10) f0[(s + 2) % 3] = w0p[256 * ((s + 2) % 3) + 32 * ((s + 2) / 3)];
+                c = mfma32x32x16h(f0[s % 3], xb[k], k == 0 ? zero : c);
+                if (T > 0) {
+                    pair0(T - 1, 3 * k);
+                    pair0(T - 1, 3 * k + 1);
+                    if (k < 2) pair0(T - 1, 3 * k + 2);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            d = c;
+        }
+        // ---- layer 1; layer 2 over its tiles ----
+        uint4 f1[3] = {w1p[0], w1p[64]};
+#pragma unroll
+        for (int T = 0; T < 4; ++T) {
+            if (T == 1) {
+                weigh(0);
+                fetch(1);
+                fetch_pe();
+            }
+            if (T == 3) weigh(1);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 b = *reinterpret_cast<const float4*>(b1p + 32 * T + 8 * q);
+                c[4 * q] = b.x;
+                c[4 * q + 1] = b.y;
+                c[4 * q + 2] = b.z;
+                c[4 * q + 3] = b.w;
+            }
+#pragma unroll
+            for (int ks = 0; ks < 8; ++ks) {
+                const int s = 8 * T + ks;
+                if (s < 30) f1[(s + 2) % 3] = w1p[64 * (s + 2)];
+                c = mfma32x32x16h(f1[s % 3], make_uint4(h0[ks][0], h0[ks][1], h0[ks][2], h0[ks][3]), c);
+                if (T > 0) {
+                    pair1(T - 1, ks);
+                } else if (ks < 4) {  // the last layer-0 tile is k-steps 6 and 7's input
+                    pair0(3, 2 * ks);
+                    pair0(3, 2 * ks + 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            d = c;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) pair1(3, j);
+        form_x();
+        // the lane halves' logits: half h finishes channel h, half 0 channel 2 too (half 1
+        // writes the unused fourth); w * sigmoid(raw) with the hardware exp and reciprocal
+        // (a few ulps, far inside the fp16 MLP's own rounding)
+        const auto r01 = __builtin_amdgcn_permlane32_swap(__float_as_uint(lg[0]),
+                                                          __float_as_uint(lg[1]), false, false);
+        const float x = __uint_as_float(r01[0]) + __uint_as_float(r01[1]) + b2a;
+        const float y = lg[2] + __shfl_xor(lg[2], 32, 64) + b2b;
+        const int64_t q = grp * 32 + n;
+        if (q < total) {
+            float* dst = reinterpret_cast<float*>(F.contrib + q) + h;
+            const bool live = weight != -1.f;
+            dst[0] = live ? weight * __builtin_amdgcn_rcpf(1.f + __expf(-x)) : 0.f;
+            dst[2] = live && h == 0 ? weight * __builtin_amdgcn_rcpf(1.f + __expf(-y)) : 0.f;
+        }
     }
 }
 
@@ -1004,9 +961,6 @@ __global__ void k_render_reset(unsigned long long* total, unsigned long long* co
     if (threadIdx.x == 0) *total = 0ull;
     if (counters && threadIdx.x < 3) counters[threadIdx.x] = 0ull;
 }
-
-constexpr size_t kRenderSmem =
-    (size_t)kPackedBytes + (size_t)kWaves * 64 * XS * 2 + (size_t)kWaves * 64 * 4 * 4;
 
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
@@ -1259,23 +1213,12 @@ int render_image(const pvdb_topology* topo, const pvdb_render_desc* d, void* ws,
         const int rc = d->payload_f32 ? launch_marches_sized<true>(A, s)
                                       : launch_marches_sized<false>(A, s);
         if (rc != PVDB_OK) return rc;
-        if (d->payload_f32)
-            hipLaunchKernelGGL(k_render_gather<true>, dim3(pvdb_blocks(A.fb.capacity, 256)),
-                               dim3(256), 0, s, A);
-        else
-            hipLaunchKernelGGL(k_render_gather<false>, dim3(pvdb_blocks(A.fb.capacity, 256)),
-                               dim3(256), 0, s, A);
-        PVDB_LAUNCHED("k_render_gather");
-    }
-    static bool smem_set = false;
-    if (!smem_set) {
-        PVDB_HIP(hipFuncSetAttribute((const void*)k_render_mlp,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRenderSmem));
-        smem_set = true;
     }
     {
         RenderStage st(1, s);
-        hipLaunchKernelGGL(k_render_mlp, dim3(ncu), dim3(64 * kWaves), kRenderSmem, s, A);
+        // two workgroups a CU, by registers; three for an fp16 payload
+        hipLaunchKernelGGL(d->payload_f32 ? k_render_mlp<true> : k_render_mlp<false>, dim3((d->payload_f32 ? 2 : 3) * ncu),
+                           dim3(64 * kMlpWaves), 0, s, A);
         PVDB_LAUNCHED("k_render_mlp");
     }
     {
