@@ -19,6 +19,8 @@
 //                  input rows, dW partials; per-record feature and sigma gradients
 //   k_scatter_agg  workgroups over 32- or 64-record chunks: corner contributions
 //                  summed per slot in an LDS hash, device atomics per distinct slot
+//   k_cell_count .. k_cell_sums  in place of k_scatter_agg for large batches: records
+//                  ordered by cell, a leaf's sums in LDS
 //   k_dw_reduce    the dW partials summed in a fixed order (+ the MLP Adam)
 //   k_sparse_adam  VDB Adam over the touched leaves (every leaf in stepmodes 0
 //                  and 2), gradients re-zeroed
@@ -228,6 +230,21 @@ struct MlpAdam {
     const float* dev_sz;
     float sz, eps, b0, b1;
 };
+
+// A large batch's record numbers by cell (fused_cells.hip): 9 x 9 x 9 cells to a
+// leaf, those whose nearest voxel can lie in it.
+constexpr int kCellSide = 9, kLeafCells = kCellSide * kCellSide * kCellSide;
+struct CellBins {
+    int32_t* count;  // [nleaf][kLeafCells] records, then their exclusive prefix in the leaf
+    int32_t* leaf;   // [nleaf + 1] where the leaf's records start in `order`
+    int4* part;      // [cell_parts()] (leaf, k, n): the k-th of n parts of a leaf's records
+    int32_t* nparts; // [1]
+    int2* at;        // [capacity] a record's cell (-1: none) and its rank there
+    int32_t* order;  // [capacity] record numbers, cell by cell
+};
+constexpr int kMinPart = 1024;  // records of a leaf below which it stays in one workgroup's hands
+// The parts of `records` records in nleaf leaves at most.
+inline int64_t cell_parts(int64_t records, int64_t nleaf) { return records / kMinPart + nleaf; }
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
 

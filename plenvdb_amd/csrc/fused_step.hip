@@ -31,6 +31,9 @@ int launch_dw_reduce(const float* part, int nparts, float* dw, const MlpAdam& ad
 int launch_scatter(int nc, const TopoView& t, const RayBuffers& R, const Records& rec,
                    int64_t capacity, const GradRows& G, uint8_t* leaf_touched, int grid_req,
                    int chunk_records, const ReduceArgs& red, hipStream_t s);
+int launch_scatter_cells(const TopoView& t, const RayBuffers& R, const Records& rec, int64_t capacity,
+                        const CellBins& B, const GradRows& G, uint8_t* leaf_touched,
+                        const ReduceArgs& red, hipStream_t s);
 }  // namespace pvdb
 
 using namespace pvdb;
@@ -41,6 +44,7 @@ constexpr int kMaxMlpGrid = 512;   // workgroups of the MLP kernels at most (dW 
 constexpr int kFwdGrid = 512;      // default forward-MLP workgroups
 constexpr int kScatterChunk = 64;  // default scatter records per chunk
 constexpr int kScatterGrid = 1024; // default scatter workgroups
+constexpr int64_t kCellMinCapacity = int64_t(12) << 20, kCellMinPerLeaf = 24 << 10;  // scatter_by_cell
 constexpr int kRayWaves = 4;       // default rays per workgroup of the wave-per-ray kernels
 // Records are indexed through int32 offsets (saturating at INT32_MAX), so a
 // capacity below that bound keeps every stored offset of a dropped record
@@ -54,10 +58,23 @@ struct Layout {
         pe, setup, zero;
     size_t xyze, ab, rgb, adj, xrow, relu, grad;
     size_t touched, dw_part, fwd, w2, w0;
+    size_t cell_count, cell_leaf, cell_part, cell_nparts, cell_at, cell_order;
     size_t bytes;
 };
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
+
+// Whether a step's scatter goes by cell (launch_scatter_cells) instead of by chunks of
+// consecutive records (launch_scatter): when the batch is large and a leaf gets many
+// of its records.  The host knows their bound, the capacity (rays through sparse
+// scenes keep a tenth of it or less).  Whole steps, us, by chunks / by cells: 8192 rays
+// in 600 leaves (capacity 3.2M) 241 / 272; 20,000 in 86 (2.6M) 166 / 205; 20,000 in 600
+// (7.7M) 471 / 487; 65,536 in 1350 (21M, 16k a leaf) 828 / 839; 65,536 in 1984 (51M, 25k)
+// 1055 / 1060; 40,000 in 600 (15M, 26k) 1401 / 1230; 65,536 in 600 (25M, 42k) 1305 / 1169;
+// 131,072 in 1984 (97M, 49k) 4250 / 3560.
+bool scatter_by_cell(int64_t records, int64_t nleaf) {
+    return nleaf > 0 && records >= kCellMinCapacity && records / nleaf >= kCellMinPerLeaf;
+}
 
 Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
     const int64_t capacity = (records + 31) & ~int64_t(31);  // whole groups of the forward MLP
@@ -94,6 +111,16 @@ Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
     L.fwd = take(2 * kFwdImage);
     L.w2 = take(2 * 128 * 32);
     L.w0 = take(2 * 16 * 128);
+    if (scatter_by_cell(records, nleaf)) {
+        L.cell_count = take(4 * (size_t)kLeafCells * nleaf);
+        L.cell_leaf = take(4 * (nleaf + 1));
+        L.cell_part = take(16 * cell_parts(capacity, nleaf));
+        L.cell_nparts = take(4);
+        L.cell_at = take(8 * capacity);
+        L.cell_order = take(4 * capacity);
+    } else {
+        L.cell_count = L.cell_leaf = L.cell_part = L.cell_nparts = L.cell_at = L.cell_order = 0;
+    }
     L.bytes = o;
     return L;
 }
@@ -678,10 +705,21 @@ int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
                            d->step_size_mlp, d->eps,   d->beta0, d->beta1};
         const ReduceArgs red{dw_part, grid_bwd, d->mlp_grad, adam, kReduceBlocks,
                              R.ray_loss, R.loss, d->n_rays};
-        if ((rc = launch_scatter(12, t, R, rec, d->capacity, grad_rows_of(d), touched,
-                                 d->launch[1] > 0 ? d->launch[1] : kScatterGrid,
-                                 d->launch[2] > 0 ? d->launch[2] : kScatterChunk, red, s)))
+        if (scatter_by_cell(d->capacity, t.nleaf)) {
+            CellBins B;
+            B.count = reinterpret_cast<int32_t*>(ws + L.cell_count);
+            B.leaf = reinterpret_cast<int32_t*>(ws + L.cell_leaf);
+            B.part = reinterpret_cast<int4*>(ws + L.cell_part);
+            B.nparts = reinterpret_cast<int32_t*>(ws + L.cell_nparts);
+            B.at = reinterpret_cast<int2*>(ws + L.cell_at);
+            B.order = reinterpret_cast<int32_t*>(ws + L.cell_order);
+            rc = launch_scatter_cells(t, R, rec, d->capacity, B, grad_rows_of(d), touched, red, s);
+            if (rc) return rc;
+        } else if ((rc = launch_scatter(12, t, R, rec, d->capacity, grad_rows_of(d), touched,
+                                        d->launch[1] > 0 ? d->launch[1] : kScatterGrid,
+                                        d->launch[2] > 0 ? d->launch[2] : kScatterChunk, red, s))) {
             return rc;
+        }
     }
     if (d->do_adam) {
         StageScope sc(8, s);
