@@ -4,7 +4,8 @@
 //   k_ray_count    wave per ray: slab test + march + occupancy -> samples per ray;
 //                  its extra workgroups pack the bf16 MLP operands and zero the
 //                  MLP gradient
-//   k_scan         exclusive scan of the counts -> record offsets, total
+//   k_scan         exclusive scan of the counts -> record offsets, total (small batches:
+//                  the forward march sums them up itself)
 //   k_ray_march    wave per ray: march again, density gather, raw2alpha, alpha cull,
 //                  transmittance product-scan with early stop, weights, weight cull;
 //                  one record per occupancy-kept sample (contiguous per ray)
@@ -104,6 +105,8 @@ struct RayBuffers {
     int32_t* count;    // occupancy-kept samples per ray
     int32_t* offset;   // exclusive prefix of count
     int32_t* total;    // [1] total records
+    int64_t* group;    // records of each workgroup's rays in the counting march, from which
+                       // the forward march forms the offsets; null: k_scan forms them
     float* t_last;     // [N]
     float4* ray_out;   // [N] rendered rgb + T_last
     float4* ray_grad;  // [N] dL/drgb (3) + dL/dT_last

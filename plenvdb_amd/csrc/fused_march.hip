@@ -172,9 +172,17 @@ __global__ void __launch_bounds__(kMaxRayWaves * 64) k_ray_count(StepParams P, T
         if (item < kPackItems) pack_mlp_item(item, pk);
         return;
     }
-    const int r = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (r >= P.n_rays) return;
+    const int wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int r = blockIdx.x * nw + wv;
     const int lane = lane_id();
+    __shared__ int wcount[kMaxRayWaves];
+    if (r >= P.n_rays) {  // uniform over the wave
+        if (R.group) {
+            if (lane == 0) wcount[wv] = 0;
+            __syncthreads();
+        }
+        return;
+    }
     // the view direction, loaded now and encoded after the march (its loads
     // then add no latency to the wave)
     float vd0 = 0.f, vd1 = 0.f, vd2 = 0.f;
@@ -203,6 +211,15 @@ __global__ void __launch_bounds__(kMaxRayWaves * 64) k_ray_count(StepParams P, T
         count += __popcll(km);
     });
     if (lane == 0) R.count[r] = count;
+    if (R.group) {
+        if (lane == 0) wcount[wv] = count;
+        __syncthreads();
+        if (threadIdx.x == 0) {  // the first ray of a workgroup exists
+            int64_t sum = 0;
+            for (int w = 0; w < nw; ++w) sum += wcount[w];
+            R.group[blockIdx.x] = sum;
+        }
+    }
     if (R.pe && lane < 28) {
         // the MLP's input columns 12..39 for this ray's samples (dvgo.py:354-358):
         // the view direction, sin then cos of it at 1, 2, 4, 8 (hardware sin/cos,
@@ -294,6 +311,50 @@ __global__ void __launch_bounds__(1024) k_scan(RayBuffers R, int n) {
     if (tid == 0) R.total[0] = (int)(carry < kSat ? carry : kSat);
 }
 
+// Sum over the wavefront of a non-negative value below 2^49: 24 bits and the rest
+// separately, on the DPP datapath.
+__device__ __forceinline__ int64_t wave_sum(int64_t x) {
+    auto total = [](int v) {
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr1, 0xf, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr2, 0xf, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr4, 0xf, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr8, 0xf, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast15, 0xa, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast31, 0xc, 0xf, false);
+        return __builtin_amdgcn_readlane(v, 63);
+    };
+    return ((int64_t)total((int)(x >> 24)) << 24) + total((int)(x & 0xffffff));
+}
+
+// The ray's record offset in place of k_scan's, by the whole workgroup: the records of
+// the workgroups before it and of its own earlier rays; stored, with the total, for
+// the later kernels.
+__device__ __forceinline__ int64_t own_offset(const RayBuffers& R, int r, int n, int64_t* wsum) {
+    const int wv = threadIdx.x >> 6, nw = blockDim.x >> 6, lane = lane_id();
+    int64_t sum = 0;
+    for (int g = threadIdx.x; g < (int)blockIdx.x; g += blockDim.x) sum += R.group[g];
+    sum = wave_sum(sum);
+    if (nw > 1) {
+        if (lane == 0) wsum[wv] = sum;
+        __syncthreads();
+        sum = 0;
+        for (int w = 0; w < nw; ++w) sum += wsum[w];
+    }
+    const int r0 = r - wv;
+    int64_t cnt = 0;
+    for (int k = r0; k <= r && r < n; ++k) {
+        sum += cnt;
+        cnt = R.count[k];
+    }
+    const int64_t kSat = 0x7fffffffll;  // as in k_scan
+    const int64_t off = sum < kSat ? sum : kSat;
+    if (lane == 0 && r < n) {
+        R.offset[r] = (int)off;
+        if (r == n - 1) R.total[0] = (int)(sum + cnt < kSat ? sum + cnt : kSat);
+    }
+    return off;
+}
+
 // Forward march: one record per occupancy-kept sample.  The sample work --
 // density gather, raw2alpha, the transmittance scan, records -- runs on 64
 // kept steps at a time, in step order, so lanes are not spent on rejected
@@ -305,7 +366,11 @@ __global__ void __launch_bounds__(kMaxRayWaves * 64) k_ray_march(StepParams P, T
                                                                  RayBuffers R, Records rec) {
     extern __shared__ int64_t queue_all[];  // 128 entries per wave (dynamic: waves x 1 KB)
     const int r = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    __shared__ int64_t wsum[kMaxRayWaves];
+    int64_t off = 0;
+    if (R.group) off = own_offset(R, r, P.n_rays, wsum);
     if (r >= P.n_rays) return;  // uniform over the wave
+    if (!R.group) off = R.offset[r];
     const int lane = lane_id();
     int64_t* queue = queue_all + 128 * (threadIdx.x >> 6);
     RaySetup s;  // the counting march's set-up (positions and step count only)
@@ -320,7 +385,6 @@ __global__ void __launch_bounds__(kMaxRayWaves * 64) k_ray_march(StepParams P, T
         s.n_steps = (int64_t)(((uint64_t)__float_as_uint(b.w) << 32) | __float_as_uint(a.w));
         s.t_min = s.t_max = 0.f;  // unused by the forward march
     }
-    const int64_t off = R.offset[r];
     const int cnt = R.count[r];  // the counting march's total bounds this ray's records
     float Tc = 1.f;  // transmittance carried from batch to batch (FP32, as the reference's T_cum)
     bool stopped = false;
@@ -719,8 +783,10 @@ int launch_ray_count(const StepParams& P, const TopoView& t, const RayBuffers& R
     const int grid = ray_blocks + (pk.prm ? (int)pvdb_blocks(kPackItems, 64 * w) : 0);
     hipLaunchKernelGGL(k_ray_count, dim3(grid), dim3(64 * w), 0, s, P, t, R, pk, ray_blocks);
     PVDB_LAUNCHED("k_ray_count");
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, R, P.n_rays);
-    PVDB_LAUNCHED("k_scan");
+    if (!R.group) {
+        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, R, P.n_rays);
+        PVDB_LAUNCHED("k_scan");
+    }
     return PVDB_OK;
 }
 
