@@ -292,6 +292,12 @@ __global__ void __launch_bounds__(256) k_zero_active(TopoView t, float* __restri
 // per (slot, V consecutive channels), so neighbouring threads read neighbouring
 // 4V-byte pieces; a thread reads its own and its neighbours' values and writes
 // only its own gradient, so no two threads touch one element.
+//
+// A workgroup lies within one leaf, so the leaf's origin and its six neighbours are
+// the same for all its threads, and a thread's eight loads are issued together
+// behind those two lookups: with lookups of its own at the leaf's faces, behind the
+// gradient's load and branches, a thread made four round trips to memory in a row.
+// 600 leaves, 12 channels and one, nothing cached: 19.6 -> 17.0 us for both grids.
 template <int V>
 __global__ void __launch_bounds__(256) k_tv_add_grad(TopoView t, const float* __restrict__ vals,
                                                      float* __restrict__ grad, int C, int rx,
@@ -304,13 +310,10 @@ __global__ void __launch_bounds__(256) k_tv_add_grad(TopoView t, const float* __
     // (a bijection; the last n % 8 blocks keep their index)
     const unsigned nblk = gridDim.x, per = nblk / 8, bid = blockIdx.x;
     const unsigned lblk = bid < 8 * per ? (bid % 8) * per + bid / 8 : bid;
-    const int64_t tid = (int64_t)lblk * blockDim.x + threadIdx.x;
-    if (tid >= t.nleaf * 512 * G) return;
-    const int64_t s = tid / G;
-    const int q = (int)(tid - s * G);
-    int x, y, z;
-    slot_coord(t, s, x, y, z);
-    if (x < 0 || y < 0 || z < 0 || x >= rx || y >= ry || z >= rz) return;
+    const int64_t leaf = lblk / (2u * G);  // 512 G threads a leaf
+    const unsigned in_leaf = (lblk - (unsigned)leaf * (2u * G)) * 256u + threadIdx.x;
+    const int off = (int)(in_leaf / G), q = (int)(in_leaf - (unsigned)off * G);
+    const int64_t s = leaf * 512 + off;
     using Vec = std::conditional_t<V == 4, float4, float>;
     auto ld = [&](const float* p, float* o) {
         const Vec w = *reinterpret_cast<const Vec*>(p);
@@ -321,40 +324,45 @@ __global__ void __launch_bounds__(256) k_tv_add_grad(TopoView t, const float* __
         }
     };
     const int64_t e = s * C + (int64_t)q * V;
-    float g0[V];
+    float g0[V], v[V];
     ld(grad + e, g0);
-    bool any = dense_mode != 0;
-#pragma unroll
-    for (int c = 0; c < V; ++c) any = any || g0[c] != 0.f;
-    if (!any) return;
-    // neighbour slots: -2 past the box (no term), -1 in a missing leaf (value 0);
-    // inside this leaf the neighbour is slot +-1, +-8, +-64 (offset x<<6|y<<3|z),
-    // only a leaf face goes through the leaf table
-    const int lx = x & 7, ly = y & 7, lz = z & 7;
-    int64_t nb[6];
-    nb[0] = z > 0 ? (lz != 0 ? s - 1 : pvdb::slot_of(t, x, y, z - 1)) : -2;
-    nb[1] = z < rz - 1 ? (lz != 7 ? s + 1 : pvdb::slot_of(t, x, y, z + 1)) : -2;
-    nb[2] = y > 0 ? (ly != 0 ? s - 8 : pvdb::slot_of(t, x, y - 1, z)) : -2;
-    nb[3] = y < ry - 1 ? (ly != 7 ? s + 8 : pvdb::slot_of(t, x, y + 1, z)) : -2;
-    nb[4] = x > 0 ? (lx != 0 ? s - 64 : pvdb::slot_of(t, x - 1, y, z)) : -2;
-    nb[5] = x < rx - 1 ? (lx != 7 ? s + 64 : pvdb::slot_of(t, x + 1, y, z)) : -2;
-    const float w[6] = {wz6, wz6, wy6, wy6, wz6, wz6};
-    float v[V], acc[V];
     ld(vals + e, v);
+    const int ox = t.origins[3 * leaf], oy = t.origins[3 * leaf + 1], oz = t.origins[3 * leaf + 2];
+    const int32_t nl[6] = {pvdb::leaf_of(t, ox, oy, oz - 1), pvdb::leaf_of(t, ox, oy, oz + 8),
+                           pvdb::leaf_of(t, ox, oy - 1, oz), pvdb::leaf_of(t, ox, oy + 8, oz),
+                           pvdb::leaf_of(t, ox - 1, oy, oz), pvdb::leaf_of(t, ox + 8, oy, oz)};
+    const int lx = off >> 6, ly = (off >> 3) & 7, lz = off & 7;
+    const int x = ox + lx, y = oy + ly, z = oz + lz;
+    if (x < 0 || y < 0 || z < 0 || x >= rx || y >= ry || z >= rz) return;
+    if (!dense_mode) {
+        bool any = false;
+#pragma unroll
+        for (int c = 0; c < V; ++c) any = any || g0[c] != 0.f;
+        if (!any) return;
+    }
+    // per direction: whether the neighbour lies in the box, on this leaf's far side, and
+    // its offset from here in its leaf
+    const bool in[6] = {z > 0, z < rz - 1, y > 0, y < ry - 1, x > 0, x < rx - 1};
+    const bool out[6] = {lz == 0, lz == 7, ly == 0, ly == 7, lx == 0, lx == 7};
+    const int step[3] = {1, 8, 64};
+    const float w[6] = {wz6, wz6, wy6, wy6, wz6, wz6};
+    float u[6][V], acc[V];
+#pragma unroll
+    for (int n = 0; n < 6; ++n) {  // a missing leaf's value is 0; this slot's stands in for the load
+        const int d = step[n >> 1], sign = n & 1 ? 1 : -1;
+        const int64_t at = !out[n] ? s + sign * d : nl[n] >= 0 ? (int64_t)nl[n] * 512 + off - sign * 7 * d : s;
+        ld(vals + at * C + (int64_t)q * V, u[n]);
+    }
 #pragma unroll
     for (int c = 0; c < V; ++c) acc[c] = 0.f;
 #pragma unroll
     for (int n = 0; n < 6; ++n) {
-        if (nb[n] == -2) continue;
-        float u[V];
-        if (nb[n] >= 0) {
-            ld(vals + nb[n] * C + (int64_t)q * V, u);
-        } else {
+        const bool missing = out[n] && nl[n] < 0;
 #pragma unroll
-            for (int c = 0; c < V; ++c) u[c] = 0.f;
+        for (int c = 0; c < V; ++c) {
+            const float term = w[n] * fminf(fmaxf(v[c] - (missing ? 0.f : u[n][c]), -1.f), 1.f);
+            acc[c] = in[n] ? acc[c] + term : acc[c];
         }
-#pragma unroll
-        for (int c = 0; c < V; ++c) acc[c] += w[n] * fminf(fmaxf(v[c] - u[c], -1.f), 1.f);
     }
     float r[V];
 #pragma unroll
