@@ -402,8 +402,7 @@ __global__ void __launch_bounds__(kMaxRayWaves * 64) k_ray_march(StepParams P, T
             y = ((py - P.mn[1]) / P.len[1]) * P.rm1[1];
             z = ((pz - P.mn[2]) / P.len[2]) * P.rm1[2];
             const Cell cell = make_cell(x, y, z);
-            LeafCache cache;
-            const float sigma = gather_density(t, density, cell, cache);
+            const float sigma = gather_density(t, density, cell);
             e = expf(sigma + P.act_shift);
             alpha = 1.f - powf(1.f + e, -P.interval);
         }
@@ -653,10 +652,9 @@ __global__ void __launch_bounds__(kMaxRayWaves * 64) k_direct_composite(StepPara
         for (int c = 0; c < NC; ++c) v[c] = 0.f;
         if (bits & kAliveW) {
             const float4 p = rec.xyze[q];
-            LeafCache cache;
             float rgb[NC + 1];
             float k0[NC];
-            gather_color<NC>(topo, color, make_cell(p.x, p.y, p.z), cache, k0);
+            gather_color<NC>(topo, color, make_cell(p.x, p.y, p.z), k0);
 #pragma unroll
             for (int c = 0; c < NC; ++c) rgb[c] = 1.f / (1.f + expf(-k0[c]));
             rgb[NC] = 0.f;

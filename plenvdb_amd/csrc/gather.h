@@ -46,19 +46,70 @@ struct LeafCache {
 };
 
 
-// Density at an index-space point, density rule of densityvdb.cu:115-122.
+// leaf_of with a selected index instead of a branch around the load, for a table
+// that exists (uniform: the one-level layout of a topology with leaves).
+__device__ __forceinline__ bool one_level(const TopoView& t) { return !t.two_level && t.nleaf > 0; }
+__device__ __forceinline__ int32_t leaf_at(const TopoView& t, int i, int j, int k) {
+    const int a = (i >> 3) - t.lo0, b = (j >> 3) - t.lo1, c = (k >> 3) - t.lo2;
+    const bool in = (unsigned)a < (unsigned)t.d0 && (unsigned)b < (unsigned)t.d1 &&
+                    (unsigned)c < (unsigned)t.d2;
+    const int32_t l = t.table[in ? ((int64_t)a * t.d1 + b) * t.d2 + c : 0];
+    return in ? l : -1;
+}
+
+// Slots (-1: no leaf) of the cell's corners, in corner order.  The eight lookups do
+// not depend on one another, so a sample waits for the leaf table once, and for its
+// values once: with a leaf cache walked corner by corner each value was waited for
+// before the next corner's lookup.  The forward march of 8192 rays 19.6 -> 15.2 us, of 1021
+// 13.5 -> 10.2; k_direct_composite (3 channels, 8192 rays) 21.4 -> 17.0; the point
+// gather of 1.2M densities 14.6 -> 11.3, of 200k 12-channel rows 12.0 -> 9.3.
+__device__ __forceinline__ void corner_slots(const TopoView& t, const Cell& cell, int64_t (&s)[8]) {
+    if (one_level(t)) {  // uniform
+        int32_t l[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            l[q] = leaf_at(t, cell.i0 + ((kCx >> q) & 1), cell.j0 + ((kCy >> q) & 1),
+                           cell.k0 + ((kCz >> q) & 1));
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            s[q] = l[q] < 0 ? int64_t(-1)
+                            : (int64_t)l[q] * 512 + voxel_offset(cell.i0 + ((kCx >> q) & 1),
+                                                                 cell.j0 + ((kCy >> q) & 1),
+                                                                 cell.k0 + ((kCz >> q) & 1));
+        return;
+    }
+    LeafCache cache;
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+        s[q] = cache.slot(t, cell.i0 + ((kCx >> q) & 1), cell.j0 + ((kCy >> q) & 1),
+                          cell.k0 + ((kCz >> q) & 1));
+}
+
+// The cell's fractions towards corner q.
+__device__ __forceinline__ void corner_fracs(const Cell& cell, int q, float& a, float& b, float& d) {
+    a = ((kCx >> q) & 1) ? cell.u : 1.f - cell.u;
+    b = ((kCy >> q) & 1) ? cell.v : 1.f - cell.v;
+    d = ((kCz >> q) & 1) ? cell.w : 1.f - cell.w;
+}
+
+// Density at an index-space point, density rule of densityvdb.cu:115-122.  With NO
+// slot, slot 0's value is loaded in its place (a topology without leaves has none).
 __device__ __forceinline__ float gather_density(const TopoView& t, const float* __restrict__ vals,
-                                                const Cell& cell, LeafCache& cache) {
-    float acc = 0.f;
+                                                const Cell& cell) {
+    int64_t s[8];
+    corner_slots(t, cell, s);
+    float v[8], acc = 0.f;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = 0.f;
+    if (t.nleaf > 0) {  // uniform
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = vals[s[q] >= 0 ? s[q] : 0];
+    }
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-        const int dx = (kCx >> q) & 1, dy = (kCy >> q) & 1, dz = (kCz >> q) & 1;
-        const float a = dx ? cell.u : 1.f - cell.u;
-        const float b = dy ? cell.v : 1.f - cell.v;
-        const float d = dz ? cell.w : 1.f - cell.w;
-        const int64_t s = cache.slot(t, cell.i0 + dx, cell.j0 + dy, cell.k0 + dz);
-        const float val = s >= 0 ? vals[s] : 0.f;
-        acc = acc + ((val * a) * b) * d;
+        float a, b, d;
+        corner_fracs(cell, q, a, b, d);
+        acc = acc + (((s[q] >= 0 ? v[q] : 0.f) * a) * b) * d;
     }
     return acc;
 }
@@ -66,38 +117,47 @@ __device__ __forceinline__ float gather_density(const TopoView& t, const float* 
 // NC colour channels at an index-space point, colour rule of
 // colorvdb.cu:16-26,96-103: the corner weight (a*b)*c first, then
 // out[c] += val[c] * weight, corners in the order above (a missing leaf adds 0).
-template <int NC>
+// kWide: rows are 16-byte aligned (NC a multiple of 4).  At most four corners' rows of
+// twelve channels are in registers at a time.
+template <int NC, bool kWide = NC % 4 == 0>
 __device__ __forceinline__ void gather_color(const TopoView& t, const float* __restrict__ vals,
-                                             const Cell& cell, LeafCache& cache,
-                                             float (&out)[NC]) {
+                                             const Cell& cell, float (&out)[NC]) {
+    constexpr int kAtOnce = NC > 4 ? 4 : 8;
+    int64_t s[8];
+    corner_slots(t, cell, s);
 #pragma unroll
     for (int c = 0; c < NC; ++c) out[c] = 0.f;
+    const bool some = t.nleaf > 0;  // uniform; without leaves there are no values to load
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        const int dx = (kCx >> q) & 1, dy = (kCy >> q) & 1, dz = (kCz >> q) & 1;
-        const float a = dx ? cell.u : 1.f - cell.u;
-        const float b = dy ? cell.v : 1.f - cell.v;
-        const float d = dz ? cell.w : 1.f - cell.w;
-        const float sc = (a * b) * d;
-        const int64_t s = cache.slot(t, cell.i0 + dx, cell.j0 + dy, cell.k0 + dz);
-        float v[NC];
-        if constexpr (NC % 4 == 0) {  // 16-byte rows
-            const float4* src = reinterpret_cast<const float4*>(vals) + (s >= 0 ? s : 0) * (NC / 4);
+    for (int q0 = 0; q0 < 8; q0 += kAtOnce) {
+        float v[kAtOnce][NC];
 #pragma unroll
-            for (int k = 0; k < NC / 4; ++k) {
-                const float4 r = s >= 0 ? src[k] : make_float4(0.f, 0.f, 0.f, 0.f);
-                v[4 * k] = r.x;
-                v[4 * k + 1] = r.y;
-                v[4 * k + 2] = r.z;
-                v[4 * k + 3] = r.w;
+        for (int k = 0; k < kAtOnce; ++k) {
+            const float* src = vals + (s[q0 + k] >= 0 ? s[q0 + k] : 0) * NC;
+            if (!some) continue;
+            if constexpr (kWide) {
+#pragma unroll
+                for (int e = 0; e < NC / 4; ++e) {
+                    const float4 r = reinterpret_cast<const float4*>(src)[e];
+                    v[k][4 * e] = r.x;
+                    v[k][4 * e + 1] = r.y;
+                    v[k][4 * e + 2] = r.z;
+                    v[k][4 * e + 3] = r.w;
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < NC; ++c) v[k][c] = src[c];
             }
-        } else {
-            const float* src = vals + (s >= 0 ? s : 0) * NC;
-#pragma unroll
-            for (int c = 0; c < NC; ++c) v[c] = s >= 0 ? src[c] : 0.f;
         }
 #pragma unroll
-        for (int c = 0; c < NC; ++c) out[c] = out[c] + v[c] * sc;
+        for (int k = 0; k < kAtOnce; ++k) {
+            float a, b, d;
+            corner_fracs(cell, q0 + k, a, b, d);
+            const float sc = (a * b) * d;
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                out[c] = out[c] + (some && s[q0 + k] >= 0 ? v[k][c] : 0.f) * sc;
+        }
     }
 }
 

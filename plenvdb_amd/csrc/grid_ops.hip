@@ -32,11 +32,24 @@ __global__ void __launch_bounds__(256) k_tri_fwd(TopoView t, const float* __rest
                                                  int cdyn, const float* __restrict__ xs,
                                                  const float* __restrict__ ys,
                                                  const float* __restrict__ zs, int64_t n,
-                                                 float* __restrict__ out) {
+                                                 float* __restrict__ out, int wide) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     const int CC = C > 0 ? C : cdyn;
     const Cell cell = make_cell(xs[p], ys[p], zs[p]);
+    if constexpr (ORDER == 0) {
+        out[p] = pvdb::gather_density(t, vals, cell);
+        return;
+    } else if constexpr (C > 0) {
+        float o[C];
+        if (C % 4 == 0 && wide)  // uniform
+            pvdb::gather_color<C>(t, vals, cell, o);
+        else
+            pvdb::gather_color<C, false>(t, vals, cell, o);
+#pragma unroll
+        for (int c = 0; c < C; ++c) out[p * C + c] = o[c];
+        return;
+    }
     LeafCache cache;
     float acc[C > 0 ? C : 48];
 #pragma unroll
@@ -460,7 +473,7 @@ template <int C, int ORDER>
 void launch_fwd(const TopoView& t, const float* vals, int cdyn, const float* xs, const float* ys,
                 const float* zs, int64_t n, float* out, hipStream_t s) {
     hipLaunchKernelGGL((k_tri_fwd<C, ORDER>), dim3(pvdb_blocks(n, 256)), dim3(256), 0, s, t, vals,
-                       cdyn, xs, ys, zs, n, out);
+                       cdyn, xs, ys, zs, n, out, reinterpret_cast<uintptr_t>(vals) % 16 == 0);
 }
 template <int C, int ORDER>
 void launch_bwd(const TopoView& t, float* grad, int cdyn, const float* xs, const float* ys,
