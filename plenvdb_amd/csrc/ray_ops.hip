@@ -136,6 +136,11 @@ __global__ void k_raw2alpha_bwd(const float* __restrict__ e, const float* __rest
     gs[p] = (float)(m * (double)pw * (double)interval * (double)ga[p]);
 }
 
+// lane k's value (k uniform over the wavefront)
+__device__ __forceinline__ float lane_value(float x, int k) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), k));
+}
+
 // __set_i_for_segment_start_end (render_utils_kernel.cu:625-634) plus the
 // i_end of the last ray.
 __global__ void k_segment_bounds(const int64_t* __restrict__ ray_id, int64_t n,
@@ -150,43 +155,79 @@ __global__ void k_segment_bounds(const int64_t* __restrict__ ray_id, int64_t n,
 }
 
 // alpha2weight (render_utils_kernel.cu:576-603): float T_cum times the double
-// (1. - alpha), stop after the first T < 1e-3.
-__global__ void k_alpha2weight(const float* __restrict__ alpha, int64_t n_rays,
-                               float* __restrict__ w, float* __restrict__ T,
-                               float* __restrict__ t_last, const int64_t* __restrict__ i_start,
-                               int64_t* __restrict__ i_end) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_rays) return;
+// (1. - alpha), stop after the first T < 1e-3.  A wavefront per ray: its lanes load
+// and store 64 samples together, and all of them run the running product (the
+// same operations, sample by sample) on values read from a lane, so the chain waits
+// for arithmetic only; a thread per ray waited for memory at each of its samples, on
+// a fraction of the chip.  8191 rays, 200k samples: 38.0 -> 21.0 us.
+__global__ void __launch_bounds__(256) k_alpha2weight(const float* __restrict__ alpha,
+                                                      int64_t n_rays, float* __restrict__ w,
+                                                      float* __restrict__ T,
+                                                      float* __restrict__ t_last,
+                                                      const int64_t* __restrict__ i_start,
+                                                      int64_t* __restrict__ i_end) {
+    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= n_rays) return;  // uniform over the wave
+    const int lane = (int)(threadIdx.x & 63);
     const int64_t is = i_start[r], ie = i_end[r];
     float Tc = 1.f;
-    int64_t i;
-    for (i = is; i < ie; ++i) {
-        T[i] = Tc;
-        w[i] = Tc * alpha[i];
-        Tc = (float)((double)Tc * (1.0 - (double)alpha[i]));
-        if ((double)Tc < 1e-3) {
-            i += 1;
-            break;
+    int64_t end = is > ie ? is : ie;  // an empty ray's end is its start
+    for (int64_t base = is; base < end; base += 64) {
+        const int m = (int)(end - base < 64 ? end - base : 64);
+        const float a = lane < m ? alpha[base + lane] : 0.f;
+        float mine = 0.f;
+        int done = m;
+        for (int k = 0; k < m; ++k) {
+            mine = lane == k ? Tc : mine;
+            Tc = (float)((double)Tc * (1.0 - (double)lane_value(a, k)));
+            if ((double)Tc < 1e-3) {
+                done = k + 1;
+                break;
+            }
         }
+        if (lane < done) {
+            T[base + lane] = mine;
+            w[base + lane] = mine * a;
+        }
+        if ((double)Tc < 1e-3) end = base + done;
     }
-    i_end[r] = i;
-    t_last[r] = Tc;
+    if (lane == 0) {
+        i_end[r] = end;
+        t_last[r] = Tc;
+    }
 }
 
-// alpha2weight backward (render_utils_kernel.cu:653-676).
-__global__ void k_alpha2weight_bwd(const float* __restrict__ alpha, const float* __restrict__ w,
-                                   const float* __restrict__ T, const float* __restrict__ t_last,
-                                   const int64_t* __restrict__ i_start,
-                                   const int64_t* __restrict__ i_end, int64_t n_rays,
-                                   const float* __restrict__ gw, const float* __restrict__ glast,
-                                   float* __restrict__ ga) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_rays) return;
+// alpha2weight backward (render_utils_kernel.cu:653-676), a wavefront per ray as above:
+// the running sum sample by sample, each sample's gradient in its own lane.
+// 4096 rays, 100k samples: 61.8 -> 12.7 us.
+__global__ void __launch_bounds__(256) k_alpha2weight_bwd(
+    const float* __restrict__ alpha, const float* __restrict__ w, const float* __restrict__ T,
+    const float* __restrict__ t_last, const int64_t* __restrict__ i_start,
+    const int64_t* __restrict__ i_end, int64_t n_rays, const float* __restrict__ gw,
+    const float* __restrict__ glast, float* __restrict__ ga) {
+    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= n_rays) return;  // uniform over the wave
+    const int lane = (int)(threadIdx.x & 63);
+    const int64_t is = i_start[r];
     float back = glast[r] * t_last[r];
-    for (int64_t i = i_end[r] - 1; i >= i_start[r]; --i) {
-        const double den = (double)(1.f - alpha[i]) + 1e-10;
-        ga[i] = (float)((double)(gw[i] * T[i]) - (double)back / den);
-        back += gw[i] * w[i];
+    for (int64_t top = i_end[r]; top > is; top -= 64) {  // the samples top - 1, top - 2, ...
+        const int m = (int)(top - is < 64 ? top - is : 64);
+        const int64_t i = top - 1 - lane;
+        float g = 0.f, a = 0.f, t = 0.f, part = 0.f, mine = 0.f;
+        if (lane < m) {
+            g = gw[i];
+            a = alpha[i];
+            t = T[i];
+            part = g * w[i];
+        }
+        for (int k = 0; k < m; ++k) {
+            mine = lane == k ? back : mine;
+            back += lane_value(part, k);
+        }
+        if (lane < m) {
+            const double den = (double)(1.f - a) + 1e-10;
+            ga[i] = (float)((double)(g * t) - (double)mine / den);
+        }
     }
 }
 
@@ -419,7 +460,7 @@ int pvdb_alpha2weight(const float* alpha, int64_t n_rays, float* weight, float* 
     PVDB_CHECK_ARG(n_rays >= 0, "n_rays must be >= 0");
     if (n_rays == 0) return PVDB_OK;
     PVDB_CHECK_ARG(alpha && weight && T && alphainv_last && i_start && i_end, "null pointer");
-    hipLaunchKernelGGL(k_alpha2weight, dim3(pvdb_blocks(n_rays, 256)), dim3(256), 0,
+    hipLaunchKernelGGL(k_alpha2weight, dim3(pvdb_blocks(n_rays, 4)), dim3(256), 0,
                        (hipStream_t)stream, alpha, n_rays, weight, T, alphainv_last, i_start,
                        i_end);
     PVDB_LAUNCHED("k_alpha2weight");
@@ -435,7 +476,7 @@ int pvdb_alpha2weight_bwd(const float* alpha, const float* weight, const float* 
     PVDB_CHECK_ARG(alpha && weight && T && alphainv_last && i_start && i_end && grad_weights &&
                        grad_last && grad_alpha,
                    "null pointer");
-    hipLaunchKernelGGL(k_alpha2weight_bwd, dim3(pvdb_blocks(n_rays, 256)), dim3(256), 0,
+    hipLaunchKernelGGL(k_alpha2weight_bwd, dim3(pvdb_blocks(n_rays, 4)), dim3(256), 0,
                        (hipStream_t)stream, alpha, weight, T, alphainv_last, i_start, i_end,
                        n_rays, grad_weights, grad_last, grad_alpha);
     PVDB_LAUNCHED("k_alpha2weight_bwd");
