@@ -344,13 +344,13 @@ int pvdb_fused_records(const pvdb_topology* topo, const pvdb_step_desc* desc, vo
 
 /* ---- merged-VDB renderer ----------------------------------------------------
  * MGRenderer (plenvdb/lib/vdb/plenvdb.h:933-1068, plenvdb.cpp:135-171;
- * render_an_image_cuda renderer.cu:370-424) as three kernels on `stream`,
- * with no host synchronisation and no allocation: a march kernel runs both of
- * the reference's marches per pixel (first_look_merged's count and t_min /
- * t_max rewrite, then ray_marching_merged from the rewritten t_min, each with
- * its own summation order, renderer.cu:222-367) and writes one record per
- * kept sample; an MLP kernel evaluates the RGB MLP on fp16 MFMA over the
- * records; a composite kernel adds each pixel's contributions to T * bg in
+ * render_an_image_cuda renderer.cu:370-424) as four kernels on `stream`,
+ * with no host synchronisation and no allocation: two march kernels run the
+ * reference's marches per pixel (first_look_merged's count and t_min / t_max
+ * rewrite, then ray_marching_merged from the rewritten t_min, each with
+ * its own summation order, renderer.cu:222-367), the second writing one record per
+ * kept sample; an MLP kernel gathers the records' colour and evaluates the RGB MLP
+ * on fp16 MFMA; a composite kernel adds each pixel's contributions to T * bg in
  * sample order.  The merged index grid (vdb_compression.py:19-59) is a
  * topology whose active voxels are the non-zero indices plus `slot_idx` (the
  * index of every slot, 0 when inactive).  Differences from the reference: the
