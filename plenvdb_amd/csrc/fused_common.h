@@ -93,9 +93,9 @@ struct Records {
     uint4* xrow;       // [5 per record] the backward's MLP input row, X columns 0..39 as bf16
                        // hi parts: the 12 gathered colour features, the 27 view-direction
                        // encoding inputs and the bias input (a zero row unless weight-kept)
-    uint32_t* relu;    // [8 per record] forward ReLU masks: word 4l + g = layer l's
-                       // hidden features 16m + 4g + i (m < 8, i < 4; g < 4) at
-                       // bit 16 (i % 2) + 2m + i / 2
+    uint32_t* relu;    // [8 per record] forward ReLU masks: word 4l + 2h + T / 2 = the rows of
+                       // tile T of layer l that lane half h holds (rows 8q + 4h + i: features
+                       // mlp_feature(l, row)) at bit 16 (i % 2) + 8 (T % 2) + 2q + i / 2
     float4* grad;      // [4 per record] dL/dfeature (12) and dL/dsigma; in the direct-colour
                        // configurations rgb (NC) between the composite's two passes, then
                        // dL/dk0 (NC) and dL/dsigma at float kSigmaAt<NC>
@@ -133,11 +133,12 @@ constexpr int kStepCache = 256;
 // Packed bf16 MLP weights for MFMA (row-major, zero padded):
 //   w2  [128][32]  W2 (cols 0..2 used)         w0  [16][128]  W0 rows 0..15 (0..11 used)
 // fwd: the forward's weights and bias splits as its LDS image (kFwdImage),
-// and fp32 biases b1[128], b2[3].
+// and fp32 biases b0[128], b1[128], b2[3].
 struct MlpPacked {
     const uint4* fwd;
     const uint16_t* w2;
     const uint16_t* w0;
+    const float* b0;
     const float* b1;
     const float* b2;
 };
@@ -166,17 +167,27 @@ struct PackArgs {
     uint32_t* zero;  // [64] RayBuffers::zero
 };
 
+// The hidden feature at row r < 32 of a tile of layer l.  A lane half h of a
+// 32x32 product's D fragment holds rows 8q + 4h + i (q, i < 4); with the rows in
+// these orders its values are, in order, whole groups of eight consecutive
+// features of the next product's K: in layer 0 the groups 2t + h, t < 2
+// (32x32x16's order), in layer 1 the groups 2h + t.
+__host__ __device__ constexpr int mlp_feature(int l, int r) {
+    return l == 0 ? (r & 19) | ((r & 4) << 1) | ((r & 8) >> 1)
+                  : (r & 3) | ((r >> 3) << 2) | ((r & 4) << 2);
+}
+
 // The forward MLP's LDS image, in bf16 values (what each part holds stands at
 // SmemFwd):
-//   [6][128][8]    W0^T columns by chunk, b0's split
-//   [4][9][64][8]  per row tile b1's split, then W1^T's eight k-steps, K permuted
-//   [8][2][4][8]   W2^T rows, K permuted
-//   [2][8]         the biases' inputs
+//   [6][128][8]    W0^T columns by chunk, b0's split; rows in layer 0's order
+//   [4][9][64][8]  per row tile b1's split, then W1^T's eight k-steps; rows in layer 1's order
+//   [4][4][4][8]   W2^T rows
+//   [8]            the biases' inputs
 // Packed once a step, so that every workgroup's copy is contiguous: reading the
 // fragments out of the row-major weights, 64 lines an instruction, took a small
 // step longer than its arithmetic.
-constexpr int kImgW1 = 6 * 128 * 8, kImgW2 = kImgW1 + 4 * 9 * 64 * 8, kImgOnes = kImgW2 + 8 * 2 * 4 * 8,
-              kFwdImage = kImgOnes + 2 * 8;
+constexpr int kImgW1 = 6 * 128 * 8, kImgW2 = kImgW1 + 4 * 9 * 64 * 8, kImgOnes = kImgW2 + 4 * 4 * 4 * 8,
+              kFwdImage = kImgOnes + 8;
 constexpr int kPackItems = kMlpParams > kFwdImage ? kMlpParams : kFwdImage;
 
 __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l);
@@ -192,22 +203,21 @@ __device__ __forceinline__ uint16_t bias_part(float b, int j) {
 
 __device__ __forceinline__ uint16_t fwd_image_item(int t, const float* prm) {
     const int j = t & 7;
-    // the hidden feature at position 8h + j of k-step ks
-    auto feature = [j](int ks, int h) { return 16 * ks + 8 * (j >> 2) + 4 * h + (j & 3); };
     if (t < kImgW1) {
-        const int chunk = t >> 10, o = (t >> 3) & 127, i = 8 * chunk + j;
+        const int chunk = t >> 10, row = (t >> 3) & 127, i = 8 * chunk + j;
+        const int o = (row & ~31) + mlp_feature(0, row & 31);
         if (chunk == 5) return bias_part(prm[kB0 + o], j);
         return i < 39 ? f2bf_bits(prm[kW0 + i * 128 + o]) : (uint16_t)0;
     }
     if (t < kImgW2) {
         const int q = t - kImgW1, T = q / (9 * 512), step = (q >> 9) % 9, lane = (q >> 3) & 63;
-        const int h = lane >> 5, o = 32 * T + (lane & 31);
+        const int h = lane >> 5, o = 32 * T + mlp_feature(1, lane & 31);
         if (step == 0) return h == 0 ? bias_part(prm[kB1 + o], j) : (uint16_t)0;
-        return f2bf_bits(prm[kW1 + feature(step - 1, h) * 128 + o]);
+        return f2bf_bits(prm[kW1 + (16 * (step - 1) + 8 * h + j) * 128 + o]);
     }
     if (t < kImgOnes) {
-        const int q = t - kImgW2, ks = q >> 6, h = (q >> 5) & 1, o = (q >> 3) & 3;
-        return o < 3 ? f2bf_bits(prm[kW2 + feature(ks, h) * 3 + o]) : (uint16_t)0;
+        const int q = t - kImgW2, group = q >> 5, o = (q >> 3) & 3;
+        return o < 3 ? f2bf_bits(prm[kW2 + (8 * group + j) * 3 + o]) : (uint16_t)0;
     }
     return t - kImgOnes < 3 ? (uint16_t)0x3f80 : (uint16_t)0;  // 1, 1, 1, 0 ..
 }

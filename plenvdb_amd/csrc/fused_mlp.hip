@@ -15,6 +15,14 @@
 // sample's feature gradient by a whole term.  dW products (activation x
 // gradient) take the hi parts only.
 //
+// The order of every sum but dW's, which run over samples, is part of the results: the
+// bias, then for every 32 inputs the products with their hi, mid and lo parts, eight
+// inputs at a time (an MFMA's sum over K is eight terms at a time into the accumulator,
+// each eight in no order, so two 32x32x16 are one 16x16x32, bit for bit).  In another
+// order about two pre-activations of 190k records end on the other side of zero,
+// and colour moments move by up to 1.4e-3 of the largest.  tests/test_gpu_mlp_order.py
+// holds the order.
+//
 // k_mlp_fwd gathers the colour features and writes each record's rgb, ReLU masks
 // and bf16 input row (so the backward reads 80 bytes per record instead of
 // redoing 8 gathers).  k_mlp_bwd takes each sample's dL/dlogit and dL/dsigma from
@@ -49,24 +57,20 @@ __device__ __forceinline__ bf16x8 as_bf8(const uint4& v) { return __builtin_bit_
 // A wavefront takes a group of 32 records through the whole network by itself:
 // its activations never leave its registers, so there is no barrier and no
 // exchange between wavefronts once the weights are in LDS.  The D fragment of
-// v_mfma_f32_32x32x16_bf16 (lane (h, n), h = lane / 32: features
-// 32T + 8q + 4h + i of sample n, q, i < 4) is the next layer's B fragment when
-// that layer's weights are stored with their K index permuted to match:
-// position 8h + j of k-step 2T + t stands for feature
-// 32T + 16t + 8 (j / 4) + 4h + j % 4.  A weight fragment read from LDS (8 LDS
-// cycles) covers the three parts of the split activations: 96 cycles of its
-// SIMD's matrix core.  X and H0 enter their products as (hi, mid, lo) triples,
+// v_mfma_f32_32x32x16_bf16 (lane (h, n), h = lane / 32: rows 8q + 4h + i of
+// sample n, q, i < 4) is the next layer's B fragment, K in its natural order, when
+// the features stand in layer 0's row order (mlp_feature).  A weight fragment read
+// from LDS (8 LDS cycles) covers the three parts of the split activations: 96 cycles
+// of its SIMD's matrix core.  X and H0 enter their products as (hi, mid, lo) triples,
 // so the pre-activations, and with them the ReLU masks the backward applies,
 // carry fp32 precision; H1 enters the logits as (hi, lo) pairs.
 //
 // X has 40 columns (12 features, 27 encoding inputs, the bias input) in three
-// parts.  Stacked along K they are 15 chunks of 8 columns, two to a k-step, in
-// the order
-//   hi A, hi B | mid A, mid B | lo A, lo B | hi 2, hi 3 | hi 4, mid 2 |
-//   mid 3, mid 4 | lo 2, lo 3 | lo 4, ones
-// where chunk A is features 0..7, B features 8..11 and columns 12..15, and
-// 2..4 columns 8c..8c + 7; they sit in a tile of the wavefront's own in LDS.
-// The ones meet b0's own split, so the accumulators start at zero.
+// parts.  Stacked along K, behind the ones that meet b0's own split, they are 16 chunks
+// of 8 columns, two to a k-step, in the order
+//   ones, hi 0 | hi 1, 2 | hi 3, mid 0 | mid 1, 2 | mid 3, lo 0 | lo 1, 2 | lo 3, hi 4 |
+//   mid 4, lo 4
+// and sit in a tile of the wavefront's own in LDS.
 //
 // The last group's rows past the records are stored like the others (the
 // workspace holds whole groups) and never read.
@@ -78,11 +82,12 @@ __device__ __forceinline__ bf16x8 as_bf8(const uint4& v) { return __builtin_bit_
 // zeros, which keeps the loop free of branches that the loads would wait in.
 //
 // What bounds it: a group is 132 MFMAs of 32 cycles of its SIMD's matrix core
-// (and 32 of 8) and about 1150 vector instructions of 4 cycles; two wavefronts
-// per SIMD (250 registers) overlap them in part.  32x32x16 MFMAs are half as many
+// (and 16 of 16) and about 1150 vector instructions of 4 cycles; two wavefronts
+// per SIMD (256 registers) overlap them in part.  32x32x16 MFMAs are half as many
 // to issue as 16x16x32 ones.  The splits stay an unpacking and a subtraction:
 // a dot-product instruction does both at once, but runs on the matrix core
-// and does not overlap with MFMAs.  The logits, 3 of 32 rows, use 4x4x4 MFMAs.
+// and does not overlap with MFMAs.  The logits, 3 of 16 rows, use 16x16x32 MFMAs, in
+// layer 1's row order two lane swaps from its D fragments.
 //
 // Measured against four wavefronts that shared a group (32 hidden features each,
 // activations exchanged through LDS, three barriers a group): 7.80M records with
@@ -93,11 +98,11 @@ __device__ __forceinline__ bf16x8 as_bf8(const uint4& v) { return __builtin_bit_
 constexpr int kFwdWaves = 4;
 constexpr int kXChunks = 15;
 struct alignas(16) SmemFwd {
-    uint4 w0[6 * 128];             // [chunk][hidden feature]: W0^T columns 8c .. 8c + 7; b0's split
+    uint4 w0[6 * 128];             // [chunk][tile row]: W0^T columns 8c .. 8c + 7; b0's split
     uint4 w1[4 * 9 * 64];          // [row tile][step][lane]: b1's split, then W1^T's A
-                                   // fragments of the eight k-steps, K permuted
-    uint4 w2[8 * 2 * 4];           // W2^T rows [k-step][h][logit, zeros], K permuted
-    uint4 ones[2];                 // [h] the inputs that the biases' splits are multiplied with
+                                   // fragments of the eight k-steps
+    uint4 w2[4 * 4 * 4];           // W2^T rows [tile][group of eight features][logit, zeros]
+    uint4 ones;                    // the inputs that the biases' splits are multiplied with
     uint4 x[kFwdWaves][GS][kXChunks];
 };
 
@@ -179,16 +184,16 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
     const int64_t ngroups = (total + GS - 1) / GS;
     const int64_t stride = (int64_t)gridDim.x * kFwdWaves;
     uint4* const xr = sm.x[wv][n];  // this lane's sample
-    const uint4* const xlast = h ? &sm.ones[0] : &xr[14];
-    // W0 fragments: this lane's rows of the k-steps' chunk pairs (A, B), (2, 3),
-    // (4, 2), (3, 4) and (4, bias)
-    const uint4* const w0ab = sm.w0 + 128 * h + n;
-    const uint4* const w023 = sm.w0 + 128 * (2 + h) + n;
-    const uint4* const w042 = sm.w0 + 128 * (4 - 2 * h) + n;
+    const uint4* const xfirst = h ? &xr[0] : &sm.ones;
+    // W0 fragments: this lane's rows of the k-steps' chunk pairs (bias, 0), (1, 2),
+    // (3, 0), (3, 4) and (4, 4)
+    const uint4* const w0b0 = sm.w0 + (h ? 0 : 128 * 5) + n;
+    const uint4* const w012 = sm.w0 + 128 * (1 + h) + n;
+    const uint4* const w030 = sm.w0 + (h ? 0 : 128 * 3) + n;
     const uint4* const w034 = sm.w0 + 128 * (3 + h) + n;
-    const uint4* const w04b = sm.w0 + 128 * (4 + h) + n;
+    const uint4* const w044 = sm.w0 + 128 * 4 + n;
     const uint4* const w1p = sm.w1 + lane;
-    const uint4* const w2p = sm.w2 + 4 * h + (n & 3);
+    const uint4* const w2p = sm.w2 + 4 * (lane >> 4) + min(lane & 15, 3);
 
     const int32_t* const none = reinterpret_cast<const int32_t*>(R.zero + 12);  // a leaf index of -1
     // the group two ahead: its records (position, flags); zero flags past the end
@@ -279,9 +284,9 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
             nbits & kAliveW ? R.pe + 96 * (int64_t)(nbits & kRayMask)
                             : reinterpret_cast<const uint16_t*>(R.zero));
         pe[0] = row[1 + h];
-        pe[1] = row[3 + 2 * h];
-        pe[2] = row[6 + h];
-        pe[3] = row[9 + h];
+        pe[1] = row[5 + h];
+        pe[2] = row[9 + h];
+        pe[3] = row[3 + 4 * h];
         pe[4] = row[11];
         peb[0] = reinterpret_cast<const uint2*>(row + 4 * h)[1];
         peb[1] = reinterpret_cast<const uint2*>(row + 8 - 4 * h)[1];
@@ -303,14 +308,15 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
             f[p] = hi[p];
-            f[8 + p] = mi[p];
-            f[16 + p] = lo[p];
+            f[16 + p] = mi[p];
+            f[32 + p] = lo[p];
         }
-        uint2* b = reinterpret_cast<uint2*>(xr) + 3;  // chunk B's half of part p: b[4 p]
-        b[4 * h] = peb[0];
-        b[8 - 4 * h] = peb[1];
+        uint2* b = reinterpret_cast<uint2*>(xr) + 3;  // chunk 1's half of part p: b[8 p]
+        b[8 * h] = peb[0];
+        b[16 - 8 * h] = peb[1];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) reinterpret_cast<u32x4*>(xr)[6 + 2 * t + h] = pe[t];
+        for (int t = 0; t < 3; ++t) reinterpret_cast<u32x4*>(xr)[2 + 4 * t + h] = pe[t];
+        reinterpret_cast<u32x4*>(xr)[12 + h] = pe[3];
         if (h == 0) reinterpret_cast<u32x4*>(xr)[14] = pe[4];
     };
 
@@ -339,16 +345,14 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
         const int64_t q0 = grp * GS;
         const bool alive = (nbits & kAliveW) != 0u;
         uint4 xb[8];  // this group's X fragments
+        xb[0] = *xfirst;
 #pragma unroll
-        for (int t = 0; t < 7; ++t) xb[t] = xr[2 * t + h];
-        xb[7] = *xlast;
+        for (int t = 1; t < 8; ++t) xb[t] = xr[2 * t - 1 + h];
         {  // the backward's input row: X columns 0..39 (hi)
             uint4* row = rec.xrow + 5 * q0 + 5 * n;
-            row[h] = xb[0];
-            row[2 + h] = xb[3];
-            // half 1 stores chunk 3 a second time
-            row[4 - h] = make_uint4(h ? xb[3].x : xb[4].x, h ? xb[3].y : xb[4].y,
-                                    h ? xb[3].z : xb[4].z, h ? xb[3].w : xb[4].w);
+            row[h] = xr[h];
+            row[2 + h] = xr[2 + h];
+            row[4] = xr[12];  // both halves, the same values
         }
         lookup();
         load_records(grp + 2 * stride);
@@ -357,72 +361,95 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
         // layer's B fragments while the matrix core works, and every weight
         // fragment is read two steps ahead of its use.  The scheduling barriers
         // keep the compiler from gathering either kind together again.
-        uint32_t mask0[2] = {0u, 0u}, mask1[2] = {0u, 0u};  // words h and h + 2 (q even, odd)
+        uint32_t mask0[2] = {0u, 0u}, mask1[2] = {0u, 0u};  // words 2h and 2h + 1 (T / 2)
         uint32_t h0[8][3][4];  // layer 1's B fragments [k-step][part][dword]
-        uint32_t h1[2][4];     // layer 2's of one k-step
+        uint32_t h1[2][2][4];  // layer 2's of a tile: [rows' half t, then samples' half s][part]
         f32x16 c, d;           // a tile in the making, the one before
-        f32x4 lg = {0.f, 0.f, 0.f, 0.f};  // the sample's logits over this lane's features
+        f32x4 lt[2], lg[2];    // samples 16s ..: the logits over a tile's features, over all before
         const f32x16 zero = {};
         auto pair0 = [&](int T, int j) {  // pair j (rows 2j, 2j + 1 of the lane) of tile T
             uint32_t(*f)[4] = h0[2 * T + (j >> 2)];
             split3(relu(d[2 * j]), relu(d[2 * j + 1]), f[0][j & 3], f[1][j & 3], f[2][j & 3]);
-            mask_pair(f[0][j & 3], 2 * (2 * T + (j >> 2)) + (j & 1), mask0[(j >> 1) & 1]);
-            pin(f[0][j & 3], f[1][j & 3], f[2][j & 3], mask0[(j >> 1) & 1]);
+            mask_pair(f[0][j & 3], 8 * (T & 1) + j, mask0[T >> 1]);
+            pin(f[0][j & 3], f[1][j & 3], f[2][j & 3], mask0[T >> 1]);
+        };
+        // the logits over tiles 0 .. T
+        auto add_logits = [&](int T) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int o = 0; o < 3; ++o) lg[s][o] = T == 0 ? lt[s][o] : lg[s][o] + lt[s][o];
         };
         uint4 w2f;
         auto pair1 = [&](int T, int j) {
-            if ((j & 3) == 1) w2f = w2p[8 * (2 * T + (j >> 2))];
-            split2(relu(d[2 * j]), relu(d[2 * j + 1]), h1[0][j & 3], h1[1][j & 3]);
-            mask_pair(h1[0][j & 3], 2 * (2 * T + (j >> 2)) + (j & 1), mask1[(j >> 1) & 1]);
-            pin(h1[0][j & 3], h1[1][j & 3], mask1[0], mask1[1]);
-            if ((j & 3) == 3) {  // layer 2's k-step 2T + j / 4
+            uint32_t(*f)[4] = h1[j >> 2];
+            split2(relu(d[2 * j]), relu(d[2 * j + 1]), f[0][j & 3], f[1][j & 3]);
+            mask_pair(f[0][j & 3], 8 * (T & 1) + j, mask1[T >> 1]);
+            pin(f[0][j & 3], f[1][j & 3], mask1[0], mask1[1]);
+            if (j == 2 && T > 0) add_logits(T - 1);
+            if (j == 5) w2f = w2p[16 * T];
+            if (j >= 4) {
+                // a lane's two groups of eight features (2h + t) to the four of one
+                // sample half, a group to each 16 lanes
 #pragma unroll
                 for (int p = 0; p < 2; ++p) {
-                    lg = mfma4x4x4(w2f.x, w2f.y, h1[p][0], h1[p][1], lg);
-                    lg = mfma4x4x4(w2f.z, w2f.w, h1[p][2], h1[p][3], lg);
+                    const auto r = __builtin_amdgcn_permlane16_swap(h1[0][p][j & 3], h1[1][p][j & 3],
+                                                                    false, false);
+                    h1[0][p][j & 3] = r[0];
+                    h1[1][p][j & 3] = r[1];
                 }
+            }
+            if (j == 7) {  // layer 2 over the tile's 32 features
+                const bf16x8 w = as_bf8(w2f);
+                const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < 2; ++s) lt[s] = mfma16x16x32(w, as_bf8(frag(h1[s][0])), z);
+#pragma unroll
+                for (int s = 0; s < 2; ++s) lt[s] = mfma16x16x32(w, as_bf8(frag(h1[s][1])), lt[s]);
             }
         };
         // ---- layer 0: H0^T = relu(W0^T X^T + b0) ----
-        uint4 fa = w0ab[0], fb = w023[0];
+        uint4 fa = w0b0[0], fb = w012[0], fc = w030[0];
 #pragma unroll
         for (int T = 0; T < 4; ++T) {
             if (T == 3) fetch(0, raw);  // the next group's inputs, from here to layer 1's end
-            const uint4 f2 = w042[32 * T];
             c = mfma32x32x16(fa, xb[0], zero);
             if (T > 0) pair0(T - 1, 0);
             __builtin_amdgcn_sched_barrier(0);
-            c = mfma32x32x16(fa, xb[1], c);
+            fa = w034[32 * T];
+            c = mfma32x32x16(fb, xb[1], c);
             if (T > 0) pair0(T - 1, 1);
             __builtin_amdgcn_sched_barrier(0);
-            const uint4 f3 = w034[32 * T];
-            c = mfma32x32x16(fa, xb[2], c);
+            c = mfma32x32x16(fc, xb[2], c);
             if (T > 0) pair0(T - 1, 2);
             __builtin_amdgcn_sched_barrier(0);
             c = mfma32x32x16(fb, xb[3], c);
             if (T > 0) pair0(T - 1, 3);
             __builtin_amdgcn_sched_barrier(0);
-            const uint4 f4 = w04b[32 * T];
-            c = mfma32x32x16(fb, xb[6], c);
+            c = mfma32x32x16(fc, xb[4], c);
             if (T > 0) pair0(T - 1, 4);
             __builtin_amdgcn_sched_barrier(0);
-            fa = T < 3 ? w0ab[32 * (T + 1)] : w1p[0];
-            c = mfma32x32x16(f2, xb[4], c);
+            fc = w044[32 * T];
+            c = mfma32x32x16(fb, xb[5], c);
             if (T > 0) pair0(T - 1, 5);
             __builtin_amdgcn_sched_barrier(0);
-            fb = T < 3 ? w023[32 * (T + 1)] : w1p[64];
-            c = mfma32x32x16(f3, xb[5], c);
+            fb = T < 3 ? w012[32 * (T + 1)] : w1p[64];
+            c = mfma32x32x16(fa, xb[6], c);
             if (T > 0) pair0(T - 1, 6);
             __builtin_amdgcn_sched_barrier(0);
-            c = mfma32x32x16(f4, xb[7], c);
+            fa = T < 3 ? w0b0[32 * (T + 1)] : w1p[0];
+            c = mfma32x32x16(fc, xb[7], c);
             if (T > 0) pair0(T - 1, 7);
             __builtin_amdgcn_sched_barrier(0);
+            if (T < 3) fc = w030[32 * (T + 1)];
             d = c;
         }
         // ---- layer 1: H1^T = relu(W1^T H0^T + b1); layer 2 over its tiles ----
+        uint4 f[3] = {fa, fb};
 #pragma unroll
         for (int T = 0; T < 4; ++T) {
-            uint4 fn = w1p[64 * (9 * T + 2)];
+            // step 9T + k (the bias, then the k-steps) is in f[(9T + k) % 3]
+            f[(9 * T + 2) % 3] = w1p[64 * (9 * T + 2)];
             if (T == 1) {
                 weigh(0, raw, v);
                 fetch(1, raw);
@@ -434,24 +461,25 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
                 for (int i = 0; i < 12; ++i) v[i] += w[i];
                 fetch_pe();
             }
-            c = mfma32x32x16(fa, sm.ones[h], zero);
-            fa = fb;
-            fb = fn;
+            c = mfma32x32x16(f[(9 * T) % 3], sm.ones, zero);
 #pragma unroll
-            for (int ks = 0; ks < 8; ++ks) {
-                fn = w1p[64 * min(9 * T + ks + 3, 35)];
-                c = mfma32x32x16(fa, frag(h0[ks][0]), c);
-                c = mfma32x32x16(fa, frag(h0[ks][1]), c);
-                c = mfma32x32x16(fa, frag(h0[ks][2]), c);
-                fa = fb;
-                fb = fn;
-                if (T > 0) {
-                    pair1(T - 1, ks);
-                } else if (ks < 4) {  // the last layer-0 tile is k-steps 6 and 7's input
-                    pair0(3, 2 * ks);
-                    pair0(3, 2 * ks + 1);
+            for (int kt = 0; kt < 4; ++kt) {  // 32 features: their hi parts, mid parts, lo parts
+                const int s = 9 * T + 1 + 2 * kt;
+                if (s + 2 < 36) f[(s + 2) % 3] = w1p[64 * (s + 2)];
+#pragma unroll
+                for (int m = 0; m < 6; ++m) {
+                    c = mfma32x32x16(f[(s + (m & 1)) % 3], frag(h0[2 * kt + (m & 1)][m >> 1]), c);
+                    if (m == 4 && s + 3 < 36) f[s % 3] = w1p[64 * (s + 3)];
+                    if (m % 3 != 2) continue;
+                    const int slot = 2 * kt + m / 3;
+                    if (T > 0) {
+                        pair1(T - 1, slot);
+                    } else if (slot < 4) {  // the last layer-0 tile is k-steps 6 and 7's input
+                        pair0(3, 2 * slot);
+                        pair0(3, 2 * slot + 1);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                __builtin_amdgcn_sched_barrier(0);
             }
             d = c;
         }
@@ -459,20 +487,23 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
         for (int j = 0; j < 8; ++j) pair1(3, j);
         store_x(v);
         wave_lds_fence();
+        add_logits(3);
         // ---- the masks and rgb ----
         {
-            uint32_t* mw = rec.relu + 8 * q0 + 8 * n + h;
-            mw[0] = mask0[0];
-            mw[2] = mask0[1];
-            mw[4] = mask1[0];
-            mw[6] = mask1[1];
-            // the two lane halves' sums: half h is left with logit h, both with
-            // logit 2; half h finishes channel h, half 0
+            uint2* mw = reinterpret_cast<uint2*>(rec.relu + 8 * q0 + 8 * n + 2 * h);
+            mw[0] = make_uint2(mask0[0], mask0[1]);
+            mw[2] = make_uint2(mask1[0], mask1[1]);
+            // the first 16 lanes hold both sample halves' logits: those of 16 .. 31 to the
+            // lanes after them, then logit 1 to half 1; half h finishes channel h, half 0
             // channel 2 too (half 1 writes the unused fourth)
-            const auto r01 = __builtin_amdgcn_permlane32_swap(
-                __float_as_uint(lg[0]), __float_as_uint(lg[1]), false, false);
-            const float x = __uint_as_float(r01[0]) + __uint_as_float(r01[1]);
-            const float y = lg[2] + __shfl_xor(lg[2], 32, 64);
+            uint32_t l[3];
+#pragma unroll
+            for (int o = 0; o < 3; ++o)
+                l[o] = __builtin_amdgcn_permlane16_swap(__float_as_uint(lg[0][o]),
+                                                        __float_as_uint(lg[1][o]), false, false)[0];
+            const float x = __uint_as_float(
+                __builtin_amdgcn_permlane32_swap(l[0], l[1], false, false)[0]);
+            const float y = __uint_as_float(l[2]);
             const float a = sigmoidf_(x + b2a), b = sigmoidf_(y + b2b);
             float* rgb = reinterpret_cast<float*>(rec.rgb + q0) + 4 * n + h;
             rgb[0] = alive ? a : 0.f;
@@ -487,12 +518,11 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
 // its group's chain
 //   g_H1^T = W2 g_L^T (masked), g_H0^T = W1 g_H1^T (masked), g_X^T = W0[0:12] g_H0^T
 // with the gradients as (hi, lo) pairs, in registers from end to end as in the
-// forward: a D fragment of 32x32x16 is the next product's B fragment under the
-// permuted K order.  The other, the weight wavefront, recomputes
+// forward: all rows are in layer 0's order.  The other, the weight wavefront, recomputes
 //   H0^T = relu(W0^T X^T + b0), H1 = relu(H0 W1 + b1)
-// from hi parts (for the dW operands only: the gradients are masked by the
-// forward's own ReLU masks; H1 comes out a feature to a lane, since its operands
-// are the same fragments in the other order), adds its group's H1^T g_L to dW2, and
+// from hi parts (for the dW operands only; H1 comes out a feature to a lane, in
+// layer 1's order, since its operands are the same fragments in the other order),
+// adds its group's H1^T g_L to dW2, and
 // then a slice of the whole round's dW1 += H0^T g_H1 (64 x 64) and dW0 += X^T g_H0
 // (all inputs x 32).  Those contract over samples, so their operands cross
 // wavefronts: H0, g_H1, g_H0 (hi) and X lie in LDS a row to a sample, and are read
@@ -533,11 +563,13 @@ struct alignas(16) SmemBwd {
     uint16_t g0[kRoundRec * 128];
     uint16_t h0[kRoundRec * 128];
     uint16_t x[kRoundRec * 40 + 24];  // X by sample; loads of columns 40..63 run into the next row
-    uint4 w0[6 * 128];              // the forward image's W0^T chunks and b0's split
+    uint4 w0[5 * 128];              // the forward image's W0^T chunks
     uint16_t w1[32 * kFragPitch];   // the forward image's W1^T fragments [row tile][k-step]
-    uint4 w2[128];                  // W2's rows as g_H1's A fragments, b1 in the last word
+    uint2 w2[128];                  // W2's rows
+    float b0[128], b1[128];
     uint4 w0g[8 * 2 * 12];          // W0[0:12] as g_X's A fragments [k-step][h][feature]
     uint16_t gl[kBwdPairs][3 * GS]; // dL/dlogit (hi) by logit
+    uint32_t m1[kBwdPairs][4][GS];  // layer 1's ReLU mask words by word
 };
 static_assert(sizeof(SmemBwd) <= 160 * 1024, "a CU's LDS");
 
@@ -582,7 +614,7 @@ __device__ __forceinline__ float keep_if(uint32_t m, int k, float x) {
 __device__ __forceinline__ void stage_bwd_weights(SmemBwd& sm, const MlpPacked& W) {
     constexpr int NTH = 64 * kBwdWaves;
     const int tid = threadIdx.x;
-    for (int e = tid; e < 6 * 128; e += NTH) sm.w0[e] = W.fwd[e];
+    for (int e = tid; e < 5 * 128; e += NTH) sm.w0[e] = W.fwd[e];
     const uint4* img = W.fwd + kImgW1 / 8;  // [row tile][9 steps, the first the bias][lane]
 #pragma unroll
     for (int k = 0; k < 32 * 64 / NTH; ++k) {
@@ -590,14 +622,13 @@ __device__ __forceinline__ void stage_bwd_weights(SmemBwd& sm, const MlpPacked& 
         *reinterpret_cast<uint4*>(sm.w1 + f * kFragPitch + (l >> 5) * kHalfPitch + 8 * (l & 31)) =
             img[((f >> 3) * 9 + 1 + (f & 7)) * 64 + l];
     }
-    if (tid < 128) {  // K: the logits' hi parts, their lo parts
-        const uint2 w = *reinterpret_cast<const uint2*>(W.w2 + 32 * tid);  // w0 w1 | w2 0
-        sm.w2[tid] = make_uint4(w.x, (w.y & 0xffffu) | (w.x << 16), (w.x >> 16) | (w.y << 16),
-                                __float_as_uint(W.b1[tid]));
+    if (tid < 128) {
+        sm.w2[tid] = *reinterpret_cast<const uint2*>(W.w2 + 32 * tid);  // w0 w1 | w2 0
+        sm.b0[tid] = W.b0[tid];
+        sm.b1[tid] = W.b1[tid];
     } else if (tid < 128 + 8 * 2 * 12) {
         const int e = tid - 128, m = e % 12, h = (e / 12) & 1, ks = e / 24;
-        const uint2* src = reinterpret_cast<const uint2*>(W.w0 + 128 * m + 16 * ks + 4 * h);
-        sm.w0g[e] = make_uint4(src[0].x, src[0].y, src[2].x, src[2].y);
+        sm.w0g[e] = *reinterpret_cast<const uint4*>(W.w0 + 128 * m + 16 * ks + 8 * h);
     }
 }
 
@@ -618,42 +649,43 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
     // where this lane's sample stores its pieces, and what it points the
     // transposing loads at: row rr (+ 4h + 8jj + 16t) and piece pc of 16 c16 features
     const int rr = (lane & 15) >> 2, pc = lane & 3, c16 = (lane >> 4) & 1;
-    // the bytes of this lane's first piece in its sample's row: piece 8T + 2q + h lies at
-    // the same offset ^ (64 T + 16 q).  Anew in each round: as loop invariants the
-    // sixteen addresses would take as many registers
+    // the bytes of this lane's first piece in its sample's row: piece
+    // 8T + 4 (q / 2) + 2h + q % 2, which holds the lane's rows 8q + 4h .. of tile T (layer
+    // 0's order), lies at the same offset ^ (64 T + 32 (q / 2) + 8 (q % 2)).  Anew in each
+    // round: as loop invariants the sixteen addresses would take as many registers
     auto row_at = [&]() {
-        uint32_t at = 256 * (GS * w + n) + 8 * ((((n & 3) << 3) | (n >> 2)) ^ h);
+        uint32_t at = 256 * (GS * w + n) + 8 * ((((n & 3) << 3) | (n >> 2)) ^ (2 * h));
         asm volatile("" : "+v"(at));
         return at;
     };
     auto piece = [](uint16_t* rows, uint32_t at, int T, int q) {
-        return reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(rows) + (at ^ (64u * T + 16u * q)));
+        return reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(rows) +
+                                        (at ^ (64u * T + 32u * (q >> 1) + 8u * (q & 1))));
     };
 
     if (wv >= kBwdPairs) {
         // ---- the gradient chain ----
         float4 adj, nadj;
-        uint32_t mk[4], nmk[4], bits, nbits;  // ReLU mask words: layer 0's h, h + 2, layer 1's
+        uint2 mk0, nmk0, nmk1;  // this lane half's ReLU mask words of the two layers
+        uint32_t bits, nbits;
         auto load = [&](int64_t rnd) {  // the next round's
             const int64_t q = rnd * kRoundRec + GS * w + n;
             nadj = make_float4(0.f, 0.f, 0.f, 0.f);
-            nmk[0] = nmk[1] = nmk[2] = nmk[3] = nbits = 0u;
+            nmk0 = nmk1 = make_uint2(0u, 0u);
+            nbits = 0u;
             if (q < total) {
                 nadj = rec.adj[q];
                 nbits = __float_as_uint(rec.ab[q].y);
-                const uint32_t* m = rec.relu + 8 * q + h;
-                nmk[0] = m[0];
-                nmk[1] = m[2];
-                nmk[2] = m[4];
-                nmk[3] = m[6];
+                nmk0 = reinterpret_cast<const uint2*>(rec.relu)[4 * q + h];
+                nmk1 = reinterpret_cast<const uint2*>(rec.relu)[4 * q + 2 + h];
             }
         };
         float db1[64], db2[3] = {0.f, 0.f, 0.f};  // this lane's sample of each round
 #pragma unroll
         for (int i = 0; i < 64; ++i) db1[i] = 0.f;
-        // W1 rows (lane: in-feature n of a tile) out of the W1^T fragments
+        // W1 rows (in layer 0's order) out of the W1^T fragments
         const uint16_t* const wa = sm.w1 + c16 * kFragPitch + (pc & 1) * kHalfPitch +
-                                   8 * (4 * h + rr) + 4 * (pc >> 1);
+                                   8 * (16 * h + rr) + 4 * (pc >> 1);
         const uint4* const w0p = sm.w0g + 12 * h + (n < 12 ? n : 0);
         const f32x16 zero = {};
         uint32_t gh[8][4], glo[8][4];  // g_H1's B fragments [k-step][dword], hi and lo
@@ -661,19 +693,27 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
         f32x16 d;                      // a finished tile, split while the next one's MFMAs run
         float va, vb;
         // pair j (rows 2j, 2j + 1 of the lane) of tile T in two steps: masked, then split
-        auto mask_of = [&](int T, int j, uint32_t ma, uint32_t mb) {
-            const uint32_t m = (j >> 1) & 1 ? mb : ma;
-            const int p = 2 * (2 * T + (j >> 2)) + (j & 1);
+        auto mask_of = [&](uint32_t m, int p, int j) {
             va = keep_if(m, p, d[2 * j]);
             vb = keep_if(m, 16 + p, d[2 * j + 1]);
         };
+        auto mask0 = [&](int T, int j) { mask_of(T & 2 ? mk0.y : mk0.x, 8 * (T & 1) + j, j); };
+        // g_H1's rows are in layer 0's order: feature 16 (j / 4) + 8h + .. of the tile is the
+        // forward's row pair 4h + j % 4 of lane half j / 4
+        uint32_t mk1[2];
+        auto mask1 = [&](int T, int j) {
+            if (j == 0 && !(T & 1))
+#pragma unroll
+                for (int f = 0; f < 2; ++f) mk1[f] = sm.m1[w][2 * f + (T >> 1)][n] >> (4 * h);
+            mask_of(mk1[j >> 2], 8 * (T & 1) + (j & 3), j);
+        };
         auto w1 = [&](int T, int ks) {
-            const uint16_t* a = wa + ((ks >> 1) * 8 + 2 * T) * kFragPitch + 128 * (ks & 1);
+            const uint16_t* a = wa + ((ks >> 1) * 8 + 2 * T) * kFragPitch + 32 * (ks & 1);
             return ld_tr2(a, a + 64);
         };
         // pair j of g_H1's tile T: gh, glo and db1
         auto pair1 = [&](int T, int j) {
-            mask_of(T, j, mk[2], mk[3]);
+            mask1(T, j);
             db1[16 * T + 2 * j] += va;
             db1[16 * T + 2 * j + 1] += vb;
             uint32_t &hi = gh[2 * T + (j >> 2)][j & 3], &lo = glo[2 * T + (j >> 2)][j & 3];
@@ -685,10 +725,12 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
         // layer 0's features of tile T into the records' gradients
         auto add_gx = [&](int T) {
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const uint4 f = w0p[24 * (2 * T + t)];
-                gx = mfma32x32x16(f, make_uint4(lo[4 * t], lo[4 * t + 1], lo[4 * t + 2], lo[4 * t + 3]), gx);
-                gx = mfma32x32x16(f, make_uint4(hi[4 * t], hi[4 * t + 1], hi[4 * t + 2], hi[4 * t + 3]), gx);
+            for (int p = 0; p < 2; ++p) {  // the hi parts, then the lo parts
+                const uint32_t* v = p ? lo : hi;
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    gx = mfma32x32x16(w0p[24 * (2 * T + t)],
+                                      make_uint4(v[4 * t], v[4 * t + 1], v[4 * t + 2], v[4 * t + 3]), gx);
             }
         };
         auto pair0_split = [&](int j) {
@@ -701,8 +743,10 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
             // ---- interval 1 ----
             adj = nadj;
             bits = nbits;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) mk[i] = nmk[i];
+            mk0 = nmk0;
+            sm.m1[w][2 * h][n] = nmk1.x;
+            sm.m1[w][2 * h + 1][n] = nmk1.y;
+            wave_lds_fence();  // this wavefront reads both halves'
             {
                 uint32_t h01, l01, h2, l2;
                 split2(adj.x, adj.y, h01, l01);
@@ -716,11 +760,11 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
                     g[GS] = (uint16_t)(h01 >> 16);
                     g[2 * GS] = (uint16_t)h2;
                 }
-                const uint4 b = h ? make_uint4(0u, 0u, 0u, 0u)
-                                  : make_uint4(h01, h2 | (l01 << 16), (l01 >> 16) | (l2 << 16), 0u);
+                // the hi parts in half 0's k, the lo parts in half 1's
+                const uint4 b = make_uint4(h ? l01 : h01, h ? l2 : h2, 0u, 0u);
                 auto w2 = [&](int T) {
-                    const uint4 f = sm.w2[32 * T + n];
-                    return make_uint4(h ? 0u : f.x, h ? 0u : f.y, h ? 0u : f.z, 0u);
+                    const uint2 f = sm.w2[32 * T + mlp_feature(0, n)];
+                    return make_uint4(f.x, f.y, 0u, 0u);
                 };
                 // g_H1 a tile at a time, each followed by its k-steps of g_H0's first tile
                 // under the next one's split
@@ -742,8 +786,8 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         if (T > 0) {
-                            const int ks = 2 * T - 2 + (k >> 1);
-                            c = mfma32x32x16(k < 2 ? f0 : f1, frag(k & 1 ? gh[ks] : glo[ks]),
+                            const int ks = 2 * T - 2 + (k & 1);
+                            c = mfma32x32x16(k & 1 ? f1 : f0, frag(k < 2 ? gh[ks] : glo[ks]),
                                              T == 1 && k == 0 ? zero : c);
                         }
                         if (T < 4) {
@@ -761,34 +805,40 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
             load(rnd + stride);
             const uint32_t at = row_at();
             gx = zero;
-            uint4 f[3] = {w1(1, 0), w1(1, 1)};  // read two steps ahead
+            uint4 f[3] = {w1(1, 0), w1(1, 1)};  // step k is in f[k % 3]
 #pragma unroll
             for (int T = 1; T < 4; ++T) {
                 f32x16 c = zero;
 #pragma unroll
-                for (int ks = 0; ks < 8; ++ks) {
-                    const int k = 8 * (T - 1) + ks;
+                for (int kt = 0; kt < 4; ++kt) {  // 32 features: their hi parts, their lo parts
+                    const int k = 8 * (T - 1) + 2 * kt;
                     if (k < 22) f[(k + 2) % 3] = w1(1 + (k + 2) / 8, (k + 2) & 7);
-                    c = mfma32x32x16(f[k % 3], frag(glo[ks]), c);
-                    mask_of(T - 1, ks, mk[0], mk[1]);
-                    if (T == 1 && (ks & 1))  // g_H1's rows, between the first MFMAs
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const uint32_t* g = gh[ks - 1 + (q >> 1)] + 2 * (q & 1);
-                            *piece(sm.g1, at, ks >> 1, q) = make_uint2(g[0], g[1]);
+                    for (int m = 0; m < 4; ++m) {
+                        const int ks = 2 * kt + (m & 1), j = 2 * kt + (m >> 1);
+                        c = mfma32x32x16(f[(k + (m & 1)) % 3], frag(m < 2 ? gh[ks] : glo[ks]), c);
+                        if (m == 2 && k < 22) f[k % 3] = w1(1 + (k + 3) / 8, (k + 3) & 7);
+                        if (m & 1) {
+                            pair0_split(j);
+                            if (j & 1) *piece(sm.g0, at, T - 1, j >> 1) = make_uint2(hi[j - 1], hi[j]);
+                        } else {
+                            mask0(T - 1, j);
+                            if (T == 1 && m == 2)  // g_H1's rows, between the first MFMAs
+#pragma unroll
+                                for (int q = 0; q < 4; ++q) {
+                                    const uint32_t* g = gh[j - 1 + (q >> 1)] + 2 * (q & 1);
+                                    *piece(sm.g1, at, j >> 1, q) = make_uint2(g[0], g[1]);
+                                }
                         }
-                    __builtin_amdgcn_sched_barrier(0);
-                    c = mfma32x32x16(f[k % 3], frag(gh[ks]), c);
-                    pair0_split(ks);
-                    if (ks & 1) *piece(sm.g0, at, T - 1, ks >> 1) = make_uint2(hi[ks - 1], hi[ks]);
-                    __builtin_amdgcn_sched_barrier(0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
                 add_gx(T - 1);
                 d = c;
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                mask_of(3, j, mk[0], mk[1]);
+                mask0(3, j);
                 pair0_split(j);
                 if (j & 1) *piece(sm.g0, at, 3, j >> 1) = make_uint2(hi[j - 1], hi[j]);
             }
@@ -810,7 +860,8 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
 #pragma unroll
         for (int i = 0; i < 64; ++i) {
             const float v = half_sum(db1[i]);
-            if (n == 31) red[kRedDb1 + 128 * w + 32 * (i >> 4) + 8 * ((i >> 2) & 3) + 4 * h + (i & 3)] = v;
+            if (n == 31)
+                red[kRedDb1 + 128 * w + 32 * (i >> 4) + 16 * ((i >> 3) & 1) + 8 * h + (i & 7)] = v;
         }
 #pragma unroll
         for (int o = 0; o < 3; ++o) {
@@ -826,7 +877,7 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
         for (int a = 0; a < 2; ++a) dW1[a][0] = dW1[a][1] = dW0[a] = zero;
 #pragma unroll
         for (int T = 0; T < 4; ++T) dW2[T] = f32x4{0.f, 0.f, 0.f, 0.f};
-        uint4 xb[3];  // the group's X fragments: columns 8h, 16 + 8h, and 32 (h = 1: the bias inputs)
+        uint4 xb[3];  // the group's X fragments: columns 8h, 16 + 8h, and 32 (h = 1: zeros)
         auto load = [&](int64_t rnd) {
             const int64_t q = rnd * kRoundRec + GS * w + n;
             xb[0] = xb[1] = xb[2] = make_uint4(0u, 0u, 0u, 0u);
@@ -838,7 +889,9 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
             }
         };
         const uint4* const w0p = sm.w0 + 128 * h + n;
+        const float* const b0p = sm.b0 + 8 * h;
         const uint16_t* const w1p = sm.w1 + h * kHalfPitch + 8 * n;
+        const float* const b1p = sm.b1 + mlp_feature(1, n);  // of this lane's feature of tile 0
         // dW1 and dW0 of the round in the buffers
         auto dw = [&]() {
             uint4 fr[2][7];  // a k-step's operands, read one step ahead
@@ -900,10 +953,7 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
                 uint4* xr = reinterpret_cast<uint4*>(sm.x + (GS * w + n) * 40);
                 xr[h] = xb[0];
                 xr[2 + h] = xb[1];
-                if (h == 0)
-                    xr[4] = xb[2];
-                else
-                    xb[2] = make_uint4(0x3f803f80u, 0x3f80u, 0u, 0u);
+                if (h == 0) xr[4] = xb[2];
             }
             uint32_t h0[8][4];
             const uint32_t at = row_at();
@@ -916,8 +966,17 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
 #pragma unroll
             for (int T = 0; T < 4; ++T) {
 #pragma unroll
+                for (int q = 0; q < 4; ++q) {  // the accumulators start at the bias
+                    const float4 b = *reinterpret_cast<const float4*>(b0p + 32 * T + 16 * (q >> 1) + 4 * (q & 1));
+                    c[4 * q] = b.x;
+                    c[4 * q + 1] = b.y;
+                    c[4 * q + 2] = b.z;
+                    c[4 * q + 3] = b.w;
+                }
+#pragma unroll
                 for (int k = 0; k < 3; ++k) {
-                    c = mfma32x32x16(w0p[256 * k + 32 * T], xb[k], k == 0 ? zero : c);
+                    // h = 1's last chunk meets zeros
+                    c = mfma32x32x16(w0p[(k < 2 ? 256 * k : 512 - 128 * h) + 32 * T], xb[k], c);
                     if (T > 0) {
                         pair0(T - 1, 3 * k);
                         pair0(T - 1, 3 * k + 1);
@@ -941,7 +1000,7 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
             };
 #pragma unroll
             for (int T = 0; T < 4; ++T) {
-                const float b1 = __uint_as_float(sm.w2[32 * T + n].w);
+                const float b1 = b1p[32 * T];
 #pragma unroll
                 for (int i = 0; i < 16; ++i) c[i] = b1;
 #pragma unroll
@@ -963,14 +1022,17 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
             for (int j = 0; j < 8; ++j) pair1(3, j);
             __syncthreads();
         }
-        if (r0 < nrounds) dw();
+        if ((int)blockIdx.x < (int)nrounds) dw();
         __syncthreads();  // the buffers are free for the reductions
+        int f1 = n;
+        asm volatile("" : "+v"(f1));  // not a register through the loop
+        f1 = mlp_feature(1, f1);
 #pragma unroll
         for (int T = 0; T < 4; ++T)
 #pragma unroll
             for (int o = 0; o < 3; ++o) {
                 const float v = dW2[T][o] + __shfl_xor(dW2[T][o], 32, 64);
-                if (h == 0) red[384 * w + 3 * (32 * T + n) + o] = v;
+                if (h == 0) red[384 * w + 3 * (32 * T + f1) + o] = v;
             }
         // ---- this workgroup's dW partial ----
 #pragma unroll

@@ -622,6 +622,7 @@ int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
     W.fwd = reinterpret_cast<const uint4*>(fwd);
     W.w2 = w2;
     W.w0 = w0;
+    W.b0 = direct ? nullptr : d->mlp + kB0;
     W.b1 = direct ? nullptr : d->mlp + kB1;
     W.b2 = direct ? nullptr : d->mlp + kB2;
 
