@@ -519,10 +519,10 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
 //   g_H1^T = W2 g_L^T (masked), g_H0^T = W1 g_H1^T (masked), g_X^T = W0[0:12] g_H0^T
 // with the gradients as (hi, lo) pairs, in registers from end to end as in the
 // forward: all rows are in layer 0's order.  The other, the weight wavefront, recomputes
-//   H0^T = relu(W0^T X^T + b0), H1 = relu(H0 W1 + b1)
+//   H0^T = W0^T X^T + b0, H1 = H0 W1 + b1 under the forward's masks
 // from hi parts (for the dW operands only; H1 comes out a feature to a lane, in
-// layer 1's order, since its operands are the same fragments in the other order),
-// adds its group's H1^T g_L to dW2, and
+// layer 1's order, since its operands are the same fragments in the other order,
+// and its mask bits out of LDS), adds its group's H1^T g_L to dW2, and
 // then a slice of the whole round's dW1 += H0^T g_H1 (64 x 64) and dW0 += X^T g_H0
 // (all inputs x 32).  Those contract over samples, so their operands cross
 // wavefronts: H0, g_H1, g_H0 (hi) and X lie in LDS a row to a sample, and are read
@@ -593,14 +593,6 @@ __device__ __forceinline__ float half_sum(float x) {
     x += dpp_mov<kDppRowShr8>(x, 0.f);
     x += dpp_mov<kDppRowBcast15, 0xa>(x, 0.f);
     return x;
-}
-
-// relu of two floats as a bf16 pair: rounding keeps order and zero, so the max,
-// of packed integers as in relu, may follow the conversion
-__device__ __forceinline__ uint32_t relu_bf2(float a, float b) {
-    uint32_t r;
-    asm("v_pk_max_i16 %0, %1, 0" : "=v"(r) : "v"(pk_bf(a, b)));
-    return r;
 }
 
 // x where bit k of m is set, else +0: the bit sign-extended by one v_bfe_i32
@@ -878,20 +870,26 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
 #pragma unroll
         for (int T = 0; T < 4; ++T) dW2[T] = f32x4{0.f, 0.f, 0.f, 0.f};
         uint4 xb[3];  // the group's X fragments: columns 8h, 16 + 8h, and 32 (h = 1: zeros)
+        uint2 m0;     // layer 0's ReLU mask words of this lane half
         auto load = [&](int64_t rnd) {
             const int64_t q = rnd * kRoundRec + GS * w + n;
             xb[0] = xb[1] = xb[2] = make_uint4(0u, 0u, 0u, 0u);
+            m0 = make_uint2(0u, 0u);
             if (q < total) {
                 const uint4* row = rec.xrow + 5 * q;
                 xb[0] = row[h];
                 xb[1] = row[2 + h];
                 if (h == 0) xb[2] = row[4];
+                m0 = reinterpret_cast<const uint2*>(rec.relu)[4 * q + h];
             }
         };
         const uint4* const w0p = sm.w0 + 128 * h + n;
         const float* const b0p = sm.b0 + 8 * h;
         const uint16_t* const w1p = sm.w1 + h * kHalfPitch + 8 * n;
-        const float* const b1p = sm.b1 + mlp_feature(1, n);  // of this lane's feature of tile 0
+        // layer 1: the bias of this lane's feature of tile 0, and where its mask bits are
+        const float* const b1p = sm.b1 + mlp_feature(1, n);
+        const int bit1 = 16 * (n & 1) + 2 * (n >> 3) + ((n >> 1) & 1);
+        const uint32_t* const m1p = &sm.m1[w][2 * ((n >> 2) & 1)][4 * h];
         // dW1 and dW0 of the round in the buffers
         auto dw = [&]() {
             uint4 fr[2][7];  // a k-step's operands, read one step ahead
@@ -958,9 +956,11 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
             uint32_t h0[8][4];
             const uint32_t at = row_at();
             f32x16 c, d;  // a tile in the making, the one before
-            auto pair0 = [&](int T, int j) {
+            // masked by the forward's bits, not by these values' signs
+            auto pair0 = [&](int T, int j, uint32_t m) {
                 uint32_t* f = h0[2 * T + (j >> 2)];
-                f[j & 3] = relu_bf2(d[2 * j], d[2 * j + 1]);
+                const int p = 8 * (T & 1) + j;
+                f[j & 3] = pk_bf(keep_if(m, p, d[2 * j]), keep_if(m, 16 + p, d[2 * j + 1]));
                 if (j & 1) *piece(sm.h0, at, T, j >> 1) = make_uint2(f[(j & 3) - 1], f[j & 3]);
             };
 #pragma unroll
@@ -978,14 +978,16 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
                     // h = 1's last chunk meets zeros
                     c = mfma32x32x16(w0p[(k < 2 ? 256 * k : 512 - 128 * h) + 32 * T], xb[k], c);
                     if (T > 0) {
-                        pair0(T - 1, 3 * k);
-                        pair0(T - 1, 3 * k + 1);
-                        if (k < 2) pair0(T - 1, 3 * k + 2);
+                        const uint32_t m = (T - 1) & 2 ? m0.y : m0.x;
+                        pair0(T - 1, 3 * k, m);
+                        pair0(T - 1, 3 * k + 1, m);
+                        if (k < 2) pair0(T - 1, 3 * k + 2, m);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 d = c;
             }
+            const uint32_t m0_3 = m0.y;
             load(rnd + stride);
             uint2 gl[4];  // dL/dlogit (lane & 3; the fourth's sums go unused) of samples 8q + 4h ..
 #pragma unroll
@@ -994,8 +996,16 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
             auto w1 = [&](int k) { return *reinterpret_cast<const uint4*>(w1p + k * kFragPitch); };
             uint4 f1[3] = {w1(0), w1(1)};  // read two steps ahead
             uint32_t r[2];
+            uint4 m1[4];  // the mask words of this lane's samples 8q + 4h ..
             auto pair1 = [&](int T, int j) {
-                r[j & 1] = relu_bf2(d[2 * j], d[2 * j + 1]);
+                if (j == 0 && !(T & 1))
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        m1[q] = *reinterpret_cast<const uint4*>(m1p + GS * (T >> 1) + 8 * q);
+                const uint4& m = m1[j >> 1];
+                const int b = bit1 + 8 * (T & 1);
+                r[j & 1] = pk_bf(keep_if(j & 1 ? m.z : m.x, b, d[2 * j]),
+                                 keep_if(j & 1 ? m.w : m.y, b, d[2 * j + 1]));
                 if (j & 1) dW2[T] = mfma4x4x4(gl[j >> 1].x, gl[j >> 1].y, r[0], r[1], dW2[T]);
             };
 #pragma unroll
@@ -1011,8 +1021,8 @@ __global__ void __launch_bounds__(64 * kBwdWaves) k_mlp_bwd(StepParams P, MlpPac
                     if (T > 0)
                         pair1(T - 1, ks);
                     else if (ks < 4) {  // the last layer-0 tile is k-steps 6 and 7's input
-                        pair0(3, 2 * ks);
-                        pair0(3, 2 * ks + 1);
+                        pair0(3, 2 * ks, m0_3);
+                        pair0(3, 2 * ks + 1, m0_3);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }

@@ -1,12 +1,17 @@
-"""The MLP's ReLU pattern: the order in which the forward sums a pre-activation.
+"""The MLP's ReLU pattern: the order in which the forward sums a pre-activation, and
+the backward's use of the same pattern for its own recomputed activations.
 
-It is the bias, then for every 32 inputs the products with their hi, their mid
+The order is the bias, then for every 32 inputs the products with their hi, their mid
 and their lo bf16 parts, eight inputs at a time.  Weights and inputs are powers of two
 2^10 apart, so a term 2^30 below the sum so far (or below another of its eight) is
 lost and one 2^20 below it kept exactly, whatever the rounding: the order alone
 decides which small terms survive where large ones cancel, and with them the sign.
 A bias gradient is zero exactly where a mask is off for every sample (all samples
 have the same encoding inputs, and the colour's weights are zero).
+
+With recomputed activations r from hi parts and the forward's mask on everywhere,
+dW = sum of r g over samples for the bias gradient's sum of g: r is exact, and the
+products take g in bf16, half an ulp of 2^-8 off.
 """
 import numpy as np
 import pytest
@@ -109,3 +114,35 @@ def test_layer1_order(seed):
                   "w2": _signs(rng, 128, 3) * 2.0 ** -50, "b2": np.zeros(3)})
     print("[case] layer 1, units on:", int((pre > 0).sum()), flush=True)
     np.testing.assert_array_equal(g["b1"] != 0, pre > 0)
+
+
+def test_dw_operands_take_the_forward_pattern():
+    """Units whose pre-activation is 1/2 + 2^-10 .., but -1/2 from the hi parts alone: the
+    forward has them on, and the dW products take the recomputed -1/2.  And units that are
+    off, but 1/2 from the hi parts: no gradient."""
+    rng = np.random.default_rng(3)
+    on = np.arange(128) % 2 == 0
+    w0 = np.zeros((39, 128))
+    w0[12] = np.where(on, 1024.0, -1024.0)           # times V: +-(1024 + 1 + 2^-10)
+    w0[31] = -w0[12]
+    w0[38] = np.where(on, -0.5, 0.5)
+    g = _trainer({"w0": w0, "b0": np.zeros(128), "w1": _signs(rng, 128, 128) * 0.1,
+                  "b1": np.ones(128), "w2": _signs(rng, 128, 3) * 0.1, "b2": np.zeros(3)})
+    np.testing.assert_array_equal(g["b0"] != 0, on)
+    assert np.all(g["w1"][~on] == 0)
+    want = -0.5 * np.broadcast_to(g["b1"], (64, 128))
+    print("[case] dW1", float(np.abs(g["w1"][on] / want - 1).max()), flush=True)
+    assert np.abs(g["b1"]).min() > 0 and np.abs(g["w1"][on] - want).max() <= 2 ** -8 * np.abs(want).max()
+
+    b0 = np.where(np.arange(128) % 4 == 0, V, 1.0)   # H0, exactly
+    w1 = np.zeros((128, 128))
+    w1[0] = np.where(on, 1024.0, -1024.0)            # H0[0] = V, the other two 1
+    w1[1] = -w1[0]
+    w1[2] = np.where(on, -0.5, 0.5)
+    g = _trainer({"w0": np.zeros((39, 128)), "b0": b0, "w1": w1, "b1": np.zeros(128),
+                  "w2": _signs(rng, 128, 3) * 0.1, "b2": np.zeros(3)})
+    np.testing.assert_array_equal(g["b1"] != 0, on)
+    assert np.all(g["w2"][~on] == 0)
+    want = -0.5 * np.broadcast_to(g["b2"], (64, 3))
+    print("[case] dW2", float(np.abs(g["w2"][on] / want - 1).max()), flush=True)
+    assert np.abs(g["b2"]).min() > 0 and np.abs(g["w2"][on] - want).max() <= 2 ** -8 * np.abs(want).max()
