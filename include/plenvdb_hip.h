@@ -264,7 +264,12 @@ typedef struct pvdb_step_desc {
      * rgb = sigmoid(k0) (dvgo.py:72-75,344-346); target then holds k0_dim
      * values per ray and ray_out k0_dim + 1 (rgb, T_last); mlp* are ignored. */
     int32_t k0_dim;
-    void* workspace; /* dev, pvdb_fused_workspace_bytes() bytes, 256-byte aligned */
+    /* dev, pvdb_fused_workspace_bytes() bytes, 256-byte aligned.  A workspace for some
+     * rays, records and leaves serves steps of fewer of any of them (after another
+     * pvdb_fused_init); large batches whose scatter goes by cell take their room
+     * for it out of what pvdb_fused_workspace_bytes() gives for their own sizes, and
+     * scatter by chunks, more slowly, without it */
+    void* workspace;
     int64_t workspace_bytes;
     /* max records (occupancy-kept samples) per step, in [1, 2^31 - 2].  Records
      * past it are dropped: the step then covers the first `capacity` records in

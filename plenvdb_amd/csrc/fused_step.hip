@@ -63,8 +63,9 @@ struct Layout {
         pe, setup, zero;
     size_t xyze, ab, rgb, adj, xrow, relu, grad;
     size_t touched, dw_part, fwd, w2, w0;
+    size_t base;  // the bytes that a step needs
     size_t cell_count, cell_leaf, cell_part, cell_nparts, cell_at, cell_order;
-    size_t bytes;
+    size_t bytes;  // with room for the scatter by cell
 };
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
@@ -81,6 +82,9 @@ bool scatter_by_cell(int64_t records, int64_t nleaf) {
     return nleaf > 0 && records >= kCellMinCapacity && records / nleaf >= kCellMinPerLeaf;
 }
 
+// What a step needs grows with each of its sizes, so a workspace for some rays, records
+// and leaves serves every step of no more of them; the scatter by cell's part, which
+// fewer leaves can ask for, lies behind it and is used where it fits.
 Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
     const int64_t capacity = (records + 31) & ~int64_t(31);  // whole groups of the forward MLP
     Layout L;
@@ -93,7 +97,7 @@ Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
     L.count = take(4 * n_rays);
     L.offset = take(4 * n_rays);
     L.total = take(4);
-    L.group = take(8 * (n_rays <= kGroupedRays ? n_rays : 0));
+    L.group = take(8 * (n_rays <= kGroupedRays ? n_rays : kGroupedRays));
     L.t_last = take(4 * n_rays);
     L.ray_out = take(16 * n_rays);
     L.ray_grad = take(16 * n_rays);
@@ -117,6 +121,7 @@ Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
     L.fwd = take(2 * kFwdImage);
     L.w2 = take(2 * 128 * 32);
     L.w0 = take(2 * 16 * 128);
+    L.base = o;
     if (scatter_by_cell(records, nleaf)) {
         L.cell_count = take(4 * (size_t)kLeafCells * nleaf);
         L.cell_leaf = take(4 * (nleaf + 1));
@@ -129,6 +134,14 @@ Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
     }
     L.bytes = o;
     return L;
+}
+
+Layout layout_of(const pvdb_step_desc* d, const TopoView& t) {
+    return layout_for(d->n_rays, d->capacity, t.nleaf);
+}
+
+bool by_cell(const pvdb_step_desc* d, const TopoView& t, const Layout& L) {
+    return scatter_by_cell(d->capacity, t.nleaf) && d->workspace_bytes >= (int64_t)L.bytes;
 }
 
 __global__ void k_fill_u8(uint8_t* p, int64_t n, uint8_t v) {
@@ -487,12 +500,12 @@ int pvdb_fused_init(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
     PVDB_CHECK_ARG(d && d->workspace, "null descriptor or workspace");
     PVDB_CHECK_ARG(aligned(d->workspace, 256), "workspace must be 256-byte aligned");
     const TopoView t = view_of(topo);
-    const Layout L = layout_for(d->n_rays, d->capacity, t.nleaf);
-    PVDB_CHECK_ARG(d->workspace_bytes >= (int64_t)L.bytes, "workspace too small");
+    const Layout L = layout_of(d, t);
+    PVDB_CHECK_ARG(d->workspace_bytes >= (int64_t)L.base, "workspace too small");
     uint8_t* ws = reinterpret_cast<uint8_t*>(d->workspace);
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_fill_u8, dim3(pvdb_blocks(L.bytes, 256)), dim3(256), 0, s, ws,
-                       (int64_t)L.bytes, (uint8_t)0);
+    hipLaunchKernelGGL(k_fill_u8, dim3(pvdb_blocks(L.base, 256)), dim3(256), 0, s, ws,
+                       (int64_t)L.base, (uint8_t)0);
     PVDB_LAUNCHED("k_fill_u8");
     return PVDB_OK;
 }
@@ -551,8 +564,8 @@ int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
     PVDB_CHECK_ARG(aligned(d->ray_out, direct ? 4 : 16),
                    "ray_out must be 16-byte aligned (4-byte without the MLP)");
     const TopoView t = view_of(topo);
-    const Layout L = layout_for(d->n_rays, d->capacity, t.nleaf);
-    PVDB_CHECK_ARG(d->workspace && d->workspace_bytes >= (int64_t)L.bytes, "workspace too small");
+    const Layout L = layout_of(d, t);
+    PVDB_CHECK_ARG(d->workspace && d->workspace_bytes >= (int64_t)L.base, "workspace too small");
     uint8_t* ws = reinterpret_cast<uint8_t*>(d->workspace);
     hipStream_t s = (hipStream_t)stream;
 
@@ -713,7 +726,7 @@ int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
                            d->step_size_mlp, d->eps,   d->beta0, d->beta1};
         const ReduceArgs red{dw_part, grid_bwd, d->mlp_grad, adam, kReduceBlocks,
                              R.ray_loss, R.loss, d->n_rays};
-        if (scatter_by_cell(d->capacity, t.nleaf)) {
+        if (by_cell(d, t, L)) {
             CellBins B;
             B.count = reinterpret_cast<int32_t*>(ws + L.cell_count);
             B.leaf = reinterpret_cast<int32_t*>(ws + L.cell_leaf);
@@ -744,7 +757,7 @@ int pvdb_fused_records(const pvdb_topology* topo, const pvdb_step_desc* d, void*
         return PVDB_EHANDLE;
     }
     PVDB_CHECK_ARG(d && d->workspace, "null descriptor or workspace");
-    const Layout L = layout_for(d->n_rays, d->capacity, view_of(topo).nleaf);
+    const Layout L = layout_of(d, view_of(topo));
     uint8_t* ws = reinterpret_cast<uint8_t*>(d->workspace);
     if (xyze) *xyze = ws + L.xyze;
     if (ab) *ab = ws + L.ab;
