@@ -325,8 +325,11 @@ int pvdb_fused_set_scalars(float* adam_scalars, float stepsz_density, float step
                            float step_size_mlp, void* stream);
 /* The default launch shapes (pvdb_step_desc.launch) on the current device. */
 int pvdb_fused_launch_defaults(int32_t* launch4);
-/* Workspace bytes for n_rays rays, `capacity` records and nleaf leaves (-1 on bad sizes). */
+/* Workspace bytes for n_rays rays, `capacity` records and nleaf leaves (-1 on bad sizes);
+ * _for: of the model with that k0_dim (0, the MLP's, needs the most). */
 int64_t pvdb_fused_workspace_bytes(int64_t n_rays, int64_t capacity, int64_t nleaf);
+int64_t pvdb_fused_workspace_bytes_for(int64_t n_rays, int64_t capacity, int64_t nleaf,
+                                       int32_t k0_dim);
 /* Clears the workspace (touched-leaf flags, buffers); call once after allocating it. */
 int pvdb_fused_init(const pvdb_topology* topo, const pvdb_step_desc* desc, void* stream);
 int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* desc, void* stream);

@@ -78,14 +78,15 @@ size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 // (7.7M) 471 / 487; 65,536 in 1350 (21M, 16k a leaf) 828 / 839; 65,536 in 1984 (51M, 25k)
 // 1055 / 1060; 40,000 in 600 (15M, 26k) 1401 / 1230; 65,536 in 600 (25M, 42k) 1305 / 1169;
 // 131,072 in 1984 (97M, 49k) 4250 / 3560.
-bool scatter_by_cell(int64_t records, int64_t nleaf) {
-    return nleaf > 0 && records >= kCellMinCapacity && records / nleaf >= kCellMinPerLeaf;
+bool scatter_by_cell(int64_t records, int64_t nleaf, int32_t k0_dim) {
+    return k0_dim == 0 && nleaf > 0 && records >= kCellMinCapacity &&
+           records / nleaf >= kCellMinPerLeaf;
 }
 
 // What a step needs grows with each of its sizes, so a workspace for some rays, records
 // and leaves serves every step of no more of them; the scatter by cell's part, which
 // fewer leaves can ask for, lies behind it and is used where it fits.
-Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
+Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf, int32_t k0_dim) {
     const int64_t capacity = (records + 31) & ~int64_t(31);  // whole groups of the forward MLP
     Layout L;
     size_t o = 0;
@@ -122,7 +123,7 @@ Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
     L.w2 = take(2 * 128 * 32);
     L.w0 = take(2 * 16 * 128);
     L.base = o;
-    if (scatter_by_cell(records, nleaf)) {
+    if (scatter_by_cell(records, nleaf, k0_dim)) {
         L.cell_count = take(4 * (size_t)kLeafCells * nleaf);
         L.cell_leaf = take(4 * (nleaf + 1));
         L.cell_part = take(16 * cell_parts(capacity, nleaf));
@@ -137,11 +138,11 @@ Layout layout_for(int64_t n_rays, int64_t records, int64_t nleaf) {
 }
 
 Layout layout_of(const pvdb_step_desc* d, const TopoView& t) {
-    return layout_for(d->n_rays, d->capacity, t.nleaf);
+    return layout_for(d->n_rays, d->capacity, t.nleaf, d->k0_dim);
 }
 
 bool by_cell(const pvdb_step_desc* d, const TopoView& t, const Layout& L) {
-    return scatter_by_cell(d->capacity, t.nleaf) && d->workspace_bytes >= (int64_t)L.bytes;
+    return scatter_by_cell(d->capacity, t.nleaf, d->k0_dim) && d->workspace_bytes >= (int64_t)L.bytes;
 }
 
 __global__ void k_fill_u8(uint8_t* p, int64_t n, uint8_t v) {
@@ -487,9 +488,14 @@ int pvdb_fused_timing(int32_t enable, double* total_ms, int32_t* calls, int32_t 
 
 const char* pvdb_fused_stage_name(int32_t i) { return (i >= 0 && i < kStages) ? kStageNames[i] : ""; }
 
-int64_t pvdb_fused_workspace_bytes(int64_t n_rays, int64_t capacity, int64_t nleaf) {
+int64_t pvdb_fused_workspace_bytes_for(int64_t n_rays, int64_t capacity, int64_t nleaf,
+                                       int32_t k0_dim) {
     if (n_rays < 0 || capacity < 0 || nleaf < 0) return -1;
-    return (int64_t)layout_for(n_rays, capacity, nleaf).bytes;
+    return (int64_t)layout_for(n_rays, capacity, nleaf, k0_dim).bytes;
+}
+
+int64_t pvdb_fused_workspace_bytes(int64_t n_rays, int64_t capacity, int64_t nleaf) {
+    return pvdb_fused_workspace_bytes_for(n_rays, capacity, nleaf, 0);
 }
 
 int pvdb_fused_init(const pvdb_topology* topo, const pvdb_step_desc* d, void* stream) {

@@ -57,12 +57,12 @@ lib.EXTRA_SIGS.update({
 })
 
 
-def _workspace_bytes(n_rays: int, capacity: int, nleaf: int) -> int:
+def _workspace_bytes(n_rays: int, capacity: int, nleaf: int, k0_dim: int = 0) -> int:
     L = lib.load()
-    fn = L.pvdb_fused_workspace_bytes
+    fn = L.pvdb_fused_workspace_bytes_for
     fn.restype = C.c_int64
-    fn.argtypes = [C.c_int64, C.c_int64, C.c_int64]
-    b = int(fn(n_rays, capacity, nleaf))
+    fn.argtypes = [C.c_int64, C.c_int64, C.c_int64, C.c_int32]
+    b = int(fn(n_rays, capacity, nleaf, k0_dim))
     if b < 0:
         raise RuntimeError("bad workspace sizes")
     return b
@@ -162,7 +162,7 @@ class FusedTrainer:
         if capacity is None:
             capacity = self._capacity_bound()
         self.capacity = int(capacity)
-        self.ws_bytes = _workspace_bytes(self.n_rays, self.capacity, self.topo.nleaf)
+        self.ws_bytes = _workspace_bytes(self.n_rays, self.capacity, self.topo.nleaf, self.k0_dim)
         self.workspace = torch.empty(self.ws_bytes, dtype=torch.uint8, device=dev)
         self.ray_out = torch.zeros(self.n_rays, self.n_out + 1, device=dev)
         self.loss = torch.zeros(1, device=dev)

@@ -53,3 +53,10 @@ def test_a_larger_leaf_sets_workspace_serves_a_smaller_one():
         a, b = (getattr(t, k).cpu().numpy() for t in (tr, ch))
         assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b), k
         np.testing.assert_array_equal(a != 0, b != 0)
+
+
+def test_models_without_the_mlp_reserve_no_cells():
+    from plenvdb_amd.fused import _workspace_bytes
+
+    sizes = (8192, 25 << 20, 600)
+    assert _workspace_bytes(*sizes, 3) == _workspace_bytes(*sizes, 12) < _workspace_bytes(*sizes, 0) - (12 * 25 << 20)
