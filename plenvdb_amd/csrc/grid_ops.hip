@@ -287,8 +287,9 @@ __global__ void k_set_by_mask(TopoView t, float* __restrict__ vals,
 // contiguous: a thread per slot wrote its row in C stores 4 C bytes apart.  309k slots,
 // 12 channels: 16.5 -> 5.9 us.
 template <int V>
-__global__ void __launch_bounds__(256) k_zero_active(TopoView t, float* __restrict__ grad, int C) {
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(256) k_zero_active(TopoView t, float* __restrict__ grad, int C,
+                                                     int64_t q0) {
+    const int64_t q = q0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t s = q / (C / V);
     if (s >= t.nleaf * 512 || !slot_active(t, s)) return;
     if constexpr (V == 4)
@@ -480,8 +481,12 @@ void launch_bwd(const TopoView& t, float* grad, int cdyn, const float* xs, const
                 const float* zs, const float* g, int64_t n, hipStream_t s) {
     if constexpr (C > 0) {
         if (t.nleaf < (int64_t(1) << 23) - 1) {  // every slot below the hash's empty key
-            hipLaunchKernelGGL((k_tri_bwd_agg<C, ORDER>), dim3(pvdb_blocks(n, kBwdPoints)),
-                               dim3(256), 0, s, t, grad, xs, ys, zs, g, n);
+            const int64_t most = pvdb_launch_items(kBwdPoints, 256);
+            for (int64_t p = 0; p < n; p += most) {
+                const int64_t m = n - p < most ? n - p : most;
+                hipLaunchKernelGGL((k_tri_bwd_agg<C, ORDER>), dim3(pvdb_blocks(m, kBwdPoints)),
+                                   dim3(256), 0, s, t, grad, xs + p, ys + p, zs + p, g + C * p, m);
+            }
             return;
         }
     }
@@ -637,9 +642,13 @@ int pvdb_zero_active(const pvdb_topology* topo, float* grad, int32_t channels, v
     if (t.nleaf == 0) return PVDB_OK;
     const bool vec4 = channels % 4 == 0 && reinterpret_cast<uintptr_t>(grad) % 16 == 0;
     const int64_t n = t.nleaf * 512 * (vec4 ? channels / 4 : channels);
-    hipLaunchKernelGGL(vec4 ? k_zero_active<4> : k_zero_active<1>, dim3(pvdb_blocks(n, 256)),
-                       dim3(256), 0, (hipStream_t)stream, t, grad, channels);
-    PVDB_LAUNCHED("k_zero_active");
+    const int64_t most = pvdb_launch_items(256, 256);
+    for (int64_t q = 0; q < n; q += most) {
+        const int64_t m = n - q < most ? n - q : most;
+        hipLaunchKernelGGL(vec4 ? k_zero_active<4> : k_zero_active<1>, dim3(pvdb_blocks(m, 256)),
+                           dim3(256), 0, (hipStream_t)stream, t, grad, channels, q);
+        PVDB_LAUNCHED("k_zero_active");
+    }
     return PVDB_OK;
 }
 

@@ -147,6 +147,12 @@ int hip_fail(hipError_t e, const char* what);
         if (e_ != hipSuccess) return pvdb::hip_fail(e_, "launch " name); \
     } while (0)
 
+// Items that one launch can take, `per_block` of them to a workgroup of `threads`
+// threads: a grid of 2^32 work items or more runs its size modulo 2^32, without an error.
+static inline int64_t pvdb_launch_items(int per_block, int threads) {
+    return ((int64_t(1) << 32) / threads - 1) * per_block;
+}
+
 static inline unsigned pvdb_blocks(int64_t n, int threads) {
     int64_t b = (n + threads - 1) / threads;
     return (unsigned)(b < 1 ? 1 : b);

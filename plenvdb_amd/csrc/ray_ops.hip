@@ -460,10 +460,14 @@ int pvdb_alpha2weight(const float* alpha, int64_t n_rays, float* weight, float* 
     PVDB_CHECK_ARG(n_rays >= 0, "n_rays must be >= 0");
     if (n_rays == 0) return PVDB_OK;
     PVDB_CHECK_ARG(alpha && weight && T && alphainv_last && i_start && i_end, "null pointer");
-    hipLaunchKernelGGL(k_alpha2weight, dim3(pvdb_blocks(n_rays, 4)), dim3(256), 0,
-                       (hipStream_t)stream, alpha, n_rays, weight, T, alphainv_last, i_start,
-                       i_end);
-    PVDB_LAUNCHED("k_alpha2weight");
+    const int64_t most = pvdb_launch_items(4, 256);
+    for (int64_t r = 0; r < n_rays; r += most) {
+        const int64_t n = n_rays - r < most ? n_rays - r : most;
+        hipLaunchKernelGGL(k_alpha2weight, dim3(pvdb_blocks(n, 4)), dim3(256), 0,
+                           (hipStream_t)stream, alpha, n, weight, T, alphainv_last + r, i_start + r,
+                           i_end + r);
+        PVDB_LAUNCHED("k_alpha2weight");
+    }
     return PVDB_OK;
 }
 
@@ -476,10 +480,14 @@ int pvdb_alpha2weight_bwd(const float* alpha, const float* weight, const float* 
     PVDB_CHECK_ARG(alpha && weight && T && alphainv_last && i_start && i_end && grad_weights &&
                        grad_last && grad_alpha,
                    "null pointer");
-    hipLaunchKernelGGL(k_alpha2weight_bwd, dim3(pvdb_blocks(n_rays, 4)), dim3(256), 0,
-                       (hipStream_t)stream, alpha, weight, T, alphainv_last, i_start, i_end,
-                       n_rays, grad_weights, grad_last, grad_alpha);
-    PVDB_LAUNCHED("k_alpha2weight_bwd");
+    const int64_t most = pvdb_launch_items(4, 256);
+    for (int64_t r = 0; r < n_rays; r += most) {
+        const int64_t n = n_rays - r < most ? n_rays - r : most;
+        hipLaunchKernelGGL(k_alpha2weight_bwd, dim3(pvdb_blocks(n, 4)), dim3(256), 0,
+                           (hipStream_t)stream, alpha, weight, T, alphainv_last + r, i_start + r,
+                           i_end + r, n, grad_weights, grad_last + r, grad_alpha);
+        PVDB_LAUNCHED("k_alpha2weight_bwd");
+    }
     return PVDB_OK;
 }
 
