@@ -510,9 +510,12 @@ int pvdb_fused_init(const pvdb_topology* topo, const pvdb_step_desc* d, void* st
     PVDB_CHECK_ARG(d->workspace_bytes >= (int64_t)L.base, "workspace too small");
     uint8_t* ws = reinterpret_cast<uint8_t*>(d->workspace);
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_fill_u8, dim3(pvdb_blocks(L.base, 256)), dim3(256), 0, s, ws,
-                       (int64_t)L.base, (uint8_t)0);
-    PVDB_LAUNCHED("k_fill_u8");
+    const int64_t bytes = (int64_t)L.base, most = pvdb_launch_items(256, 256);
+    for (int64_t b = 0; b < bytes; b += most) {
+        const int64_t n = bytes - b < most ? bytes - b : most;
+        hipLaunchKernelGGL(k_fill_u8, dim3(pvdb_blocks(n, 256)), dim3(256), 0, s, ws + b, n, (uint8_t)0);
+        PVDB_LAUNCHED("k_fill_u8");
+    }
     return PVDB_OK;
 }
 

@@ -54,3 +54,19 @@ def test_zero_active():
     g = torch.full((topo.nslots * ch,), 1.0, device="cuda")
     lib.call("pvdb_zero_active", topo.handle, lib.ptr(g), ch, lib.stream())
     assert not bool(g.any())
+
+
+def test_workspace_init():
+    """A thread to a byte: a workspace of 6 GB."""
+    import ctypes as C
+
+    from plenvdb_amd import lib, scenes
+    from plenvdb_amd.fused import FusedTrainer, _workspace_bytes
+
+    tr = FusedTrainer(scenes.make_scene("c2", n_rays=16))
+    tr.desc.capacity = 26_000_000
+    n = _workspace_bytes(16, tr.desc.capacity, tr.topo.nleaf, 12)  # without room for cells
+    ws = torch.full((n,), 7, dtype=torch.uint8, device="cuda")
+    tr.desc.workspace, tr.desc.workspace_bytes = ws.data_ptr(), n
+    lib.call("pvdb_fused_init", tr.topo.handle, C.byref(tr.desc), lib.stream())
+    assert n > 1 << 32 and not bool(ws.any())
