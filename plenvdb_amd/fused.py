@@ -243,7 +243,10 @@ class FusedTrainer:
 
     def _next_step_sizes(self) -> list:
         """Advances the step counter; the Adam step sizes of this step (grid,
-        grid, MLP), in the descriptor."""
+        grid, MLP), in the descriptor.  Refuses a caller's own capture, with
+        nothing changed."""
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("a step's sizes change with every call: capture it with capture_graph()")
         self.step_count += 1
         t = self.step_count
         sz = [self._stepsz(self.lr_grid, t), self._stepsz(self.lr_grid, t),
@@ -256,8 +259,6 @@ class FusedTrainer:
         writing them to the device first costs a launch, and a copy from the
         host waits for the step before (8192 rays, replayed: 237 -> 229 us a step;
         1021 rays, launched: 106 -> 85 us)."""
-        if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError("a step's sizes change with every call: capture it with capture_graph()")
         self.desc.do_adam = mode
         self.desc.adam_scalars = None
         try:
