@@ -287,9 +287,10 @@ typedef struct pvdb_step_desc {
     const float* adam_scalars;
     /* launch shapes, 0 = built-in default (results do not depend on them):
      * [0] forward-MLP workgroups, [1] scatter workgroups, [2] scatter records
-     * per chunk (32 or 64), [3] rays per workgroup of the wave-per-ray kernels
-     * (marches and composite: 1, 2, 4 or 8); pvdb_fused_launch_defaults()
-     * fills the defaults for this device */
+     * per chunk (32 or 64; both of the scatter by chunks only,
+     * pvdb_fused_scatters_by_cell), [3] rays per workgroup of the wave-per-ray
+     * kernels (marches and composite: 1, 2, 4 or 8);
+     * pvdb_fused_launch_defaults() fills the defaults for this device */
     int32_t launch[4];
     /* loss weights of plenvdb/run.py:551-574 (cfg_train.weight_*): the MSE
      * term (1.0 in every configuration), the background entropy of T_last
@@ -330,6 +331,9 @@ int pvdb_fused_launch_defaults(int32_t* launch4);
 int64_t pvdb_fused_workspace_bytes(int64_t n_rays, int64_t capacity, int64_t nleaf);
 int64_t pvdb_fused_workspace_bytes_for(int64_t n_rays, int64_t capacity, int64_t nleaf,
                                        int32_t k0_dim);
+/* 1 when a step of these sizes, model and workspace scatters its grid gradients by cell,
+ * 0 when by chunks of consecutive records. */
+int pvdb_fused_scatters_by_cell(const pvdb_topology* topo, const pvdb_step_desc* desc);
 /* Clears the workspace (touched-leaf flags, buffers); call once after allocating it. */
 int pvdb_fused_init(const pvdb_topology* topo, const pvdb_step_desc* desc, void* stream);
 int pvdb_fused_step(const pvdb_topology* topo, const pvdb_step_desc* desc, void* stream);

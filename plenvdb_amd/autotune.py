@@ -3,8 +3,9 @@
 Four launch choices of `pvdb_fused_step` are free (`pvdb_step_desc.launch`):
 the forward MLP's workgroup count, the scatter's workgroup count, the
 scatter's records per chunk (32 or 64) and the rays (wavefronts) per workgroup
-of the wave-per-ray kernels (the two marches and the composite).  None changes
-the computed values beyond the order of the scatter's float atomics.  `tune`
+of the wave-per-ray kernels (the two marches and the composite).  A step that
+scatters by cell (large batches) has two: the scatter's choices do not apply to it.
+None changes the computed values beyond the order of the scatter's float atomics.  `tune`
 picks them per device and workload by coordinate descent: each candidate is
 timed on the stages it affects (the step's own HIP-event stage timers, several
 forward+backward passes per candidate) with the other choices held at their
@@ -81,6 +82,18 @@ def _stage_ms(tr, stages: tuple, reps: int) -> float:
     return sum(st[s][0] / max(st[s][1], 1) for s in stages)
 
 
+def choices(tr) -> tuple:
+    """The choices that the trainer's step has, in the order of the tuning: the chunk
+    length before the scatter's workgroup count; a model without the MLP has no
+    forward-MLP launch to shape, a step that scatters by cell no chunks."""
+    return (() if tr.k0_dim else (0,)) + (() if tr.scatters_by_cell() else (2, 1)) + (3,)
+
+
+def _named(tr, launch: list[int]) -> dict:
+    skip = (1, 2) if tr.scatters_by_cell() else ()
+    return {NAMES[i]: launch[i] for i in NAMES if i not in skip}
+
+
 def apply(tr, launch: list[int]) -> None:
     for i in range(4):
         tr.desc.launch[i] = int(launch[i])
@@ -99,13 +112,11 @@ def tune(tr, reps: int = 3, force: bool = False) -> dict:
                 _cache[key] = [int(v) for v in hit]
         if key in _cache:
             apply(tr, _cache[key])
-            return {"launch": {NAMES[i]: _cache[key][i] for i in NAMES}, "source": "cache"}
+            return {"launch": _named(tr, _cache[key]), "source": "cache"}
     best = defaults()
     apply(tr, best)
     timings = {}
-    # the chunk length before the scatter's workgroup count; a model without the
-    # MLP has no forward-MLP launch to shape
-    for idx in ((2, 1, 3) if tr.k0_dim else (0, 2, 1, 3)):
+    for idx in choices(tr):
         t = {}
         for v in CANDIDATES[idx]:
             tr.desc.launch[idx] = v
@@ -116,5 +127,5 @@ def tune(tr, reps: int = 3, force: bool = False) -> dict:
     tr.zero_grad()
     _cache[key] = list(best)
     _save_file({key: list(best)})
-    return {"launch": {NAMES[i]: best[i] for i in NAMES}, "source": "tuned",
+    return {"launch": _named(tr, best), "source": "tuned",
             "stage_ms": timings}

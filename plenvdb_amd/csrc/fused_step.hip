@@ -498,6 +498,12 @@ int64_t pvdb_fused_workspace_bytes(int64_t n_rays, int64_t capacity, int64_t nle
     return pvdb_fused_workspace_bytes_for(n_rays, capacity, nleaf, 0);
 }
 
+int pvdb_fused_scatters_by_cell(const pvdb_topology* topo, const pvdb_step_desc* d) {
+    if (!topo || !d) return 0;
+    const TopoView t = view_of(topo);
+    return by_cell(d, t, layout_of(d, t)) ? 1 : 0;
+}
+
 int pvdb_fused_init(const pvdb_topology* topo, const pvdb_step_desc* d, void* stream) {
     if (!topo) {
         pvdb::set_error("null topology");

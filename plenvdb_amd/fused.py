@@ -254,6 +254,13 @@ class FusedTrainer:
         self.desc.stepsz_density, self.desc.stepsz_color, self.desc.step_size_mlp = sz
         return sz
 
+    def scatters_by_cell(self) -> bool:
+        """Whether the step scatters its grid gradients by cell (large batches with the
+        MLP) instead of by chunks of consecutive records."""
+        fn = lib.load().pvdb_fused_scatters_by_cell
+        fn.restype, fn.argtypes = C.c_int, [C.c_void_p, C.POINTER(StepDesc)]
+        return bool(fn(self.topo.handle, C.byref(self.desc)))
+
     def _launch_adam(self, mode: int) -> None:
         """The step with do_adam = `mode`, launched with the step sizes by value:
         writing them to the device first costs a launch, and a copy from the
