@@ -146,7 +146,8 @@ __global__ void __launch_bounds__(1024) k_leaf_scan(CellBins B, RayBuffers R, in
                                                     int nleaf) {
     __shared__ int wsum[16], psum[16];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    // about 1024 parts in all: fewer leave CUs idle, and each adds up to 1000 rows
+    // about 1024 parts in all: fewer leave CUs idle, and each adds up to 1000 rows (more
+    // of them above 8.4M records, at 8192 a part)
     const int total = (int)min((int64_t)R.total[0], capacity);
     const int per = min(max(total / 1024, kMinPart), 8 * kMinPart);
     int carry = 0, parts0 = 0;  // below 2^31: the capacity is
