@@ -242,9 +242,9 @@ def bench_batched(args, scene):
 # x1.0); profiles/pmc_traffic_c2_train_c5_render.md holds the runs.
 TRAFFIC_SOURCE = "profiles/pmc_traffic_c2_train_c5_render.md"
 MEASURED_TRAFFIC_MB = {
-    "c2": {"mlp_bwd": 63.63, "scatter": 85.98, "mlp_fwd": 71.10, "ray_march": 12.77,
+    "c2": {"mlp_bwd": 63.64, "scatter": 85.97, "mlp_fwd": 71.14, "ray_march": 12.77,
            "composite": 13.63, "adam": 108.45, "ray_count": 4.38},
-    "c5": {"render_mlp": 1392.15},
+    "c5": {"render_mlp": 1399.87},
 }
 
 
@@ -260,7 +260,7 @@ def stage_models(r):
         # encoding rows and 32-byte set-ups out; the MLP parameters packed to
         # bf16 and the MLP gradient zeroed by the same launch
         "ray_count": ("hbm", N * (12 + 12 + 4 + 12 + 168 + 32) + S * 2
-                      + P * 4 + 2 * (25104 + 16 * 128 + 128 * 32) + P * 4),
+                      + P * 4 + 2 * (25096 + 16 * 128 + 128 * 32) + P * 4),
         # ray set-ups + offsets and the kept step indices in, 24-byte records
         # out (xyze, alpha + flags), distinct density voxels once
         "ray_march": ("hbm", N * (32 + 8) + S * (2 + 24) + ua * 4),

@@ -380,7 +380,9 @@ typedef struct pvdb_render_desc {
     int32_t H, W, inverse_y;
     float near_, stepdist, act_shift, interval, fast_color_thres, bg, t_stop;
     int32_t payload_f32;   /* payload slots hold fp32 (64 B) instead of fp16 (32 B) */
-    const void* payload;   /* dev, pvdb_render_payload_bytes() bytes */
+    /* dev, pvdb_render_payload_bytes() bytes: 32 B a slot in fp16 (64 in fp32) and the
+     * marches' density cells, 11.7 kB a leaf (23.3), 0.7 times as much again */
+    const void* payload;
     const void* weights;   /* dev, pvdb_render_weights_bytes() bytes */
     float* out;            /* dev [H*W*3] (output_an_image layout) */
     /* dev [3] or NULL: first-march density gathers, written samples, records the

@@ -91,8 +91,8 @@ __device__ __forceinline__ bf16x8 as_bf8(const uint4& v) { return __builtin_bit_
 //
 // Measured against four wavefronts that shared a group (32 hidden features each,
 // activations exchanged through LDS, three barriers a group): 7.80M records with
-// bf16 colour 2029 -> 982 us, 190k with fp32 colour 61.4 -> 36.8 us; 24k, one
-// group to a wavefront, 13.8 -> 14.8 us.  On 16x16x32 MFMAs 1204 us.  With the
+// bf16 colour 2029 -> 958 us, 190k with fp32 colour 61.4 -> 37.5 us; 24k, one
+// group to a wavefront, 13.8 -> 15.1 us.  On 16x16x32 MFMAs 1204 us.  With the
 // gather in the march (features through memory) 900 us, and the march 485 us
 // instead of 224.
 constexpr int kFwdWaves = 4;
@@ -542,16 +542,17 @@ __global__ void __launch_bounds__(64 * kFwdWaves, 2)
 // (four rows x 32 features to a wavefront half) meet in a bank.
 //
 // What bounds it: a round is 180 MFMAs of 32 cycles per SIMD and about as many
-// cycles of vector work (1200 instructions of 4), which the two wavefronts overlap
+// cycles of vector work (1400 instructions of 4), which the two wavefronts overlap
 // in part, and 40% of the time in the CU's LDS.
 //
 // Measured against eight wavefronts that shared one group (16 hidden features
 // each, every product's operands through LDS on 16x16x32 MFMAs): 7.80M records
-// 2632 -> 1175 us, 190k 98.2 -> 49.2 us, 24k 25.0 -> 14.3 us.  On the way: tiles
-// split after their MFMAs instead of between the next one's 1228 us; db1 summed
-// over lanes at each round (32 registers fewer, three instructions a pair more) and
-// the stores' and loads' addresses formed each time 1350 us; spilling registers
-// 2386 us.
+// 2632 -> 1232 us, 190k 98.2 -> 53.0 us, 24k 25.0 -> 15.0 us.  With relu of the
+// recomputed activations in place of the forward's masks, which is not the same,
+// 1144, 49.2 and 14.4 us; and at 7.80M records tiles split after their MFMAs instead
+// of between the next one's cost 53 us more, db1 summed over lanes at each round (32
+// registers fewer, three instructions a pair more) with the stores' and loads'
+// addresses formed each time 175 us.
 constexpr int kBwdPairs = 4;                   // wavefront pairs, a group each
 constexpr int kBwdWaves = 2 * kBwdPairs;
 constexpr int kRoundRec = kBwdPairs * GS;      // records of a round

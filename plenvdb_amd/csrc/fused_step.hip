@@ -76,7 +76,7 @@ size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 // scenes keep a tenth of it or less).  Whole steps, us, by chunks / by cells: 8192 rays
 // in 600 leaves (capacity 3.2M) 241 / 272; 20,000 in 86 (2.6M) 166 / 205; 20,000 in 600
 // (7.7M) 471 / 487; 65,536 in 1350 (21M, 16k a leaf) 828 / 839; 65,536 in 1984 (51M, 25k)
-// 1055 / 1060; 40,000 in 600 (15M, 26k) 1401 / 1230; 65,536 in 600 (25M, 42k) 1305 / 1169;
+// 1055 / 1060 (as good as equal: the line); 40,000 in 600 (15M, 26k) 1401 / 1230; 65,536 in 600 (25M, 42k) 1305 / 1169;
 // 131,072 in 1984 (97M, 49k) 4250 / 3560.
 bool scatter_by_cell(int64_t records, int64_t nleaf, int32_t k0_dim) {
     return k0_dim == 0 && nleaf > 0 && records >= kCellMinCapacity &&
