@@ -155,17 +155,47 @@ __global__ void k_segment_bounds(const int64_t* __restrict__ ray_id, int64_t n,
 }
 
 // alpha2weight (render_utils_kernel.cu:576-603): float T_cum times the double
-// (1. - alpha), stop after the first T < 1e-3.  A wavefront per ray: its lanes load
-// and store 64 samples together, and all of them run the running product (the
-// same operations, sample by sample) on values read from a lane, so the chain waits
-// for arithmetic only; a thread per ray waited for memory at each of its samples, on
-// a fraction of the chip.  8191 rays, 200k samples: 38.0 -> 21.0 us.
+// (1. - alpha), stop after the first T < 1e-3.  A thread per ray, for many rays: a
+// wavefront per ray (below) starts 64 times the wavefronts and makes each sample's
+// product 64 times over.
 __global__ void __launch_bounds__(256) k_alpha2weight(const float* __restrict__ alpha,
                                                       int64_t n_rays, float* __restrict__ w,
                                                       float* __restrict__ T,
                                                       float* __restrict__ t_last,
                                                       const int64_t* __restrict__ i_start,
                                                       int64_t* __restrict__ i_end) {
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r >= n_rays) return;
+    const int64_t is = i_start[r], ie = i_end[r];
+    float Tc = 1.f;
+    int64_t end = is > ie ? is : ie;  // an empty ray's end is its start
+    for (int64_t i = is; i < end; ++i) {
+        const float a = alpha[i];
+        T[i] = Tc;
+        w[i] = Tc * a;
+        Tc = (float)((double)Tc * (1.0 - (double)a));
+        if ((double)Tc < 1e-3) end = i + 1;
+    }
+    i_end[r] = end;
+    t_last[r] = Tc;
+}
+
+// The same, a wavefront per ray, for few rays: its lanes load and store 64 samples
+// together, and all of them run the running product (the same operations, sample by
+// sample) on values read from a lane, so the chain waits for arithmetic only; a thread
+// per ray waits for memory at each of its samples, on a fraction of the chip.
+// 8191 rays, 200k samples, nothing cached: 38.0 -> 21.0 us.
+//
+// Where the line lies (us, a thread / a wavefront per ray, at 0.3, 25 and 120 samples a
+// ray): 4096 rays 2.5 / 3.0, 10.4 / 7.4, 41 / 23; 8192 2.4 / 3.2, 10.6 / 9.6, 43 / 33; 12,288
+// 2.5 / 3.9, 11.4 / 12.1, 44 / 42; 65,536 2.6 / 11.1, 17 / 40, 102 / 159.
+constexpr int64_t kWaveRays = 8192;
+__global__ void __launch_bounds__(256) k_alpha2weight_wave(const float* __restrict__ alpha,
+                                                           int64_t n_rays, float* __restrict__ w,
+                                                           float* __restrict__ T,
+                                                           float* __restrict__ t_last,
+                                                           const int64_t* __restrict__ i_start,
+                                                           int64_t* __restrict__ i_end) {
     const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (r >= n_rays) return;  // uniform over the wave
     const int lane = (int)(threadIdx.x & 63);
@@ -197,10 +227,29 @@ __global__ void __launch_bounds__(256) k_alpha2weight(const float* __restrict__ 
     }
 }
 
-// alpha2weight backward (render_utils_kernel.cu:653-676), a wavefront per ray as above:
-// the running sum sample by sample, each sample's gradient in its own lane.
-// 4096 rays, 100k samples: 61.8 -> 12.7 us.
+// alpha2weight backward (render_utils_kernel.cu:653-676), a thread per ray.
 __global__ void __launch_bounds__(256) k_alpha2weight_bwd(
+    const float* __restrict__ alpha, const float* __restrict__ w, const float* __restrict__ T,
+    const float* __restrict__ t_last, const int64_t* __restrict__ i_start,
+    const int64_t* __restrict__ i_end, int64_t n_rays, const float* __restrict__ gw,
+    const float* __restrict__ glast, float* __restrict__ ga) {
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r >= n_rays) return;
+    float back = glast[r] * t_last[r];
+    for (int64_t i = i_end[r] - 1; i >= i_start[r]; --i) {
+        const double den = (double)(1.f - alpha[i]) + 1e-10;
+        ga[i] = (float)((double)(gw[i] * T[i]) - (double)back / den);
+        back += gw[i] * w[i];
+    }
+}
+
+// The same, a wavefront per ray as above: the running sum sample by sample, each
+// sample's gradient in its own lane.  4096 rays, 100k samples, nothing cached: 61.8 ->
+// 12.7 us.  The line, as above: 8192 rays 2.5 / 2.8, 15.8 / 5.6, 85 / 17 us; 16,384 2.7 /
+// 3.5, 16.2 / 7.9, 96 / 26; 32,768 2.6 / 4.6, 17.0 / 12.6, 126 / 45, but at 3 and 10
+// samples a ray 4.0 / 6.9 and 6.8 / 8.2; 655,360 rays of 3 samples 18 / 138.
+constexpr int64_t kWaveRaysBwd = 16384;
+__global__ void __launch_bounds__(256) k_alpha2weight_bwd_wave(
     const float* __restrict__ alpha, const float* __restrict__ w, const float* __restrict__ T,
     const float* __restrict__ t_last, const int64_t* __restrict__ i_start,
     const int64_t* __restrict__ i_end, int64_t n_rays, const float* __restrict__ gw,
@@ -460,14 +509,11 @@ int pvdb_alpha2weight(const float* alpha, int64_t n_rays, float* weight, float* 
     PVDB_CHECK_ARG(n_rays >= 0, "n_rays must be >= 0");
     if (n_rays == 0) return PVDB_OK;
     PVDB_CHECK_ARG(alpha && weight && T && alphainv_last && i_start && i_end, "null pointer");
-    const int64_t most = pvdb_launch_items(4, 256);
-    for (int64_t r = 0; r < n_rays; r += most) {
-        const int64_t n = n_rays - r < most ? n_rays - r : most;
-        hipLaunchKernelGGL(k_alpha2weight, dim3(pvdb_blocks(n, 4)), dim3(256), 0,
-                           (hipStream_t)stream, alpha, n, weight, T, alphainv_last + r, i_start + r,
-                           i_end + r);
-        PVDB_LAUNCHED("k_alpha2weight");
-    }
+    const bool wave = n_rays <= kWaveRays;
+    hipLaunchKernelGGL(wave ? k_alpha2weight_wave : k_alpha2weight,
+                       dim3(pvdb_blocks(n_rays, wave ? 4 : 256)), dim3(256), 0, (hipStream_t)stream,
+                       alpha, n_rays, weight, T, alphainv_last, i_start, i_end);
+    PVDB_LAUNCHED("k_alpha2weight");
     return PVDB_OK;
 }
 
@@ -480,14 +526,12 @@ int pvdb_alpha2weight_bwd(const float* alpha, const float* weight, const float* 
     PVDB_CHECK_ARG(alpha && weight && T && alphainv_last && i_start && i_end && grad_weights &&
                        grad_last && grad_alpha,
                    "null pointer");
-    const int64_t most = pvdb_launch_items(4, 256);
-    for (int64_t r = 0; r < n_rays; r += most) {
-        const int64_t n = n_rays - r < most ? n_rays - r : most;
-        hipLaunchKernelGGL(k_alpha2weight_bwd, dim3(pvdb_blocks(n, 4)), dim3(256), 0,
-                           (hipStream_t)stream, alpha, weight, T, alphainv_last + r, i_start + r,
-                           i_end + r, n, grad_weights, grad_last + r, grad_alpha);
-        PVDB_LAUNCHED("k_alpha2weight_bwd");
-    }
+    const bool wave = n_rays <= kWaveRaysBwd;
+    hipLaunchKernelGGL(wave ? k_alpha2weight_bwd_wave : k_alpha2weight_bwd,
+                       dim3(pvdb_blocks(n_rays, wave ? 4 : 256)), dim3(256), 0, (hipStream_t)stream,
+                       alpha, weight, T, alphainv_last, i_start, i_end, n_rays, grad_weights, grad_last,
+                       grad_alpha);
+    PVDB_LAUNCHED("k_alpha2weight_bwd");
     return PVDB_OK;
 }
 
