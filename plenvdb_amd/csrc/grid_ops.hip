@@ -38,14 +38,14 @@ __global__ void __launch_bounds__(256) k_tri_fwd(TopoView t, const float* __rest
     const int CC = C > 0 ? C : cdyn;
     const Cell cell = make_cell(xs[p], ys[p], zs[p]);
     if constexpr (ORDER == 0) {
-        out[p] = pvdb::gather_density(t, vals, cell);
+        out[p] = pvdb::gather_density<true>(t, vals, cell);
         return;
     } else if constexpr (C > 0) {
         float o[C];
         if (C % 4 == 0 && wide)  // uniform
-            pvdb::gather_color<C>(t, vals, cell, o);
+            pvdb::gather_color<C, C % 4 == 0, true>(t, vals, cell, o);
         else
-            pvdb::gather_color<C, false>(t, vals, cell, o);
+            pvdb::gather_color<C, false, true>(t, vals, cell, o);
 #pragma unroll
         for (int c = 0; c < C; ++c) out[p * C + c] = o[c];
         return;
