@@ -31,7 +31,8 @@ def test_point_scatter():
 
 
 def test_alphas_to_weights():
-    """A wavefront to a ray: 2^26 rays.  The last has two samples, the first one."""
+    """2^26 rays, for which a wavefront to a ray would be too many work items.  The last has
+    two samples, the first one."""
     from plenvdb_amd import render_utils as ru
 
     n = (1 << 26) + 5
